@@ -305,23 +305,30 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
   // workgroup id of a single contraction. `args(T)` is the call for square
   // tiles of T.
   const bool batched = m.batch >= 0;
-  auto args = [&](uint32_t T) {
+  auto operands = [&](const std::string& rest) {  // "(A, B, C, M, N, K, epi[, rest]"
     std::string a = "t" + std::to_string(ta), b = "t" + std::to_string(tb), cc = "t" + std::to_string(tc);
-    std::string pre, tile;
     if (batched) {
-      const std::string Ts = std::to_string(T) + "u";
-      pre = "  const uint32_t tiles = ((M + " + Ts + " - 1u) / " + Ts + ") * ((N + " + Ts + " - 1u) / " + Ts +
-            "), bb = blockIdx.x / tiles;\n";
       if (m.a_batched) a = "(" + a + " + (size_t)bb * M * K)";
       if (m.b_batched) b = "(" + b + " + (size_t)bb * K * N)";
       cc = "(" + cc + " + (size_t)bb * M * N)";
-      tile = ", blockIdx.x - bb * tiles";
     }
     if (f16) {
       a = "reinterpret_cast<const __bf16*>(" + a + ")";
       b = "reinterpret_cast<const __bf16*>(" + b + ")";
     }
-    return std::make_pair(pre, "(" + a + ", " + b + ", " + cc + ", M, N, K, epi" + tile + ");\n}\n\n");
+    return "(" + a + ", " + b + ", " + cc + ", M, N, K, epi" + (rest.empty() ? "" : ", " + rest);
+  };
+  const std::string nb = batched ? ExtentExpr(g, m.batch) : "1u";
+  auto args = [&](uint32_t T) {
+    std::string pre;
+    if (batched) {
+      const std::string Ts = std::to_string(T) + "u";
+      pre = "  const uint32_t tiles = ((M + " + Ts + " - 1u) / " + Ts + ") * ((N + " + Ts + " - 1u) / " + Ts +
+            "), bb = blockIdx.x / tiles;\n";
+    }
+    std::string rest = batched ? "blockIdx.x - bb * tiles" : "";
+    if (bf16) rest = nb + ", " + (batched ? rest : "blockIdx.x");
+    return std::make_pair(pre, operands(rest) + ");\n}\n\n");
   };
   const std::string nk = m.b_nk ? "true" : "false";
   // Grid terms: [batch x] tiles of the (m, n) plane.
@@ -339,7 +346,7 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
               (m.b_batched ? "per batch" : "shared");
   o << "// " << (batched ? "batched (over @" + g.dims[m.batch].name + ") " : "") << "contraction over @"
     << g.dims[m.k].name << " on MFMA ("
-    << (f16 ? "f16 16x16x32 whole tiles, 32x32x16 edges" : bf16 ? "bf16 16x16x32 whole tiles, 32x32x16 edges" : "f32 32x32x2")
+    << (f16 ? "f16 16x16x32" : bf16 ? "bf16 16x16x32" : "f32 32x32x2")
     << "), B indexed " << (m.b_nk ? "[n][k]" : "[k][n]") << "\n";
   // Output planes of at most kGemmSmallMax elements: 32x32 tiles with K
   // split over the 16 waves of a workgroup and, when the tiles are fewer
@@ -448,24 +455,30 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
     out->kernels.push_back(k);
     return true;
   }
-  // bf16: the direct-to-LDS tiles (whole 256x256 blocks, K a positive
-  // multiple of 32, N % 8 == 0), launched when there can be one: on 4 waves
-  // of 128x128 with A in 64-deep slices when K % 64 == 0 and K >= 256 (_w),
-  // else on 8 waves of 128x64 with 32-deep slices (_v); every other tile on
-  // the 256-thread register-staged kernel, skipped when every tile is a
-  // direct-to-LDS one (M, N multiples of 256, K a positive multiple of 32).
-  // Each kernel returns at once on the other kernels' tiles.
+  // 16-bit inputs: whole 256x256 blocks of planes of at least
+  // kGemmWholeMin elements (K a positive multiple of 32, N % 8 == 0) on the
+  // direct-to-LDS kernels: 4 waves of 128x128 with A in 64-deep slices when
+  // K % 64 == 0 and K >= 256 (_w), else 8 waves of 128x64 with 32-deep slices
+  // (_v); every other tile on the 128x128 kernel for any shape, skipped when
+  // there is none. Each kernel returns at once on the other kernels' tiles.
   const std::string M = g.dims[m.m].name, N = g.dims[m.n].name, K = g.dims[m.k].name;
+  const uint64_t wholeMin = small ? kGemmWholeMin : 0u;
+  const std::string targs = "<" + nk + ", decltype(epi), " + (f16 ? "true" : "false") + ", " + std::to_string(wholeMin) + "u>";
   const auto a256 = args(256);
+  // 128x128 tiles fewer than half of kHalfTiles are launched as 64-row parts.
+  const uint32_t kHalfTiles = 256u;
+  const std::string a128 = operands(nb + (batched ? ", gt - bb * tiles, part, P" : ", gt, part, P"));
   o << "extern \"C\" __global__ void __launch_bounds__(256) " << symbol << "_w(\n    " << signature << ") {\n"
-    << epi.str() << a256.first << "  tca::hip::gemm_bf16_4w<" << nk << (f16 ? ", decltype(epi), true" : "") << ">"
-    << a256.second;
+    << epi.str() << a256.first << "  tca::hip::gemm_bf16_4w" << targs << a256.second;
   o << "extern \"C\" __global__ void __launch_bounds__(512) " << symbol << "_v(\n    " << signature << ") {\n"
-    << epi.str() << a256.first << "  tca::hip::gemm_bf16_256_w8<" << nk << (f16 ? ", decltype(epi), 4, true" : "")
-    << ">" << a256.second;
-  o << "extern \"C\" __global__ void __launch_bounds__(256) " << symbol << "(\n    " << signature << ") {\n"
-    << epi.str() << a256.first << "  tca::hip::gemm_bf16_256<" << nk << ", decltype(epi), 1, true, true, true"
-    << (f16 ? ", true" : "") << ">" << a256.second;
+    << epi.str() << a256.first << "  tca::hip::gemm_bf16_256_w8" << targs << a256.second;
+  o << "extern \"C\" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) " << symbol
+    << "(\n    " << signature << ") {\n"
+    << epi.str() << "  const uint32_t tiles = ((M + 127u) / 128u) * ((N + 127u) / 128u);\n"
+    << "  const uint32_t T = " << (batched ? ExtentExpr(g, m.batch) + " * tiles" : std::string("tiles")) << ";\n"
+    << "  const uint32_t P = tca::hip::gemm_split_chunks(K, T, 1u, " << kHalfTiles << "u);\n"
+    << "  const uint32_t gt = blockIdx.x % T, part = blockIdx.x / T;\n"
+    << (batched ? "  const uint32_t bb = gt / tiles;\n" : "") << "  tca::hip::gemm16_any" << targs << a128 << ");\n}\n\n";
   GemmKernel w;
   w.suffix = "_w";
   w.block = 256;
@@ -481,11 +494,27 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
   v.unless = {K + " 256 4294967295 64 0"};
   v.detail = ty + " mfma 16x16x32 tile=256x256 bk=32 8 waves (direct-to-LDS ring; whole tiles, K % 64 != 0 or K < 256)" + orient;
   GemmKernel e;
-  e.grid = grid;
+  e.block = 512;
+  e.grid = tiles(128);
   e.unless = {M + " 0 4294967295 256 0", N + " 0 4294967295 256 0", K + " 32 4294967295 32 0"};
-  e.detail = ty + " mfma 32x32 tile=256x256 bk=64 4 waves (edge tiles, K % 32 != 0, N % 8 != 0)" + orient;
-  if (!bigWhen.empty())
-    for (GemmKernel* k : {&w, &v, &e}) k->when.push_back(bigWhen);
+  std::string halfTerms;
+  for (const auto& t : e.grid) halfTerms += " " + t;
+  e.split = K + " 1 " + std::to_string(kHalfTiles) + " 0 " + std::to_string(e.grid.size()) + halfTerms;
+  e.detail = ty + " mfma 16x16x32 tile=128x128 (64x128 for few tiles) bk=64 8 waves, register-staged, any shape (every tile the others do not take)" + orient;
+  if (!bigWhen.empty()) {
+    // gemm16_on_whole_tiles decides on the device; the guards skip launches
+    // that it leaves idle: the any-shape kernel where every tile is whole, the
+    // 256x256 kernels on smaller planes (from K = 2048 on the 2 us of an idle
+    // launch are under a tenth).
+    const std::string plane = (batched ? g.dims[m.batch].name + "*" : std::string()) + M + "*" + N;
+    const std::string few = plane + " 0 " + std::to_string(wholeMin - 1u) + " 1 0";
+    w.when.push_back(bigWhen);
+    w.unless = {few, K + " 0 2047 1 0"};
+    v.when.push_back(plane + " " + std::to_string(wholeMin) + " 18446744073709551615 1 0");
+    v.when.push_back(bigWhen);
+    e.unless.push_back(plane + " " + std::to_string(wholeMin) + " 18446744073709551615 1 0");
+    e.when.push_back(bigWhen);
+  }
   out->kernels.push_back(w);
   out->kernels.push_back(v);
   out->kernels.push_back(e);

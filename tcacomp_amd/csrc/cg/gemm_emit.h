@@ -55,6 +55,11 @@ struct GemmEmitted {
 // kernel (32x32 tiles, K split over the waves of a workgroup and, when the
 // tiles are few, over workgroups); larger ones the 128/256 tile kernels.
 constexpr uint64_t kGemmSmallMax = 1ull << 20;
+// 16-bit planes (all batches together) of at least kGemmWholeMin elements,
+// 128 tiles of 256x256, run on the direct-to-LDS kernels where they are whole
+// tiles (gemm16_on_whole_tiles in gemm.h says why there).
+constexpr uint64_t kGemmWholeMin = 128ull << 16;
+
 
 // `nest` names the partial scratch of the small kernel's K split
 // (__gemmpart<nest>); `small` false leaves the small kernel out.

@@ -4,11 +4,11 @@
 // WarpReducer collective per output element (a shuffle tree per Reduce and
 // two barriers per Combine; .planning/quick/261030-uai-.../after-cu/gemm.cu:
 // 59-90). Here the contraction runs on MFMA:
-//   bf16 inputs : v_mfma_f32_16x16x32_bf16 (gfx950) on whole 256x256 tiles
-//                 (f16 inputs: the same kernels with the _f16 MFMAs)
-//                 (gemm_bf16_4w when K % 64 == 0 and K >= 256, else
-//                 gemm_bf16_256_w8), v_mfma_f32_32x32x16_bf16 on the edge
-//                 tiles (gemm_bf16_256); fp32 accumulate
+//   bf16 inputs : v_mfma_f32_16x16x32_bf16 (gfx950): large planes of whole
+//                 256x256 tiles on gemm_bf16_4w (K % 64 == 0 and K >= 256)
+//                 or gemm_bf16_256_w8, everything else on gemm16_any;
+//                 fp32 accumulate (f16 inputs: the same kernels with the
+//                 _f16 MFMAs)
 //   fp32 inputs : v_mfma_f32_32x32x2f32 (gemm_f32_4w on whole tiles from
 //                 M, N >= 4096 on, else gemm_f32_tile), fp32 accumulate
 // Geometry of the register-staged kernels: a 256-thread workgroup (4 waves,
@@ -83,31 +83,30 @@ __device__ __forceinline__ void gemm_tile_coords(uint32_t tiles_m, uint32_t tile
   *tn = in / rows;
 }
 
-// ------------------------------------------------------- bf16 path, 256 tiles
-// Tile: BM = BN = 256, BK = 64; 4 waves as 2x2, each 128x128 = 4x4 MFMA
-// blocks (256 fp32 accumulators per lane). Per 16-deep K step a wave reads
-// 4 A + 4 B fragments (8 x 1 KiB of LDS) for 16 MFMAs.
-//
-// LDS layout: each [256][64] bf16 tile is unpadded (128-byte rows) over 64
-// four-byte banks (256 bytes, two rows' worth; a 16-byte slot is (row
-// parity, column group)). Logical row r is stored at physical row
-// p = r ^ ((r / 8) % 2) and its column group c at c ^ ((p / 2) % 8):
-//     element (r, k) -> p*64 + ((k/8) ^ ((p/2) % 8))*8 + k%8.
-// A fragment read (32 consecutive rows, one column group per half-wave)
-// then hits 16 distinct slots in each 16-lane cycle of a 128-bit read (the
-// cycles measured on gfx950 are described at gemm_bf16_256_w8). Two such
-// tile pairs (A, B) double-buffer the K loop with one barrier per step:
-// 128 KiB of LDS.
-// SWZ = 0 keeps the plain row-XOR swizzle (c ^ (r % 8)), optimal for a
-// 32-bank / 8-lane-phase LDS; SWZ = 1 is the layout above.
-template <int SWZ>
-__device__ __forceinline__ uint32_t swz64(uint32_t row, uint32_t cg) {
-  if constexpr (SWZ == 0) {
-    return row * 64u + ((cg ^ (row & 7u)) << 3);
-  } else {
-    const uint32_t p = row ^ ((row >> 3) & 1u);
-    return p * 64u + ((cg ^ ((p >> 1) & 7u)) << 3);
+// ----------------------------------------------- 16-bit path, any shape
+// Unaligned 16-byte accesses: gfx950 serves a 16-byte vector load or store
+// at any element address (the amdhsa unaligned access mode), so rows whose
+// length is not a multiple of the vector still move 16 bytes per lane.
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ u32x4 load16_any(const uint16_t* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
+
+// The eight 16-bit values of v moved down by n places (zeros shifted in; all
+// zero from n = 8 on): a chunk that would run past the end of its row is
+// loaded from 8 elements before that end instead, so the load stays inside
+// the row, and moved into place.
+__device__ __forceinline__ u32x4 shift_down16(u32x4 v, uint32_t n) {
+  uint64_t lo = v[0] | (static_cast<uint64_t>(v[1]) << 32), hi = v[2] | (static_cast<uint64_t>(v[3]) << 32);
+  const uint32_t b = 16u * (n & 3u);
+  if (n & 4u) {
+    lo = hi;
+    hi = 0u;
   }
+  lo = b ? (lo >> b) | (hi << (64u - b)) : lo;
+  hi >>= b;
+  if (n >= 8u) lo = hi = 0u;
+  return u32x4{static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi),
+               static_cast<uint32_t>(hi >> 32)};
 }
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
@@ -117,254 +116,338 @@ typedef __attribute__((address_space(3))) void lds_void;
 // lgkmcnt[11:8] | vmcnt[5:4] at [15:14].
 constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | (7 << 4) | ((lgkm & 15) << 8) | ((vm >> 4) << 14); }
 
-// The tiles the direct-to-LDS path takes: the whole 256x256 block in range,
-// K a positive multiple of 32 and [K][N] / [N][K] rows 16-byte aligned.
-__device__ __forceinline__ bool gemm_bf16_dma_tile(uint32_t m0, uint32_t n0, uint32_t M, uint32_t N, uint32_t K) {
-  return m0 + 256u <= M && n0 + 256u <= N && K % 32u == 0u && N % 8u == 0u && K > 0u;
+// Whether the whole 256x256 tiles of `batch` planes run on the direct-to-LDS
+// kernels (one workgroup per CU, so in rounds of 256 tiles) rather than on
+// gemm16_any's 128x128 tiles. Measured at K = 4096 (time grows with K on both
+// sides): a round of 256x256 tiles takes 95 us, 128x128 tiles 0.16 us each,
+// and the ragged edges, which gemm16_any takes afterwards, 40 us. Planes that
+// are whole tiles throughout compare the first two: from WHOLE_MIN elements
+// on (150 tiles; the plan's guards carry the same bound, and skip gemm16_any
+// there); planes with edges also pay the third. WHOLE_MIN 0: always.
+template <uint64_t WHOLE_MIN>
+__host__ __device__ __forceinline__ bool gemm16_on_whole_tiles(uint32_t M, uint32_t N, uint32_t batch) {
+  if constexpr (WHOLE_MIN == 0u) return true;
+  if (static_cast<uint64_t>(M) * N * batch < WHOLE_MIN) return false;
+  if (M % 256u == 0u && N % 256u == 0u) return true;
+  const uint64_t whole = static_cast<uint64_t>(M / 256u) * (N / 256u) * batch;
+  const uint64_t t128 = static_cast<uint64_t>((M - 1u) / 128u + 1u) * ((N - 1u) / 128u + 1u) * batch;
+  return (whole + 255u) / 256u * 600u + 250u <= t128;
+}
+// K and row alignments the direct-to-LDS kernels take: K a positive multiple
+// of 32, [K][N] / [N][K] rows 16-byte aligned.
+__host__ __device__ __forceinline__ bool gemm16_direct_k(uint32_t N, uint32_t K) { return K % 32u == 0u && N % 8u == 0u && K > 0u; }
+// The (tile_m, tile_n) of tile index `tile` among the whole 256x256 tiles of
+// one plane; false past them (the edges are gemm16_any's).
+__device__ __forceinline__ bool gemm16_whole_coords(uint32_t M, uint32_t N, uint32_t tile, uint32_t* tm, uint32_t* tn) {
+  const uint32_t tiles_m = M / 256u, tiles_n = N / 256u;
+  if (tile >= tiles_m * tiles_n) return false;
+  gemm_tile_coords(tiles_m, tiles_n, tm, tn, tile);
+  return true;
 }
 
-// SKIP_DMA: the direct-to-LDS tiles belong to another kernel
-// (gemm_bf16_256_w8); this one returns at once on them.
-template <bool B_NK, typename Epi, int SWZ = 1, bool SPREAD = true, bool PREFETCH = true, bool SKIP_DMA = false,
-          bool F16 = false>
-__device__ __forceinline__ void gemm_bf16_256(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
-                                              float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
-                                              uint32_t tile = ~0u) {
-  constexpr uint32_t BM = 256, BN = 256, BK = 64, TILE = BM * BK;
-  __shared__ __attribute__((aligned(16))) uint16_t lds[2][2][TILE];  // [buffer][A, B]
-  const uint32_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  uint32_t tm, tn;
-  gemm_tile_coords(tiles_m, tiles_n, &tm, &tn, tile == ~0u ? blockIdx.x : tile);
-  const uint32_t m0 = tm * BM, n0 = tn * BN;
-  if (SKIP_DMA && gemm_bf16_dma_tile(m0, n0, M, N, K)) return;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t wm = (wave >> 1) * 128u, wn = (wave & 1u) * 128u;
-  const bool vec_a = (K % 8u) == 0u;
-  const bool vec_b = B_NK ? (K % 8u) == 0u : (N % 8u) == 0u;
-  const uint16_t* __restrict__ A16 = reinterpret_cast<const uint16_t*>(A);
-  const uint16_t* __restrict__ B16 = reinterpret_cast<const uint16_t*>(B);
+__device__ __forceinline__ uint32_t swz_rows64(uint32_t row, uint32_t g) { return row * 64u + ((g ^ (row & 6u)) << 3); }
+// The 16-byte slot of a [K][BN] slice's row k is XORed with this (measured
+// bank cycles at gemm_bf16_256_w8): rows of 256 bytes and more cover the 64
+// banks, rows of 128 bytes pair up by the parity of k.
+template <uint32_t BN>
+__device__ __forceinline__ uint32_t kn_slot_xor(uint32_t k) {
+  if constexpr (BN >= 128u) return ((k & 3u) | (((k >> 3) & 1u) << 2)) << 1;
+  else return (((k >> 1) & 1u) | (((k >> 3) & 1u) << 1)) << 1;
+}
+template <uint32_t BN>
+__device__ __forceinline__ uint32_t swz_kn(uint32_t k, uint32_t n) {
+  return k * BN + (((n >> 3) ^ kn_slot_xor<BN>(k)) << 3) + (n & 7u);
+}
 
-  f32x16 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+// B operand of v_mfma_f32_16x16x32_bf16 (lane l: column n_col0 + l%16,
+// k = k_row0 + 8(l/16) .. +8) from a [K][BN] slice with the gfx950
+// transposing read ds_read_b64_tr_b16: within each 16-lane group, lane j
+// points at four consecutive values R_j of one k row and lane i receives
+// [R_{i/4}[i%4], R_{4+i/4}[i%4], R_{8+i/4}[i%4], R_{12+i/4}[i%4]]. With lane j
+// addressing row kb + j/4, columns n_col0 + 4(j%4), lane i gets
+// B[kb + e][n_col0 + i] for e = 0..3; a second read at kb + 4 completes its 8.
+template <uint32_t BN>
+__device__ __forceinline__ bf16x8 frag_b16_tr(const uint16_t* Bs, uint32_t n_col0, uint32_t lane, uint32_t k_row0 = 0u) {
+  const uint32_t g = lane >> 4, j = lane & 15u;
+  const uint32_t k = k_row0 + 8u * g + (j >> 2), n = n_col0 + 4u * (j & 3u);
+  const i16x4 lo =
+      __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(Bs + swz_kn<BN>(k, n)));
+  const i16x4 hi =
+      __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(Bs + swz_kn<BN>(k + 4u, n)));
+  typedef short i16x8 __attribute__((ext_vector_type(8)));
+  const i16x8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  return __builtin_bit_cast(bf16x8, v);
+}
 
-  u32x4 ra[8], rb[8];
-  // Interior tiles (the whole BMxBN block in range, rows 16-byte aligned)
-  // take unguarded vector loads addressed as a workgroup-uniform base plus a
-  // 32-bit per-lane byte offset; the test is uniform, so it is a scalar
-  // branch, not a per-lane mask.
-  const bool interior_mn = vec_a && vec_b && m0 + BM <= M && n0 + BN <= N;
-  const uint32_t off_rows = ((tid >> 3) * K + (tid & 7u) * 8u) * 2u;  // row-panel vector of this lane
-  const uint32_t off_kn = ((tid & 7u) * 8u * N + (tid >> 3) * 8u) * 2u;  // [K][N] block of this lane
-  auto at = [](const uint16_t* base, uint32_t byte_off) {
-    return *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(base) + byte_off);
-  };
-  // Rows of a K-contiguous panel (A, or B as [n][k]): 2048 16-byte vectors.
-  auto load_rows = [&](const uint16_t* __restrict__ P, uint32_t rows, uint32_t r0, uint32_t k0, bool vec, u32x4* r) {
-    if (interior_mn && k0 + BK <= K) {
+// One BM x BN tile of C at (m0, n0), every shape: ragged edges, K of any
+// length, rows of any alignment. KG groups of WGM x WGN waves each hold the
+// whole tile, a wave (BM/WGM) x (BN/WGN) of it as blocks of
+// v_mfma_f32_16x16x32, and take every KG-th 64-deep slice of K; their sums
+// meet in LDS in group order. A slice goes global memory -> registers (16
+// bytes per lane, D of the group's slices ahead) -> LDS (two buffers per
+// group, one barrier per slice) -> fragments.
+// No load is guarded: rows past the end re-read the last row (their results
+// are not stored), and a chunk past the end of its row is loaded from 8
+// elements before it and moved into place on its way into LDS
+// (shift_down16), so the K tail adds zeros. With guarded loads and one wave
+// per SIMD the kernel before took 269 us for 1001 x 1501 x 1003 (13 now) and
+// 362 for 257 x 4096 x 4096 (31); 1000 x 4096 x 1024 went from 97 to 15 us.
+// What bounds it: the waves of a workgroup load, write and compute in step,
+// so the 0.27 us of MFMAs and fragment reads of a 128x128 slice and the 0.3 us
+// of its loads and LDS writes overlap little (0.5-0.6 us a slice). Measured
+// at 2048 x 2048 x 4096 and not better than the 44 us here: 4 waves per
+// workgroup and two workgroups per CU 47, two groups of 4 waves on
+// alternate slices 43 (but 106 against 94 at 3000^3), the same with the groups half a turn
+// apart 44, operands loaded straight into a 4-deep LDS ring 45 (8 waves) and
+// 55 (4 waves). `TINY` (K-contiguous rows or
+// [K][N] rows shorter than one chunk) loads those element by element.
+// `lds` holds KG * 2 * 64 * (BM + BN) values.
+template <uint32_t BM, uint32_t BN, uint32_t WGM, uint32_t WGN, uint32_t KG, int D, bool B_NK, bool F16, bool TINY,
+          typename Epi>
+__device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                                            float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
+                                            uint32_t m0, uint32_t n0, uint16_t* lds) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr uint32_t THREADS = 64u * WGM * WGN, TM = BM / WGM, TN = BN / WGN;
+  constexpr int IM = TM / 16, JN = TN / 16, CA = BM * 8 / THREADS, CB = BN * 8 / THREADS;
+  static_assert(CA >= 1 && CB >= 1 && (D == 1 || D % 2 == 0), "whole chunks per thread; the buffer of a slice is static");
+  constexpr uint32_t ASL = BM * 64u, BUF = ASL + BN * 64u;
+  const uint32_t lane = threadIdx.x & 63u, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t grp = wave_id / (WGM * WGN), wave = wave_id % (WGM * WGN), tid = wave * 64u + lane;
+  const uint32_t wm = (wave / WGN) * TM, wn = (wave % WGN) * TN;
+  uint16_t* glds = lds + grp * (2u * BUF);
+  // Chunk i of this thread: row (i * THREADS + tid) / 8 of a K-contiguous
+  // panel at k chunk tid % 8, or row k = (i * THREADS + tid) / (BN / 8) of a
+  // [K][N] slice at column chunk tid % (BN / 8).
+  const uint32_t kch = (tid & 7u) * 8u, row0 = tid >> 3;
+  const uint32_t bk0 = tid / (BN / 8u), bn = n0 + (tid % (BN / 8u)) * 8u;
+  const uint16_t* pa[CA];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) r[i] = at(P + static_cast<uint64_t>(r0 + i * 32u) * K + k0, off_rows);
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t v = i * 256u + tid, rr = v >> 3, gk = k0 + (v & 7u) * 8u, gr = r0 + rr;
-      if (vec && gr < rows && gk + 8u <= K) {
-        r[i] = *reinterpret_cast<const u32x4*>(P + static_cast<uint64_t>(gr) * K + gk);
-      } else {
-        uint32_t h[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) h[e] = (gr < rows && gk + e < K) ? P[static_cast<uint64_t>(gr) * K + gk + e] : 0u;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[i][e] = h[2 * e] | (h[2 * e + 1] << 16);
-      }
-    }
-  };
-  // [K][N] panel: thread owns an 8(k) x 8(n) block; kb = tid % 8, nb = tid / 8.
-  auto load_b_kn = [&](uint32_t k0) {
-    const uint32_t kb = tid & 7u, nb = tid >> 3;
-    if (interior_mn && k0 + BK <= K) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) rb[i] = at(B16 + static_cast<uint64_t>(k0 + i) * N + n0, off_kn);
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t gk = k0 + kb * 8u + i, gn = n0 + nb * 8u;
-      if (vec_b && gk < K && gn + 8u <= N) {
-        rb[i] = *reinterpret_cast<const u32x4*>(B16 + static_cast<uint64_t>(gk) * N + gn);
-      } else {
-        uint32_t h[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) h[e] = (gk < K && gn + e < N) ? B16[static_cast<uint64_t>(gk) * N + gn + e] : 0u;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) rb[i][e] = h[2 * e] | (h[2 * e + 1] << 16);
-      }
-    }
-  };
-  // Stores of the staged slice into an LDS buffer, in halves so they can be
-  // spread between the MFMA steps of the current slice.
-  auto store_a = [&](uint32_t buf, int half) {
-    uint16_t* As = lds[buf][0];
-#pragma unroll
-    for (int i = half * 4; i < half * 4 + 4; ++i) {
-      const uint32_t v = i * 256u + tid;
-      *reinterpret_cast<u32x4*>(&As[swz64<SWZ>(v >> 3, v & 7u)]) = ra[i];
-    }
-  };
-  auto store_b = [&](uint32_t buf, int half) {
-    uint16_t* Bs = lds[buf][1];
-    if constexpr (B_NK) {
-#pragma unroll
-      for (int i = half * 4; i < half * 4 + 4; ++i) {
-        const uint32_t v = i * 256u + tid;
-        *reinterpret_cast<u32x4*>(&Bs[swz64<SWZ>(v >> 3, v & 7u)]) = rb[i];
-      }
-    } else {
-      // 8x8 transpose in registers: column n of the block gets its 8 k values.
-      const uint32_t kb = tid & 7u, nb = tid >> 3;
-#pragma unroll
-      for (int n = half * 4; n < half * 4 + 4; ++n) {
-        const int d = n >> 1;
-        u32x4 w;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t lo = rb[2 * q][d], hi = rb[2 * q + 1][d];
-          w[q] = (n & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-        }
-        *reinterpret_cast<u32x4*>(&Bs[swz64<SWZ>(nb * 8u + n, kb)]) = w;
-      }
-    }
-  };
-  auto load_a = [&](uint32_t k0) { load_rows(A16, M, m0, k0, vec_a, ra); };
-  auto load_b = [&](uint32_t k0) {
-    if constexpr (B_NK) load_rows(B16, N, n0, k0, vec_b, rb);
-    else load_b_kn(k0);
-  };
-  auto frag = [&](const uint16_t* T, uint32_t row0, uint32_t cg) {
-    return *reinterpret_cast<const bf16x8*>(&T[swz64<SWZ>(row0 + (lane & 31u), cg)]);
-  };
-
-  // SPREAD: while slice kt is multiplied out of LDS buffer kt%2, slice kt+1
-  // (already in registers) is written into the other buffer a quarter per
-  // MFMA step, and the registers refill with slice kt+2 as soon as they are
-  // written out. Otherwise slice kt+1 is loaded at the top of the step and
-  // written after the MFMAs. One barrier per slice either way.
-  //
-  // The MFMA takes the B fragment as its first operand: it then computes the
-  // C^T block, so each lane ends up holding four consecutive columns of one
-  // row of C (a 16-byte store) instead of four rows of one column.
-  const uint32_t nk = (K + BK - 1) / BK;
-  if (nk > 0) {
-    load_a(0);
-    load_b(0);
-    store_a(0, 0);
-    store_a(0, 1);
-    store_b(0, 0);
-    store_b(0, 1);
+  for (int i = 0; i < CA; ++i) {
+    const uint32_t r = m0 + row0 + i * (THREADS / 8u);
+    pa[i] = A + static_cast<uint64_t>(r < M ? r : M - 1u) * K;
   }
-  if (SPREAD && nk > 1) {
-    load_a(BK);
-    load_b(BK);
+  const uint16_t* pb[B_NK ? CB : 1];
+  uint32_t bsh = 0u;  // [K][N]: places this thread's chunks move down (columns past N)
+  if constexpr (B_NK) {
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+      const uint32_t r = n0 + row0 + i * (THREADS / 8u);
+      pb[i] = B + static_cast<uint64_t>(r < N ? r : N - 1u) * K;
+    }
+  } else {
+    const uint32_t last = N >= 8u ? N - 8u : 0u, at = bn < last ? bn : last;
+    bsh = bn - at;
+    pb[0] = B + at;
   }
-  __syncthreads();
-  for (uint32_t kt = 0; kt < nk; ++kt) {
-    const uint32_t buf = kt & 1u, nbuf = buf ^ 1u;
-    const bool has1 = kt + 1 < nk, has2 = kt + 2 < nk;
-    const uint16_t* As = lds[buf][0];
-    const uint16_t* Bs = lds[buf][1];
-    if (!SPREAD && has1) {
-      load_a((kt + 1) * BK);
-      load_b((kt + 1) * BK);
-    }
-    bf16x8 fa[4], fb[4];
-    if constexpr (PREFETCH) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) fa[i] = frag(As, wm + i * 32u, lane >> 5);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) fb[j] = frag(Bs, wn + j * 32u, lane >> 5);
-    }
-#pragma unroll
-    for (uint32_t ks = 0; ks < BK / 16; ++ks) {
-      const uint32_t cg = ks * 2u + (lane >> 5);
-      bf16x8 ga[4], gb[4];
-      if constexpr (PREFETCH) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ga[i] = fa[i];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) gb[j] = fb[j];
-        if (ks + 1 < BK / 16) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) fa[i] = frag(As, wm + i * 32u, cg + 2u);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) fb[j] = frag(Bs, wn + j * 32u, cg + 2u);
-        }
-        // Keep the next step's LDS reads issued ahead of this step's MFMAs:
-        // without the fence the scheduler sinks them and re-waits on LDS
-        // latency between MFMA groups.
-        __builtin_amdgcn_sched_barrier(0);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ga[i] = frag(As, wm + i * 32u, cg);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) gb[j] = frag(Bs, wn + j * 32u, cg);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mfma_32x32x16_16b<F16>(gb[j], ga[i], acc[i][j]);
-      if (SPREAD && has1) {
-        if (ks == 0) store_a(nbuf, 0);
-        if (ks == 1) store_a(nbuf, 1);
-        if (ks == 2) store_b(nbuf, 0);
-        if (ks == 3) store_b(nbuf, 1);
-      }
-      if (SPREAD && has2) {
-        if (ks == 1) load_a((kt + 2) * BK);
-        if (ks == 3) load_b((kt + 2) * BK);
+  auto load_k = [&](const uint16_t* row, uint32_t k0) -> u32x4 {  // a chunk of a K-contiguous row
+    const uint32_t k = k0 + kch;
+    if constexpr (TINY) {
+      if (K < 8u) {
+        u32x4 v = {0u, 0u, 0u, 0u};
+        for (uint32_t e = 0; e < 8u; ++e)
+          if (k + e < K) v[e >> 1] |= static_cast<uint32_t>(row[k + e]) << (16u * (e & 1u));
+        return v;
       }
     }
-    if (!SPREAD && has1) {
-      store_a(nbuf, 0);
-      store_a(nbuf, 1);
-      store_b(nbuf, 0);
-      store_b(nbuf, 1);
+    return load16_any(row + (k < K - 8u ? k : K - 8u));
+  };
+  auto load_n = [&](uint32_t k) -> u32x4 {  // a chunk of row k of a [K][N] operand
+    const uint16_t* row = pb[0] + static_cast<uint64_t>(k < K ? k : K - 1u) * N;
+    if constexpr (TINY) {
+      if (N < 8u) {
+        u32x4 v = {0u, 0u, 0u, 0u};
+        for (uint32_t e = 0; e < 8u; ++e)
+          if (bn + e < N) v[e >> 1] |= static_cast<uint32_t>(row[bn + e]) << (16u * (e & 1u));
+        return v;
+      }
     }
+    return load16_any(row);
+  };
+  u32x4 ra[D][CA], rb[D][CB];
+  auto load = [&](int d, uint32_t k0) {
+#pragma unroll
+    for (int i = 0; i < CA; ++i) ra[d][i] = load_k(pa[i], k0);
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+      if constexpr (B_NK) rb[d][i] = load_k(pb[i], k0);
+      else rb[d][i] = load_n(k0 + bk0 + i * (THREADS / (BN / 8u)));
+    }
+  };
+  const bool edge_n = !B_NK && n0 + BN > N && !(TINY && N < 8u);
+  auto write = [&](auto last, int d, uint32_t buf, uint32_t k0) {
+    constexpr bool kLast = decltype(last)::value;  // may be the last, short slice
+    uint16_t* As = glds + buf * BUF;
+    uint16_t* Bs = As + ASL;
+    if (kLast && k0 + 64u > K && !(TINY && K < 8u)) {
+      const uint32_t k = k0 + kch, n = k - (k < K - 8u ? k : K - 8u);
+#pragma unroll
+      for (int i = 0; i < CA; ++i) ra[d][i] = shift_down16(ra[d][i], n);
+      if constexpr (B_NK) {
+#pragma unroll
+        for (int i = 0; i < CB; ++i) rb[d][i] = shift_down16(rb[d][i], n);
+      }
+    }
+    if constexpr (!B_NK) {
+      if (edge_n) {
+#pragma unroll
+        for (int i = 0; i < CB; ++i) rb[d][i] = shift_down16(rb[d][i], bsh);
+      }
+      if (kLast && k0 + 64u > K) {
+#pragma unroll
+        for (int i = 0; i < CB; ++i)
+          if (k0 + bk0 + i * (THREADS / (BN / 8u)) >= K) rb[d][i] = u32x4{0u, 0u, 0u, 0u};
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < CA; ++i)
+      *reinterpret_cast<u32x4*>(&As[swz_rows64(row0 + i * (THREADS / 8u), tid & 7u)]) = ra[d][i];
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+      if constexpr (B_NK)
+        *reinterpret_cast<u32x4*>(&Bs[swz_rows64(row0 + i * (THREADS / 8u), tid & 7u)]) = rb[d][i];
+      else
+        *reinterpret_cast<u32x4*>(&Bs[swz_kn<BN>(bk0 + i * (THREADS / (BN / 8u)), (tid % (BN / 8u)) * 8u)]) = rb[d][i];
+    }
+  };
+  f32x4 acc[IM][JN];
+#pragma unroll
+  for (int i = 0; i < IM; ++i)
+#pragma unroll
+    for (int j = 0; j < JN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto compute = [&](uint32_t buf) {
+    const uint16_t* As = glds + buf * BUF;
+    const uint16_t* Bs = As + ASL;
+#pragma unroll
+    for (uint32_t h = 0; h < 2u; ++h) {
+      bf16x8 fa[IM], fb[JN];
+#pragma unroll
+      for (int i = 0; i < IM; ++i)
+        fa[i] = *reinterpret_cast<const bf16x8*>(&As[swz_rows64(wm + i * 16u + (lane & 15u), 4u * h + (lane >> 4))]);
+#pragma unroll
+      for (int j = 0; j < JN; ++j) {
+        if constexpr (B_NK)
+          fb[j] = *reinterpret_cast<const bf16x8*>(&Bs[swz_rows64(wn + j * 16u + (lane & 15u), 4u * h + (lane >> 4))]);
+        else
+          fb[j] = frag_b16_tr<BN>(Bs, wn + j * 16u, lane, 32u * h);
+      }
+      // Operand-swapped: the MFMA computes the C^T block, so a lane holds
+      // four consecutive columns of one row of C.
+#pragma unroll
+      for (int j = 0; j < JN; ++j)
+#pragma unroll
+        for (int i = 0; i < IM; ++i) acc[i][j] = mfma_16x16x32_16b<F16>(fb[j], fa[i], acc[i][j]);
+    }
+  };
+  // Turn t of a group (slice t * KG + grp) is written into LDS while turn t-1
+  // is computed and loaded D turns earlier. The main loop's loads are
+  // unconditional: with a load that may not have been issued the compiler
+  // must wait for the younger ones too. (A slice past K re-reads the rows'
+  // last chunk and is written as zeros.)
+  using Body = std::false_type;
+  using Last = std::true_type;
+  const uint32_t ns = K / 64u + (K % 64u != 0u ? 1u : 0u), nt = ns / KG + (ns % KG != 0u ? 1u : 0u);
+  constexpr int U = D == 1 ? 2 : D;  // turns per loop iteration: buffer and register set static
+  auto k_of = [&](uint32_t t) { return (t * KG + grp) * 64u; };
+  if (nt > 0u) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, k_of(d));
+    write(Last{}, 0, 0u, k_of(0));
+    load(0, k_of(D));
     __syncthreads();
   }
-  // acc[i][j][4g + q] = C[m][n + q] with m = m0 + wm + 32i + lane%32 and
-  // n = n0 + wn + 32j + 8g + 4*(lane/32).
-  const uint32_t mr = m0 + wm + (lane & 31u), nc = n0 + wn + 4u * (lane >> 5);
-  if (m0 + BM <= M && n0 + BN <= N && (N % 4u) == 0u) {
+  uint32_t t0 = 0;
+  for (; t0 + U + D < nt; t0 += U) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const uint32_t m = mr + 32u * i, n = nc + 32u * j + 8u * g;
-          float4 v;
-          v.x = epi(acc[i][j][4 * g + 0], m, n + 0);
-          v.y = epi(acc[i][j][4 * g + 1], m, n + 1);
-          v.z = epi(acc[i][j][4 * g + 2], m, n + 2);
-          v.w = epi(acc[i][j][4 * g + 3], m, n + 3);
-          *reinterpret_cast<float4*>(C + static_cast<uint64_t>(m) * N + n) = v;
-        }
-    return;
+    for (int i = 0; i < U; ++i) {
+      write(Body{}, (i + 1) % D, (i + 1) & 1, k_of(t0 + i + 1u));
+      load((i + 1) % D, k_of(t0 + i + 1u + D));
+      compute(i & 1);
+      __syncthreads();
+    }
   }
+  for (; t0 < nt; t0 += U) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const uint32_t m = mr + 32u * i, n = nc + 32u * j + 8u * (e >> 2) + (e & 3);
-        if (m < M && n < N) C[static_cast<uint64_t>(m) * N + n] = epi(acc[i][j][e], m, n);
+    for (int i = 0; i < U; ++i) {
+      const uint32_t t = t0 + i;
+      if (t < nt) {
+        if (t + 1u < nt) write(Last{}, (i + 1) % D, (i + 1) & 1, k_of(t + 1u));
+        if (t + 1u + D < nt) load((i + 1) % D, k_of(t + 1u + D));
+        compute(i & 1);
+        __syncthreads();
       }
+    }
+  }
+  // Block (i, j) is finished by group (i * JN + j) / (IM * JN / KG): the
+  // others hand it their sums through LDS (16 bytes per lane and block).
+  constexpr int OWN = IM * JN / static_cast<int>(KG);
+  if constexpr (KG > 1u) {
+    static_assert(IM * JN % KG == 0u && KG * IM * JN * THREADS * 16u <= KG * 2u * BUF * 2u, "the sums fit the slices' LDS");
+    f32x4* red = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+    for (int b = 0; b < IM * JN; ++b)
+      if (static_cast<uint32_t>(b / OWN) != grp) red[(grp * (IM * JN) + b) * THREADS + tid] = acc[b / JN][b % JN];
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < IM * JN; ++b) {
+      if (static_cast<uint32_t>(b / OWN) == grp) {
+        f32x4 v = acc[b / JN][b % JN];
+#pragma unroll
+        for (uint32_t g = 0; g < KG; ++g)
+          if (g != grp) v += red[(g * (IM * JN) + b) * THREADS + tid];
+        acc[b / JN][b % JN] = v;
+      }
+    }
+  }
+  // acc[i][j][e] = C[m][n], m = m0 + wm + 16i + lane%16, n = n0 + wn + 16j + 4(lane/16) + e.
+  const uint32_t mr = m0 + wm + (lane & 15u), nc = n0 + wn + 4u * (lane >> 4);
+#pragma unroll
+  for (int b = 0; b < IM * JN; ++b) {
+    const int i = b / JN, j = b % JN;
+    if (static_cast<uint32_t>(b / OWN) != grp) continue;
+    const uint32_t m = mr + 16u * i, n = nc + 16u * j;
+    if (m >= M) continue;
+    float* c = C + static_cast<uint64_t>(m) * N + n;
+    if (n + 4u <= N) {
+      f32x4_a4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = epi(acc[i][j][e], m, n + e);
+      *reinterpret_cast<f32x4_a4*>(c) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) c[e] = epi(acc[i][j][e], m, n + e);
+    }
+  }
+}
+
+// The contraction's tiles that gemm_bf16_4w and gemm_bf16_256_w8 do not
+// take, 8 waves per workgroup: 128x128 of C, or, when 128x128 tiles would
+// leave half the CUs without one (`parts` >= 2 workgroups were launched per
+// tile) or M <= 64, 64x128 (1024 x 2048 x 4096: 31 us against 42, 1001 x 1501
+// x 1003: 12 against 16; from 256 tiles on the taller tile reads less:
+// 2048 x 2048 x 4096 44 us against 53).
+template <bool B_NK, typename Epi, bool F16, uint64_t WHOLE_MIN>
+__device__ __forceinline__ void gemm16_any(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
+                                           float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
+                                           uint32_t batch, uint32_t tile, uint32_t part, uint32_t parts) {
+  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * 64 * 256];
+  const uint32_t tiles_m = (M - 1u) / 128u + 1u, tiles_n = (N - 1u) / 128u + 1u;
+  uint32_t tm, tn;
+  gemm_tile_coords(tiles_m, tiles_n, &tm, &tn, tile);
+  const uint32_t m0 = tm * 128u + part * 64u, n0 = tn * 128u;
+  if (part >= 2u || m0 >= M) return;
+  if (tm / 2u < M / 256u && tn / 2u < N / 256u && gemm16_direct_k(N, K) && gemm16_on_whole_tiles<WHOLE_MIN>(M, N, batch))
+    return;
+  const uint16_t* A16 = reinterpret_cast<const uint16_t*>(A);
+  const uint16_t* B16 = reinterpret_cast<const uint16_t*>(B);
+  if (K < 8u || (!B_NK && N < 8u)) {
+    if (part == 0u) gemm16_tile<128, 128, 2, 4, 1, 1, B_NK, F16, true>(A16, B16, C, M, N, K, epi, m0, n0, lds);
+  } else if (parts >= 2u || M <= 64u) {
+    gemm16_tile<64, 128, 2, 4, 1, 2, B_NK, F16, false>(A16, B16, C, M, N, K, epi, m0, n0, lds);
+  } else {
+    gemm16_tile<128, 128, 2, 4, 1, 2, B_NK, F16, false>(A16, B16, C, M, N, K, epi, m0, n0, lds);
+  }
 }
 
 // -------------------------------------------- bf16 path, 8 waves per tile
@@ -405,45 +488,23 @@ __device__ __forceinline__ void gemm_bf16_256(const __bf16* __restrict__ A, cons
 __device__ __forceinline__ uint32_t swz_rows32(uint32_t row, uint32_t cg) {
   return row * 32u + ((cg ^ (((row >> 3) & 1u) << 1)) << 3);
 }
-__device__ __forceinline__ uint32_t kn_xor(uint32_t k) { return ((k & 3u) | (((k >> 3) & 1u) << 2)) << 1; }
-__device__ __forceinline__ uint32_t swz_kn16(uint32_t k, uint32_t n) {
-  return k * 256u + (((n >> 3) ^ kn_xor(k)) << 3) + (n & 7u);
-}
 
-// B operand of v_mfma_f32_16x16x32_bf16 (lane l: column n_col0 + l%16,
-// k = 8(l/16) .. +8) from a [K][N] slice with the gfx950 transposing read
-// ds_read_b64_tr_b16: within each 16-lane group, lane j points at four
-// consecutive values R_j of one k row and lane i receives
-// [R_{i/4}[i%4], R_{4+i/4}[i%4], R_{8+i/4}[i%4], R_{12+i/4}[i%4]]. With lane j
-// addressing row kb + j/4, columns n_col0 + 4(j%4), lane i gets
-// B[kb + e][n_col0 + i] for e = 0..3; a second read at kb + 4 completes its 8.
-__device__ __forceinline__ bf16x8 frag_b16_tr(const uint16_t* Bs, uint32_t n_col0, uint32_t lane) {
-  const uint32_t g = lane >> 4, j = lane & 15u;
-  const uint32_t k = 8u * g + (j >> 2), n = n_col0 + 4u * (j & 3u);
-  const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(Bs + swz_kn16(k, n)));
-  const i16x4 hi =
-      __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(Bs + swz_kn16(k + 4u, n)));
-  typedef short i16x8 __attribute__((ext_vector_type(8)));
-  const i16x8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  return __builtin_bit_cast(bf16x8, v);
-}
-
-// Every other tile returns at once: gemm_bf16_256<..., SKIP_DMA> takes them.
+// Every other tile returns at once: gemm16_any takes them.
 // With K % 64 == 0 and K >= 256 the launch takes gemm_bf16_4w instead (4
 // waves of 128x128, A in 64-deep slices, below).
-template <bool B_NK, typename Epi, uint32_t STAGES = 4, bool F16 = false>
+template <bool B_NK, typename Epi, bool F16, uint64_t WHOLE_MIN, uint32_t STAGES = 4>
 __device__ __forceinline__ void gemm_bf16_256_w8(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
                                                  float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
-                                                 uint32_t tile = ~0u) {
+                                                 uint32_t batch, uint32_t tile) {
   static_assert(STAGES == 4 || STAGES == 5, "a ring of 4 or 5 slices (160 KiB of LDS at most)");
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   constexpr uint32_t BM = 256, BN = 256, BK = 32, SLICE = 256u * BK;
   __shared__ __attribute__((aligned(16))) uint16_t lds[STAGES * 2 * SLICE];
-  const uint32_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   uint32_t tm, tn;
-  gemm_tile_coords(tiles_m, tiles_n, &tm, &tn, tile == ~0u ? blockIdx.x : tile);
+  if (!gemm16_direct_k(N, K) || !gemm16_on_whole_tiles<WHOLE_MIN>(M, N, batch) ||
+      !gemm16_whole_coords(M, N, tile, &tm, &tn))
+    return;  // gemm16_any takes it
   const uint32_t m0 = tm * BM, n0 = tn * BN;
-  if (!gemm_bf16_dma_tile(m0, n0, M, N, K)) return;  // gemm_bf16_256<..., SKIP_DMA> takes it
   // The wave index is uniform over the wave: computed in a scalar register,
   // the LDS destination of every direct-to-LDS load (the m0 operand) is a
   // scalar value, with no readfirstlane per load.
@@ -470,7 +531,7 @@ __device__ __forceinline__ void gemm_bf16_256_w8(const __bf16* __restrict__ A, c
       offb[q] = r * K + c * 8u;
     } else {
       const uint32_t k = slot >> 5, sp = slot & 31u;  // [32][256]: 32 slots per row
-      offb[q] = k * N + ((sp ^ kn_xor(k)) << 3);
+      offb[q] = k * N + ((sp ^ kn_slot_xor<256>(k)) << 3);
     }
   }
   uint16_t* ldsp = lds;
@@ -493,7 +554,7 @@ __device__ __forceinline__ void gemm_bf16_256_w8(const __bf16* __restrict__ A, c
     if constexpr (B_NK)
       return *reinterpret_cast<const bf16x8*>(&Bs[swz_rows32(wn + j * 16u + (lane & 15u), lane >> 4)]);
     else
-      return frag_b16_tr(Bs, wn + j * 16u, lane);
+      return frag_b16_tr<256>(Bs, wn + j * 16u, lane);
   };
   bf16x8 fa[4], fh[4], fb0[4], fb1[4];  // A rows 0-63, A rows 64-127, the two B sets
   auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
@@ -697,19 +758,17 @@ __device__ __forceinline__ void mfma16_bf16_acc(f32x4_t& c, const bf16x8& b, con
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(b), "v"(a));
 }
 
-__device__ __forceinline__ uint32_t swz_rows64(uint32_t row, uint32_t g) { return row * 64u + ((g ^ (row & 6u)) << 3); }
-
-template <bool B_NK, typename Epi, bool F16 = false>
+template <bool B_NK, typename Epi, bool F16, uint64_t WHOLE_MIN>
 __device__ __forceinline__ void gemm_bf16_4w(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
                                              float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
-                                             uint32_t tile = ~0u) {
+                                             uint32_t batch, uint32_t tile) {
   constexpr uint32_t BM = 256, BN = 256, ASL = 256u * 64u, BSL = 256u * 32u;
   __shared__ __attribute__((aligned(16))) uint16_t lds[3 * ASL + 4 * BSL];
-  const uint32_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   uint32_t tm, tn;
-  gemm_tile_coords(tiles_m, tiles_n, &tm, &tn, tile == ~0u ? blockIdx.x : tile);
+  if (!gemm16_direct_k(N, K) || K % 64u != 0u || K < 256u || !gemm16_on_whole_tiles<WHOLE_MIN>(M, N, batch) ||
+      !gemm16_whole_coords(M, N, tile, &tm, &tn))
+    return;  // gemm16_any takes it
   const uint32_t m0 = tm * BM, n0 = tn * BN;
-  if (!gemm_bf16_dma_tile(m0, n0, M, N, K) || K % 64u != 0u || K < 256u) return;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t wm = (wave >> 1) * 128u, wn = (wave & 1u) * 128u;
   const uint16_t* __restrict__ A16 = reinterpret_cast<const uint16_t*>(A);
@@ -741,7 +800,7 @@ __device__ __forceinline__ void gemm_bf16_4w(const __bf16* __restrict__ A, const
       offb[q] = r * K + c * 8u;
     } else {
       const uint32_t k = slot >> 5, sp = slot & 31u;  // [32][256]: 32 slots per row
-      offb[q] = k * N + ((sp ^ kn_xor(k)) << 3);
+      offb[q] = k * N + ((sp ^ kn_slot_xor<256>(k)) << 3);
     }
   }
   uint16_t* ldsp = lds;
@@ -765,7 +824,7 @@ __device__ __forceinline__ void gemm_bf16_4w(const __bf16* __restrict__ A, const
     if constexpr (B_NK)
       return *reinterpret_cast<const bf16x8*>(&Bs[swz_rows32(wn + j * 16u + (lane & 15u), lane >> 4)]);
     else
-      return frag_b16_tr(Bs, wn + j * 16u, lane);
+      return frag_b16_tr<256>(Bs, wn + j * 16u, lane);
   };
   bf16x8 a0s[8], b0s[8], a1s[8], b1s[8];  // two fragment sets: this step's and the next one's
   auto fence = []() { __builtin_amdgcn_sched_barrier(0); };

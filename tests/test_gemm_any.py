@@ -1,0 +1,159 @@
+"""The 16-bit contractions' any-shape kernel (gemm16_any): which launches take
+it, and its results at the sizes where it can go wrong.
+
+Host-only: every tile of a plane has exactly one owner. The direct-to-LDS
+kernels and the any-shape kernel decide on the device with the same rule
+(gemm16_on_whole_tiles, compiled here for the host); the plan's guards may
+only skip a launch that the rule leaves idle.
+
+GPU: small-integer operands, so every product and partial sum is exact in
+fp32 and every output must equal the float64 product."""
+import os
+import random
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+import oracle
+from helpers import canaries, compiled, host, out_dev, run, to_dev
+from tcacomp_amd.compiler import TensorDesc
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+WHOLE_MIN = 128 << 16
+
+
+@pytest.fixture(scope="module")
+def on_whole_tiles(tmp_path_factory):
+    out = tmp_path_factory.mktemp("gemm_edge") / "gemm_edge"
+    hipcc = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    r = subprocess.run([hipcc, "--offload-arch=gfx950", "-O1", "-I",
+                        os.path.join(REPO, "tcacomp_amd", "csrc", "include"),
+                        os.path.join(REPO, "tests", "c", "gemm_edge.hip"), "-o", str(out)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+    def ask(shapes):
+        p = subprocess.run([str(out)], input="".join("%d %d %d %d\n" % s for s in shapes), capture_output=True,
+                           text=True, timeout=60)
+        assert p.returncode == 0, p.stderr
+        return [bool(int(v)) for v in p.stdout.split()]
+    return ask
+
+
+def _shapes(rng, count):
+    for _ in range(count):
+        m, n, k = (max(1, int(2 ** rng.uniform(0, 14))) for _ in range(3))
+        if rng.random() < 0.6:
+            m, n = max(256, m // 256 * 256), max(256, n // 256 * 256)
+        if rng.random() < 0.7:
+            k = max(32, k // 32 * 32)
+        if rng.random() < 0.3:
+            n = max(8, n // 8 * 8)
+        b = rng.choice((1, 1, 1, 2, 7))
+        if m * n > 1 << 20 and max(m * n, m * k, n * k) * b < 1 << 31:
+            yield m, n, k, b
+
+
+@pytest.mark.parametrize("name", ["bmm_bf16", "bmm_bf16_nt"])
+def test_every_tile_has_one_kernel(on_whole_tiles, name):
+    from tcacomp_amd import compiler, programs
+    prog = compiler.CompiledProgram(name, programs.CONFIG_PROGRAMS[name]().emit(), "")
+    shapes = list(_shapes(random.Random(11), 3000))
+    shapes += [(2048, 4096, 4096, 1), (2048, 4096 - 256, 4096, 1), (257, 36266, 512, 1), (4096, 4096, 192, 1),
+               (4352, 4096, 64, 1), (4100, 4096, 4096, 1), (1024, 1025, 4096, 8), (2048, 2048, 1024, 2)]
+    assert len(shapes) > 500
+    for (m, n, k, b), whole in zip(shapes, on_whole_tiles(shapes)):
+        sel = prog.selected_symbols([TensorDesc(0x1000, (b, m, k), 2),
+                                     TensorDesc(0x1000, (b, n, k) if name.endswith("nt") else (b, k, n), 2),
+                                     TensorDesc(0x1000, (b, m, n), 0)])
+        sel = {s[len("tca_%s_k0" % name):] for s in sel}
+        has_whole = whole and m >= 256 and n >= 256
+        edges = not has_whole or m % 256 != 0 or n % 256 != 0
+        if has_whole:  # the kernel the K rule names
+            assert ("_w" if k % 64 == 0 and k >= 256 else "_v") in sel, (m, n, k, b, sel)
+        if edges:
+            assert "" in sel, (m, n, k, b, sel)
+        assert not {"_s", "_sm"} & sel
+
+
+# M, N, K: remainders of the 64- and 128-row tiles and of the 64-deep slice, K
+# of one element, one chunk and one slice either side, rows of every
+# alignment, [K][N] rows shorter than a chunk, few rows, few columns, and
+# planes that take the 64-row tile (few 128x128 tiles), the 128-row tile
+# (many) and whole 256x256 tiles with edges.
+SHAPES = [(1025, 1025, 1), (1025, 1027, 7), (1030, 1029, 8), (1031, 1026, 9), (1089, 1032, 63), (1024, 1032, 64),
+          (1152, 1153, 65), (1100, 1101, 127), (1100, 1102, 128), (1100, 1104, 129), (1281, 1031, 200),
+          (200001, 6, 70), (210000, 5, 72), (131080, 9, 257), (3, 400000, 65), (64, 16500, 130), (65, 16500, 66),
+          (2100, 2300, 333), (2048, 2049, 320), (3100, 3330, 96), (4100, 4104, 256), (3000, 5888, 64)]
+
+
+def _say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def _dev16(a, gpu, f16):
+    import torch
+    if f16:
+        return to_dev(a.astype(np.float16), gpu)
+    return to_dev(oracle.to_bf16_bits(a).view(np.int16), gpu).view(torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("name", ["gemm_bf16", "gemm_bf16_nt", "gemm_f16"])
+def test_any_shape_exact(gpu, M, N, K, name):
+    _say("gemm any", name, M, N, K)
+    nt, f16 = name.endswith("_nt"), name == "gemm_f16"
+    rng = np.random.default_rng(M * 7 + N * 3 + K)
+    a = rng.integers(-4, 5, (M, K)).astype(np.float32)
+    b = rng.integers(-4, 5, (K, N)).astype(np.float32)
+    p = compiled(name)
+    bd = np.ascontiguousarray(b.T) if nt else b
+    sel = p.selected_symbols([TensorDesc(0x1000, (M, K), 1 if f16 else 2), TensorDesc(0x1000, bd.shape, 1 if f16 else 2),
+                              TensorDesc(0x1000, (M, N), 0)])
+    assert "tca_%s_k0" % name in sel, sel
+    c = out_dev((M, N), gpu)
+    run(p, [_dev16(a, gpu, f16), _dev16(bd, gpu, f16), c])
+    got = host(c)
+    assert canaries(got) == 0
+    assert np.array_equal(got, a @ b)  # exact in fp32: partial sums below 2^24
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["bmm_bf16", "bmm_bf16_nt"])
+@pytest.mark.parametrize("B,M,N,K", [(3, 1025, 1027, 77), (2, 130, 8300, 64), (9, 1024, 1152, 96)])
+def test_any_shape_batched_exact(gpu, name, B, M, N, K):
+    _say("bmm any", name, B, M, N, K)
+    nt = name.endswith("_nt")
+    rng = np.random.default_rng(B + M + N + K)
+    a = rng.integers(-4, 5, (B, M, K)).astype(np.float32)
+    b = rng.integers(-4, 5, (B, K, N)).astype(np.float32)
+    c = out_dev((B, M, N), gpu)
+    run(compiled(name), [_dev16(a, gpu, False), _dev16(b.transpose(0, 2, 1) if nt else b, gpu, False), c])
+    assert np.array_equal(host(c), np.matmul(a, b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["gemm_bf16", "gemm_bf16_nt"])
+def test_nonfinite_operands_stay_in_their_rows(gpu, name):
+    """Infinities and NaN at the ends of rows: a chunk loaded from before the
+    end of its row must not bring a neighbour's values in, nor a clamped row
+    leave its tile."""
+    import torch
+    M, N, K = 1030, 1029, 75
+    nt = name.endswith("_nt")
+    rng = np.random.default_rng(3)
+    a = rng.integers(-4, 5, (M, K)).astype(np.float32)
+    b = rng.integers(-4, 5, (K, N)).astype(np.float32)
+    a[5, K - 1], a[M - 1, 0], b[K - 1, 7], b[0, N - 1] = np.inf, np.nan, -np.inf, np.nan
+    with np.errstate(invalid="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+    c = out_dev((M, N), gpu)
+    ta = torch.from_numpy(a).to(gpu).to(torch.bfloat16)
+    tb = torch.from_numpy(np.ascontiguousarray(b.T) if nt else b).to(gpu).to(torch.bfloat16)
+    run(compiled(name), [ta, tb, c])
+    assert np.array_equal(host(c), want.astype(np.float32), equal_nan=True)
