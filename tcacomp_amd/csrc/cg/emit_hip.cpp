@@ -357,16 +357,28 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
     const std::string Ms = g.dims[m.m].name, Ns = g.dims[m.n].name, Ks = g.dims[m.k].name;
     const uint32_t kKcMin = bf16 ? 1024u : 512u;  // 4 steps per wave and chunk
     const uint32_t kBlocks = 512u;                // two 16-wave workgroups per CU
+    // Workgroups past the tiles return at once, but dispatching one costs
+    // 5.5 ns (16 waves each): 64 batches of 1000 x 1000 planes, 65536 tiles of
+    // 32x32 on 4096 of 128x128, spent 250 us on it.
+    const uint32_t kStride = 1024u;
     const std::string part = "__gemmpart" + std::to_string(nest), pdim = "__gemmdim" + std::to_string(nest);
     out->extra_dims.push_back(pdim + " " + std::to_string(uint64_t{kBlocks} * 1024u));
     out->extra_tensors.push_back(part + " f32 local 1 " + pdim);
     const std::string psig = ",\n    float* __restrict__ pw /* " + part + " */";
     auto body = [&](bool merge) {
       std::ostringstream b;
-      b << epi.str() << "  const uint32_t tiles = ((M + 31u) / 32u) * ((N + 31u) / 32u);\n"
-        << "  const uint32_t T = " << (batched ? ExtentExpr(g, m.batch) + " * tiles" : std::string("tiles")) << ";\n"
-        << "  const uint32_t P = tca::hip::gemm_split_chunks(K, T, " << kKcMin << "u, " << kBlocks << "u);\n"
-        << (merge ? "  const uint32_t gt = blockIdx.x;\n" : "  const uint32_t gt = blockIdx.x % T, p = blockIdx.x / T;\n");
+      const std::string h16 = bf16 ? "true" : "false";
+      // P from the 32x32 tiles, as the split record computes it.
+      b << epi.str() << "  const uint32_t P = tca::hip::gemm_split_chunks(K, " << nb
+        << " * (((M + 31u) / 32u) * ((N + 31u) / 32u)), " << kKcMin << "u, " << kBlocks << "u);\n";
+      if (merge)
+        b << "  const uint32_t tiles = ((M + 31u) / 32u) * ((N + 31u) / 32u), T = " << nb << " * tiles, gt = blockIdx.x;\n";
+      else
+        b << "  const auto shape = tca::hip::gemm_small_shape<" << h16 << ", " << nk << ">(M, N, K, " << nb << ", P);\n"
+          << "  const uint32_t tiles = ((M - 1u) / shape.m + 1u) * ((N - 1u) / shape.n + 1u), T = " << nb << " * tiles;\n"
+          << "  for (uint32_t w = blockIdx.x; w < T * P; w += gridDim.x) {\n"
+          << "  if (w != blockIdx.x) __syncthreads();\n"
+          << "  const uint32_t p = w / T, gt = tca::hip::gemm_small_tile(w - p * T, T);\n";
       std::string a = "t" + std::to_string(ta), bo = "t" + std::to_string(tb), cc = "t" + std::to_string(tc);
       if (batched) {
         b << "  const uint32_t bb = gt / tiles, tile = gt - bb * tiles;\n";
@@ -377,11 +389,10 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
         b << "  const uint32_t tile = gt;\n";
       }
       if (merge)
-        b << "  tca::hip::gemm_small_merge(" << cc << ", pw, M, N, epi, tile, gt, T, P);\n}\n\n";
+        b << "  tca::hip::gemm_small_merge<" << h16 << ">(" << cc << ", pw, M, N, epi, tile, gt, T, P);\n}\n\n";
       else
-        b << "  tca::hip::gemm_small<" << (bf16 ? "true" : "false") << ", " << (m.b_nk ? "true" : "false")
-          << ", decltype(epi)" << (f16 ? ", true" : "") << ">(" << a << ", " << bo << ", " << cc
-          << ", pw, M, N, K, epi, tile, gt, T, p, P);\n}\n\n";
+        b << "  tca::hip::gemm_small<" << h16 << ", " << nk << ", decltype(epi)" << (f16 ? ", true" : "") << ">(" << a
+          << ", " << bo << ", " << cc << ", pw, M, N, K, epi, shape, tile, gt, T, p, P);\n  }\n}\n\n";
       return b.str();
     };
     o << "extern \"C\" __global__ void __launch_bounds__(1024) " << symbol << "_s(\n    " << signature << psig
@@ -409,6 +420,7 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
                " when the tiles are fewer than " + std::to_string(kBlocks) + "; M*N <= " +
                std::to_string(kGemmSmallMax) + ")" + orient;
     GemmKernel sm = s;
+    s.stride = kStride;
     sm.suffix = "_sm";
     sm.split = splitRec + " 1 " + splitTerms;
     sm.detail = ty + " small-tile merge: the P chunk partials of each 32x32 tile added in chunk order (P > 1 only)";
@@ -995,6 +1007,7 @@ class Emitter {
     std::vector<std::string> unless;  // skip guards: the kernel is skipped when all of them hold
     std::string pack;               // packed row kernel: "<dim> <epl> <min block>"
     std::string split;              // row-split reduction: "<dim> <rows-min> <blocks> <merge> <n> <terms>"
+    uint32_t stride = 0;
   };
 
   // -------------------------------------------------------------- analysis
@@ -4794,6 +4807,7 @@ class Emitter {
       k.unless = gk.unless;
       for (const auto& a : gk.extra_args) k.args.push_back(a);
       k.split = gk.split;
+      k.stride = gk.stride;
       AddKernel(k, Family::Gemm, n.chains, gk.detail);
     }
     return true;
@@ -4833,6 +4847,7 @@ class Emitter {
       for (const auto& a : k.args) p << "arg " << a << "\n";
       if (!k.pack.empty()) p << "pack " << k.pack << "\n";
       if (!k.split.empty()) p << "split " << k.split << "\n";
+      if (k.stride != 0) p << "stride " << k.stride << "\n";
       for (const auto& w : k.when) p << "when " << w << "\n";
       for (const auto& w : k.unless) p << "unless " << w << "\n";
     }

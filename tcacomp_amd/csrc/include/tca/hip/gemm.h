@@ -37,6 +37,7 @@
 namespace tca {
 namespace hip {
 
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -84,6 +85,15 @@ __device__ __forceinline__ void gemm_tile_coords(uint32_t tiles_m, uint32_t tile
 }
 
 // ----------------------------------------------- 16-bit path, any shape
+// The thread index, computed where it is used: inside a loop over tiles the
+// compiler would otherwise keep every lane address of every tile shape in
+// registers across the loop, and spill them.
+__device__ __forceinline__ uint32_t thread_here() {
+  uint32_t t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // Unaligned 16-byte accesses: gfx950 serves a 16-byte vector load or store
 // at any element address (the amdhsa unaligned access mode), so rows whose
 // length is not a multiple of the vector still move 16 bytes per lane.
@@ -145,6 +155,9 @@ __device__ __forceinline__ bool gemm16_whole_coords(uint32_t M, uint32_t N, uint
   return true;
 }
 
+__device__ __forceinline__ uint32_t swz_rows32(uint32_t row, uint32_t cg) {
+  return row * 32u + ((cg ^ (((row >> 3) & 1u) << 1)) << 3);
+}
 __device__ __forceinline__ uint32_t swz_rows64(uint32_t row, uint32_t g) { return row * 64u + ((g ^ (row & 6u)) << 3); }
 // The 16-byte slot of a [K][BN] slice's row k is XORed with this (measured
 // bank cycles at gemm_bf16_256_w8): rows of 256 bytes and more cover the 64
@@ -152,7 +165,8 @@ __device__ __forceinline__ uint32_t swz_rows64(uint32_t row, uint32_t g) { retur
 template <uint32_t BN>
 __device__ __forceinline__ uint32_t kn_slot_xor(uint32_t k) {
   if constexpr (BN >= 128u) return ((k & 3u) | (((k >> 3) & 1u) << 2)) << 1;
-  else return (((k >> 1) & 1u) | (((k >> 3) & 1u) << 1)) << 1;
+  else if constexpr (BN == 64u) return (((k >> 1) & 1u) | (((k >> 3) & 1u) << 1)) << 1;
+  else return ((k >> 3) & 1u) << 1;  // 64-byte rows: four to the banks
 }
 template <uint32_t BN>
 __device__ __forceinline__ uint32_t swz_kn(uint32_t k, uint32_t n) {
@@ -201,18 +215,18 @@ __device__ __forceinline__ bf16x8 frag_b16_tr(const uint16_t* Bs, uint32_t n_col
 // apart 44, operands loaded straight into a 4-deep LDS ring 45 (8 waves) and
 // 55 (4 waves). `TINY` (K-contiguous rows or
 // [K][N] rows shorter than one chunk) loads those element by element.
-// `lds` holds KG * 2 * 64 * (BM + BN) values.
+// `lds` holds KG * 2 * 64 * (BM + BN) values; `thread` is threadIdx.x.
 template <uint32_t BM, uint32_t BN, uint32_t WGM, uint32_t WGN, uint32_t KG, int D, bool B_NK, bool F16, bool TINY,
           typename Epi>
 __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                                             float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
-                                            uint32_t m0, uint32_t n0, uint16_t* lds) {
+                                            uint32_t m0, uint32_t n0, uint16_t* lds, uint32_t thread) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   constexpr uint32_t THREADS = 64u * WGM * WGN, TM = BM / WGM, TN = BN / WGN;
   constexpr int IM = TM / 16, JN = TN / 16, CA = BM * 8 / THREADS, CB = BN * 8 / THREADS;
   static_assert(CA >= 1 && CB >= 1 && (D == 1 || D % 2 == 0), "whole chunks per thread; the buffer of a slice is static");
   constexpr uint32_t ASL = BM * 64u, BUF = ASL + BN * 64u;
-  const uint32_t lane = threadIdx.x & 63u, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t lane = thread & 63u, wave_id = __builtin_amdgcn_readfirstlane(thread >> 6);
   const uint32_t grp = wave_id / (WGM * WGN), wave = wave_id % (WGM * WGN), tid = wave * 64u + lane;
   const uint32_t wm = (wave / WGN) * TM, wn = (wave % WGN) * TN;
   uint16_t* glds = lds + grp * (2u * BUF);
@@ -442,11 +456,11 @@ __device__ __forceinline__ void gemm16_any(const __bf16* __restrict__ A, const _
   const uint16_t* A16 = reinterpret_cast<const uint16_t*>(A);
   const uint16_t* B16 = reinterpret_cast<const uint16_t*>(B);
   if (K < 8u || (!B_NK && N < 8u)) {
-    if (part == 0u) gemm16_tile<128, 128, 2, 4, 1, 1, B_NK, F16, true>(A16, B16, C, M, N, K, epi, m0, n0, lds);
+    if (part == 0u) gemm16_tile<128, 128, 2, 4, 1, 1, B_NK, F16, true>(A16, B16, C, M, N, K, epi, m0, n0, lds, threadIdx.x);
   } else if (parts >= 2u || M <= 64u) {
-    gemm16_tile<64, 128, 2, 4, 1, 2, B_NK, F16, false>(A16, B16, C, M, N, K, epi, m0, n0, lds);
+    gemm16_tile<64, 128, 2, 4, 1, 2, B_NK, F16, false>(A16, B16, C, M, N, K, epi, m0, n0, lds, threadIdx.x);
   } else {
-    gemm16_tile<128, 128, 2, 4, 1, 2, B_NK, F16, false>(A16, B16, C, M, N, K, epi, m0, n0, lds);
+    gemm16_tile<128, 128, 2, 4, 1, 2, B_NK, F16, false>(A16, B16, C, M, N, K, epi, m0, n0, lds, threadIdx.x);
   }
 }
 
@@ -485,9 +499,6 @@ __device__ __forceinline__ void gemm16_any(const __bf16* __restrict__ A, const _
 //   [K][N] B (512-byte rows): 16-byte slot n/8 of row k at
 //     (n/8) ^ 2*((k%4) + 4*((k/8)%2)); a transposing fragment read takes rows
 //     8g..8g+3 (+4) of one 16-column block for lane group g.
-__device__ __forceinline__ uint32_t swz_rows32(uint32_t row, uint32_t cg) {
-  return row * 32u + ((cg ^ (((row >> 3) & 1u) << 1)) << 3);
-}
 
 // Every other tile returns at once: gemm16_any takes them.
 // With K % 64 == 0 and K >= 256 the launch takes gemm_bf16_4w instead (4
@@ -749,7 +760,6 @@ __device__ __forceinline__ void gemm_bf16_256_w8(const __bf16* __restrict__ A, c
 //   assembly: no VALU writes an MFMA source register), whose completion
 //   s_waitcnt covers; an MFMA's accumulator is written again only by the
 //   64th MFMA after it.
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 template <bool F16 = false>
 __device__ __forceinline__ void mfma16_bf16_acc(f32x4_t& c, const bf16x8& b, const bf16x8& a) {
   if constexpr (F16)
@@ -1347,18 +1357,20 @@ __device__ __forceinline__ void gemm_f32_4w(const float* __restrict__ A, const f
 //     p writes its sum to a partial scratch [P][tiles][1024] and a second
 //     kernel (gemm_small_merge) adds the P partials in chunk order.
 // Every order is fixed, so the result does not depend on the schedule.
-// Operands go from memory straight into the MFMA operand registers (no LDS
-// staging: the waves of a workgroup read disjoint k, so nothing is shared
-// inside it; neighbouring tiles share panels through the L2):
+// Operands go from memory straight into the MFMA operand registers (no
+// staging of tiles: the waves of a workgroup read disjoint k, so nothing is
+// shared inside it; neighbouring tiles share panels through the L2):
 //   f32 step at k0, lane l (r = l % 32, h = l / 32): A[m0+r][k0+4h+e] and
 //   B[k0+4h+e][n0+r] for e = 0..3, one float4 where the operand is
 //   K-contiguous; MFMA e sums k0+e (lanes 0-31) and k0+4+e (lanes 32-63), so
 //   a step sums each of its 8 k once;
-//   16-bit step at k0: lane l holds A[m0+r][k0+8h .. +7] and
-//   B[k0+8h .. +7][n0+r] (the 32x32x16 operand layout), one MFMA.
-// Result element i of lane l is C[m0 + 8(i/4) + 4(l/32) + i%4][n0 + l%32];
+//   16-bit step: small16_steps.
+// f32 result element i of lane l is C[m0 + 8(i/4) + 4(l/32) + i%4][n0 + l%32];
 // a wave's tile goes to LDS element-major (word i*64 + l: conflict-free) and
 // thread t = i*64 + l of the workgroup sums word t over the waves.
+// Tiles are numbered down the columns of tiles, and the workgroups of one
+// XCD (every eighth) take a run of them: the tiles that read one panel of B
+// share an L2.
 constexpr uint32_t kSmallWaves = 16;
 
 // P chunks of K for `tiles` output tiles: enough workgroups to reach
@@ -1374,12 +1386,196 @@ __host__ __device__ __forceinline__ uint32_t gemm_split_chunks(uint32_t k, uint3
 }
 
 // Coordinates (row, column) inside a 32x32 tile of the value thread t holds
-// after the wave merge.
+// after the wave merge: its word of the MFMA result for f32, row-major for
+// 16-bit inputs.
+template <bool H16>
 __device__ __forceinline__ uint32_t small_row(uint32_t t) {
+  if constexpr (H16) return t >> 5;
   const uint32_t i = t >> 6, l = t & 63u;
   return 8u * (i >> 2) + 4u * (l >> 5) + (i & 3u);
 }
 __device__ __forceinline__ uint32_t small_col(uint32_t t) { return t & 31u; }
+
+// The tile that workgroup `i` of a chunk's T takes.
+__device__ __forceinline__ uint32_t gemm_small_tile(uint32_t i, uint32_t T) {
+  const uint32_t x = i & 7u, q = T >> 3, r = T & 7u;
+  return x * q + (x < r ? x : r) + (i >> 3);
+}
+
+// A wave's 32-deep k steps (s_begin + wave, + 16, ...) of a 16 IM x 32 tile,
+// 16-bit inputs. Four lanes load the 64 bytes of a row (loaded in the MFMA
+// operand's layout, 16 rows to 16 consecutive lanes, every lane of a quad
+// touches another line and the address unit takes 64 cycles per load instead
+// of 16: 16 x 16384 x 16384 ran at 3.5-4.1 TB/s); the step goes through the
+// wave's own 4 KiB of LDS (`stage`: 32 rows of A at a time, then B) into
+// operand layout. No load is guarded (clamped and moved into place as in
+// gemm16_tile; K >= 8, and N >= 8 for [K][N]). D steps are in flight; the main
+// loop's loads are unconditional, as there.
+template <int IM, int D, bool B_NK, bool F16>
+__device__ __forceinline__ void small16_steps(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                                              uint32_t M, uint32_t N, uint32_t K, uint32_t m0, uint32_t n0,
+                                              uint32_t s_begin, uint32_t s_end, uint16_t* stage, f32x4_t (&acc)[IM][2]) {
+  const uint32_t thread = thread_here(), lane = thread & 63u, wave = __builtin_amdgcn_readfirstlane(thread >> 6);
+  const uint32_t r = lane >> 2, kg = (lane & 3u) * 8u;  // as loaded
+  const uint16_t *pa[IM], *pb[2];
+  uint32_t bsh = 0u;
+#pragma unroll
+  for (int i = 0; i < IM; ++i) {
+    const uint32_t m = m0 + r + 16u * i;
+    pa[i] = A + static_cast<uint64_t>(m < M ? m : M - 1u) * K;
+  }
+  if constexpr (B_NK) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t n = n0 + r + 16u * j;
+      pb[j] = B + static_cast<uint64_t>(n < N ? n : N - 1u) * K;
+    }
+  } else {
+    const uint32_t n = n0 + kg, at = n < N - 8u ? n : N - 8u;
+    bsh = n - at;
+    pb[0] = pb[1] = B + at;
+  }
+  u32x4 xa[D][IM], xb[D][2];
+  auto load = [&](int d, uint32_t s) {
+    const uint32_t k = s * 32u + kg, kc = k < K - 8u ? k : K - 8u;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (B_NK) {
+        xb[d][j] = load16_any(pb[j] + kc);
+      } else {
+        const uint32_t kr = s * 32u + r + 16u * j;
+        xb[d][j] = load16_any(pb[0] + static_cast<uint64_t>(kr < K ? kr : K - 1u) * N);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < IM; ++i) xa[d][i] = load16_any(pa[i] + kc);
+  };
+#pragma unroll
+  for (int i = 0; i < IM; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  const bool edge_n = !B_NK && n0 + 32u > N;
+  auto mma = [&](auto last, int d, uint32_t s) {
+    if (decltype(last)::value && s * 32u + 32u > K) {  // the short last step
+      const uint32_t k = s * 32u + kg, n = k - (k < K - 8u ? k : K - 8u);
+#pragma unroll
+      for (int i = 0; i < IM; ++i) xa[d][i] = shift_down16(xa[d][i], n);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if constexpr (B_NK) xb[d][j] = shift_down16(xb[d][j], n);
+        else if (s * 32u + r + 16u * j >= K) xb[d][j] = u32x4{0u, 0u, 0u, 0u};
+      }
+    }
+    if constexpr (!B_NK) {
+      if (edge_n) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) xb[d][j] = shift_down16(xb[d][j], bsh);
+      }
+    }
+    // LDS operations of one wave complete in order: a region is rewritten
+    // behind the reads of what it held.
+    uint16_t* bst = stage + 1024;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      *reinterpret_cast<u32x4*>(&bst[B_NK ? swz_rows32(r + 16u * j, lane & 3u) : swz_kn<32>(r + 16u * j, kg)]) = xb[d][j];
+    bf16x8 fb[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (B_NK) fb[j] = *reinterpret_cast<const bf16x8*>(&bst[swz_rows32(16u * j + (lane & 15u), lane >> 4)]);
+      else fb[j] = frag_b16_tr<32>(bst, 16u * j, lane);
+    }
+#pragma unroll
+    for (int h = 0; h < IM / 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<u32x4*>(&stage[swz_rows32(r + 16u * i, lane & 3u)]) = xa[d][2 * h + i];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const bf16x8 fa = *reinterpret_cast<const bf16x8*>(&stage[swz_rows32(16u * i + (lane & 15u), lane >> 4)]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[2 * h + i][j] = mfma_16x16x32_16b<F16>(fb[j], fa, acc[2 * h + i][j]);
+      }
+    }
+  };
+  constexpr uint32_t W = kSmallWaves;
+  uint32_t s = s_begin + wave;
+  if (s >= s_end) return;
+  if (s + (2u * D - 1u) * W < s_end) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, s + d * W);
+    do {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        mma(std::false_type{}, d, s + d * W);
+        load(d, s + (D + d) * W);
+      }
+      s += D * W;
+    } while (s + (2u * D - 1u) * W < s_end);
+  } else {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (s + d * W < s_end) load(d, s + d * W);
+  }
+  for (; s < s_end; s += D * W) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (s + d * W < s_end) mma(std::true_type{}, d, s + d * W);
+      if (s + (D + d) * W < s_end) load(d, s + (D + d) * W);
+    }
+  }
+}
+
+// Sums the 16 waves' 16 IM x 32 tiles, 32 rows at a time, in wave order, and
+// hands `out` each element: out(row, column, sum). Rows go to LDS with their
+// 16-byte groups XORed by the row, so the writes of 16 rows are conflict-free.
+template <int IM, typename Out>
+__device__ __forceinline__ void small16_sum(const f32x4_t (&acc)[IM][2], float* red, Out&& out) {
+  const uint32_t tid = thread_here(), lane = tid & 63u, wave = tid >> 6;
+  const uint32_t row = tid >> 5, word = row * 32u + ((((tid & 31u) >> 2) ^ ((row >> 1) & 7u)) << 2) + (tid & 3u);
+#pragma unroll
+  for (int h = 0; h < IM / 2; ++h) {
+    if (h > 0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const uint32_t rr = 16u * i + (lane & 15u), cg = 4u * j + (lane >> 4);
+        *reinterpret_cast<f32x4_t*>(&red[wave * 1024u + rr * 32u + ((cg ^ ((rr >> 1) & 7u)) << 2)]) = acc[2 * h + i][j];
+      }
+    __syncthreads();
+    float sum = red[word];
+#pragma unroll
+    for (uint32_t w = 1; w < kSmallWaves; ++w) sum += red[w * 1024u + word];
+    out(32u * h + row, tid & 31u, sum);
+  }
+}
+
+// The tile a workgroup of the small kernel takes, 16-bit inputs: 32x32 while
+// K is split over workgroups (P > 1), else the largest of 128x128, 64x64 and
+// 64x32 that still gives kSmallTilesMin workgroups one tile each. A larger
+// tile reads its operands fewer times: 64 x 8192 x 8192 (B as [K][N]) takes
+// 73 us on 32x32 tiles, which read B twice, past what an L2 holds of it in
+// flight, and 54 on 64x32; 1024 x 1024 x 4096 55 on 32x32 and 22 on 64x64; 32
+// batches of 500 x 500 x 64 47 on 32x32 and 16 on 128x128. A 32x64 tile for
+// M <= 32 was within 15% either way. What bounds a few rows against a large
+// [K][N] B (16 x 16384 x 16384, 3.5 TB/s; 5.0 with [N][K]) is its 64-byte
+// pieces of rows 32 KB apart.
+constexpr uint32_t kSmallTilesMin = 192;
+struct SmallTile {
+  uint32_t m, n;
+};
+template <bool H16, bool B_NK>
+__host__ __device__ __forceinline__ SmallTile gemm_small_shape(uint32_t M, uint32_t N, uint32_t K, uint32_t batch,
+                                                               uint32_t P) {
+  if (!H16 || P > 1u || K < 8u || (!B_NK && N < 8u) || M <= 32u) return {32u, 32u};
+  const auto count = [&](uint32_t tm, uint32_t tn) {
+    return static_cast<uint64_t>((M - 1u) / tm + 1u) * ((N - 1u) / tn + 1u) * batch;
+  };
+  if (M > 64u && N > 64u && count(128u, 128u) >= kSmallTilesMin) return {128u, 128u};
+  if (N > 32u && count(64u, 64u) >= kSmallTilesMin) return {64u, 64u};
+  if (count(64u, 32u) >= kSmallTilesMin) return {64u, 32u};
+  return {32u, 32u};
+}
 
 // A wave's steps of its chunk: s = s_begin + wave + j * kSmallWaves below
 // s_end. Steps whose operands are all in range (an interior tile and a whole
@@ -1423,20 +1619,51 @@ __device__ __forceinline__ void small_steps(uint32_t s_begin, uint32_t s_end, ui
   }
 }
 
-// `tile` is the tile within its contraction (row-major over ceil(N/32)
-// columns of tiles), `gtile` the tile's index over all T tiles of the
+// `tile` is the tile within its contraction (of `shape`, column-major), `gtile` the tile's index over all T tiles of the
 // launch (batches included): the partial scratch is indexed by it.
 template <bool H16, bool B_NK, typename Epi, bool F16 = false>
 __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const void* __restrict__ Bv,
                                            float* __restrict__ C, float* __restrict__ part, uint32_t M, uint32_t N,
-                                           uint32_t K, Epi epi, uint32_t tile, uint32_t gtile, uint32_t T, uint32_t p,
-                                           uint32_t P) {
+                                           uint32_t K, Epi epi, SmallTile shape, uint32_t tile, uint32_t gtile,
+                                           uint32_t T, uint32_t p, uint32_t P) {
   constexpr uint32_t KS = H16 ? 16u : 8u;   // k per step
   constexpr uint32_t KPL = H16 ? 8u : 4u;   // k per lane and step
   __shared__ __attribute__((aligned(16))) float red[kSmallWaves * 1024u];
-  const uint32_t tiles_n = (N + 31u) / 32u;
-  const uint32_t m0 = (tile / tiles_n) * 32u, n0 = (tile % tiles_n) * 32u;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t tiles_m = (M - 1u) / shape.m + 1u;
+  const uint32_t m0 = (tile % tiles_m) * shape.m, n0 = (tile / tiles_m) * shape.n;
+  const uint32_t tid = thread_here(), lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if constexpr (H16) {
+    const uint16_t* A = static_cast<const uint16_t*>(Av);
+    const uint16_t* B = static_cast<const uint16_t*>(Bv);
+    uint16_t* lds = reinterpret_cast<uint16_t*>(red);
+    if (shape.n == 128u) {
+      gemm16_tile<128, 128, 4, 4, 1, 2, B_NK, F16, false>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
+      return;
+    }
+    if (shape.n == 64u) {
+      gemm16_tile<64, 64, 2, 4, 2, 2, B_NK, F16, false>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
+      return;
+    }
+    if (K >= 8u && (B_NK || N >= 8u)) {
+      const uint32_t steps = (K - 1u) / 32u + 1u, per = (steps - 1u) / P + 1u;
+      const uint32_t s_begin = p * per < steps ? p * per : steps;
+      const uint32_t s_end = s_begin + per < steps ? s_begin + per : steps;
+      const auto store = [&](uint32_t row, uint32_t col, float sum) {
+        if (P > 1u) part[(static_cast<uint64_t>(p) * T + gtile) * 1024u + row * 32u + col] = sum;
+        else if (m0 + row < M && n0 + col < N) C[static_cast<uint64_t>(m0 + row) * N + n0 + col] = epi(sum, m0 + row, n0 + col);
+      };
+      if (shape.m == 64u) {
+        f32x4_t acc[4][2];
+        small16_steps<4, 2, B_NK, F16>(A, B, M, N, K, m0, n0, s_begin, s_end, lds + wave * 2048u, acc);
+        small16_sum(acc, red, store);
+      } else {
+        f32x4_t acc[2][2];
+        small16_steps<2, 4, B_NK, F16>(A, B, M, N, K, m0, n0, s_begin, s_end, lds + wave * 2048u, acc);
+        small16_sum(acc, red, store);
+      }
+      return;
+    }
+  }
   const uint32_t r = lane & 31u, h = lane >> 5;
   const uint32_t am = m0 + r, bn = n0 + r;
   // Chunk p: whole steps [s_begin, s_end) (the last step of K may be short).
@@ -1485,23 +1712,11 @@ __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const vo
       acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
     };
     small_steps<KS, float4>(s_begin, s_end, wave, interior, K, load, mma);
-  } else {
+  } else {  // rows shorter than a chunk (K < 8, or N < 8 with a [K][N] operand): element by element
     const uint16_t* __restrict__ A = static_cast<const uint16_t*>(Av);
     const uint16_t* __restrict__ B = static_cast<const uint16_t*>(Bv);
-    auto load = [&](auto fast, uint32_t s, u32x4* a, u32x4* b) {
+    auto load = [&](auto, uint32_t s, u32x4* a, u32x4* b) {
       const uint32_t k0 = s * KS + KPL * h;
-      if constexpr (decltype(fast)::value) {
-        *a = *reinterpret_cast<const u32x4*>(A + static_cast<uint64_t>(am) * K + k0);
-        if constexpr (B_NK) {
-          *b = *reinterpret_cast<const u32x4*>(B + static_cast<uint64_t>(bn) * K + k0);
-        } else {
-          const uint16_t* q = B + static_cast<uint64_t>(k0) * N + bn;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            (*b)[e] = static_cast<uint32_t>(q[(2u * e) * N]) | (static_cast<uint32_t>(q[(2u * e + 1u) * N]) << 16);
-        }
-        return;
-      } else {
       uint32_t va[8], vb[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -1515,12 +1730,11 @@ __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const vo
         (*a)[e] = va[2 * e] | (va[2 * e + 1] << 16);
         (*b)[e] = vb[2 * e] | (vb[2 * e + 1] << 16);
       }
-      }
     };
     auto mma = [&](const u32x4& a, const u32x4& b) {
       acc = mfma_32x32x16_16b<F16>(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc);
     };
-    small_steps<KS, u32x4>(s_begin, s_end, wave, interior, K, load, mma);
+    small_steps<KS, u32x4>(s_begin, s_end, wave, false, K, load, mma);
   }
 #pragma unroll
   for (int i = 0; i < 16; ++i) red[wave * 1024u + static_cast<uint32_t>(i) * 64u + lane] = acc[i];
@@ -1528,22 +1742,22 @@ __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const vo
   float sum = red[tid];
 #pragma unroll
   for (uint32_t w = 1; w < kSmallWaves; ++w) sum += red[w * 1024u + tid];
+  const uint32_t sr = small_row<false>(tid), sc = small_col(tid);
   if (P > 1u) {
-    part[(static_cast<uint64_t>(p) * T + gtile) * 1024u + tid] = sum;
+    part[(static_cast<uint64_t>(p) * T + gtile) * 1024u + (H16 ? sr * 32u + sc : tid)] = sum;
     return;
   }
-  const uint32_t m = m0 + small_row(tid), n = n0 + small_col(tid);
-  if (m < M && n < N) C[static_cast<uint64_t>(m) * N + n] = epi(sum, m, n);
+  if (m0 + sr < M && n0 + sc < N) C[static_cast<uint64_t>(m0 + sr) * N + n0 + sc] = epi(sum, m0 + sr, n0 + sc);
 }
 
 // The P > 1 merge: one 1024-thread workgroup per tile, thread t adds word t
 // of the tile's P partials in chunk order, applies the epilogue and stores.
-template <typename Epi>
+template <bool H16, typename Epi>
 __device__ __forceinline__ void gemm_small_merge(float* __restrict__ C, const float* __restrict__ part, uint32_t M,
                                                  uint32_t N, Epi epi, uint32_t tile, uint32_t gtile, uint32_t T,
                                                  uint32_t P) {
-  const uint32_t tid = threadIdx.x, tiles_n = (N + 31u) / 32u;
-  const uint32_t m = (tile / tiles_n) * 32u + small_row(tid), n = (tile % tiles_n) * 32u + small_col(tid);
+  const uint32_t tid = threadIdx.x, tiles_m = (M + 31u) / 32u;
+  const uint32_t m = (tile % tiles_m) * 32u + small_row<H16>(tid), n = (tile / tiles_m) * 32u + small_col(tid);
   const float* q = part + static_cast<uint64_t>(gtile) * 1024u + tid;
   const uint64_t stride = static_cast<uint64_t>(T) * 1024u;
   float sum = q[0];

@@ -246,6 +246,10 @@ bool Parse(const std::string& text, Plan* out, std::string* err) {
         if (t.packed) return bad("a split term cannot divide by 'pack'");
         k.split_terms.push_back(t);
       }
+    } else if (kw == "stride") {
+      if (p.kernels.empty()) return bad("stride before any kernel");
+      if (tok.size() != 2 || !ParseU64(tok[1], &p.kernels.back().stride) || p.kernels.back().stride == 0)
+        return bad("stride <workgroups>");
     } else if (kw == "when" || kw == "unless") {
       if (p.kernels.empty()) return bad(kw + " before any kernel");
       Guard g;
@@ -363,6 +367,7 @@ std::string Serialize(const Plan& p) {
       for (const auto& t : k.split_terms) o << " " << TermText(p, t);
       o << "\n";
     }
+    if (k.stride != 0) o << "stride " << k.stride << "\n";
     for (const auto& g : k.when) o << "when " << GuardText(p, g) << "\n";
     for (const auto& g : k.unless) o << "unless " << GuardText(p, g) << "\n";
   }
@@ -523,6 +528,7 @@ bool GridSize(const Kernel& k, const Plan& p, const std::vector<uint32_t>& dims,
       return false;
     }
   }
+  if (k.stride != 0 && g > k.stride) g = k.stride;
   *grid = g;
   return true;
 }

@@ -25,6 +25,8 @@
 //       partials) launches only when P > 1; mode 2: the kernel launches only
 //       when P == 1 (a whole-column kernel); mode 3: as mode 0, but only when
 //       P > 1 (the partials of a nest whose P == 1 case is a mode-2 kernel).
+//   stride <n>    (for the last kernel) the kernel walks its work with the
+//       grid as its stride: at most n workgroups are launched
 //   when <dim> <lo> <hi> <mod> <rem>    (for the last kernel) the kernel runs only
 //       when lo <= dim <= hi and dim % mod == rem; every guard of a kernel must
 //       hold. <dim> may be a product of dims, d1*d2*... (its value taken in
@@ -113,6 +115,7 @@ struct Kernel {
   // only when P == 1, kSplitPartialMany = grid x P, launched only when P > 1.
   int split_mode = 0;
   std::vector<Term> split_terms;
+  uint64_t stride = 0;  // > 0: the most workgroups launched (a grid-stride kernel)
 };
 
 enum SplitMode { kSplitPartial = 0, kSplitMerge = 1, kSplitSingle = 2, kSplitPartialMany = 3 };

@@ -157,3 +157,53 @@ def test_nonfinite_operands_stay_in_their_rows(gpu, name):
     tb = torch.from_numpy(np.ascontiguousarray(b.T) if nt else b).to(gpu).to(torch.bfloat16)
     run(compiled(name), [ta, tb, c])
     assert np.array_equal(host(c), want.astype(np.float32), equal_nan=True)
+
+
+# Planes of at most 2^20 outputs: the small kernel's tile shapes (32x32 with K
+# whole and split over workgroups, 64x32, 64x64, 128x128), ragged in M, N and
+# K, rows of every alignment, more tiles than workgroups (the grid's stride).
+SMALL = [("gemm_bf16", 1, 16, 4096, 4100), ("gemm_bf16", 1, 33, 777, 1001), ("gemm_bf16_nt", 1, 33, 777, 1001),
+         ("gemm_f16", 1, 17, 3000, 65), ("gemm_bf16_nt", 1, 5, 9, 3001), ("gemm_bf16", 1, 60, 8001, 129),
+         ("gemm_bf16_nt", 1, 60, 8001, 131), ("gemm_bf16", 1, 61, 9000, 8), ("gemm_bf16", 1, 700, 1301, 200),
+         ("gemm_bf16_nt", 1, 1000, 1001, 333), ("gemm_f16_nt", 1, 1000, 1001, 1), ("gemm_bf16", 1, 3, 200001, 66),
+         ("gemm_bf16", 1, 150001, 5, 66), ("gemm_bf16", 1, 150001, 9, 66), ("bmm_bf16_nt", 32, 500, 500, 64),
+         ("bmm_bf16", 20, 500, 501, 77), ("bmm_bf16", 300, 129, 130, 8), ("bmm_bf16_nt", 70, 200, 200, 9),
+         ("bmm_bf16", 3, 40, 72, 3000), ("bmm_bf16_nt", 500, 65, 33, 40), ("bmm_bf16", 2000, 31, 33, 17)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,B,M,N,K", SMALL)
+def test_small_tile_shapes_exact(gpu, name, B, M, N, K):
+    _say("small tiles", name, B, M, N, K)
+    nt, f16, batched = name.endswith("_nt"), "_f16" in name, name.startswith("bmm")
+    rng = np.random.default_rng(B + M + N + K)
+    a = rng.integers(-4, 5, (B, M, K)).astype(np.float32)
+    b = rng.integers(-4, 5, (B, K, N)).astype(np.float32)
+    bd = b.transpose(0, 2, 1) if nt else b
+    c = out_dev((B, M, N) if batched else (M, N), gpu)
+    run(compiled(name), [_dev16(a if batched else a[0], gpu, f16), _dev16(bd if batched else bd[0], gpu, f16), c])
+    assert np.array_equal(host(c).reshape(B, M, N), np.matmul(a, b))
+
+
+def test_stride_record():
+    """`stride n` limits a kernel's workgroups to n after its split record;
+    it survives the printed form, and zero or a missing number is refused."""
+    import ctypes
+    from tcacomp_amd import _lib, compiler
+    text = ("tca-plan 1\nprogram s\ndim M 0\ntensor x f32 in 1 M\nkernel k 64 0 1 M/4\narg ptr x\n"
+            "split M 10 100000 0 1 M/64\nstride 70\nend\n")
+    for t in (text, None):
+        if t is None:
+            t = _lib.lib().tca_program_plan_text(h).decode()
+            assert "stride 70\n" in t
+        h = ctypes.c_void_p()
+        assert _lib.lib().tca_program_parse(t.encode(), ctypes.byref(h)) == 0, _lib.last_error()
+        for m, grid in ((8, 2), (20, 10), (100, 70), (10 ** 6, 70)):
+            arr = compiler._descriptors([TensorDesc(0x1000, (m,), 0)])
+            out, grids = (ctypes.c_uint8 * 1)(), (ctypes.c_uint64 * 1)()
+            assert _lib.lib().tca_program_selected(h, arr, 1, None, 0, out, grids, None, 1) == 0
+            assert grids[0] == grid, (m, grids[0])
+    for bad in ("stride 0", "stride", "stride x"):
+        h = ctypes.c_void_p()
+        assert _lib.lib().tca_program_parse(text.replace("stride 70", bad).encode(), ctypes.byref(h)) != 0
+        assert "stride <workgroups>" in _lib.last_error()
