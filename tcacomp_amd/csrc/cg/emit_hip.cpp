@@ -430,20 +430,28 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
   if (!bf16) {
     // From M, N >= 4096 on (at least 256 tiles of 256x256): whole tiles with
     // K % 32 == 0 and K >= 128 on 4 waves of 128x128 fed by a direct-to-LDS
-    // ring (_w); otherwise 256x256 tiles with 16 waves of 64x64 (_v). Below,
-    // 128x128 tiles with 4 waves (more tiles over the 256 CUs). _v and the
-    // 128x128 kernel are two instances of one loop with edge guards; both run
-    // 4 waves per SIMD: at most 128 registers per lane.
+    // ring (_w); every other shape on 64x64 tiles, halved where they are few
+    // (never from M, N >= 4096 on: _v).
     const std::string M = g.dims[m.m].name, N = g.dims[m.n].name, K = g.dims[m.k].name;
-    const auto a256 = args(256), a128 = args(128);
+    const uint32_t kHalfTiles = 1535u;
+    const auto a256 = args(256);
+    auto any = [&](bool halves) {
+      std::ostringstream b;
+      b << epi.str() << "  const uint32_t tiles = ((M + 63u) / 64u) * ((N + 63u) / 64u);\n";
+      if (halves)
+        b << "  const uint32_t T = " << nb << " * tiles, P = tca::hip::gemm_split_chunks(K, T, 1u, " << kHalfTiles << "u);\n"
+          << "  const uint32_t gt = blockIdx.x % T, part = blockIdx.x / T;\n";
+      else
+        b << "  const uint32_t gt = blockIdx.x;\n";
+      if (batched) b << "  const uint32_t bb = gt / tiles;\n";
+      b << "  tca::hip::gemm_f32_any<" << nk << ">"
+        << operands(std::string(batched ? "gt - bb * tiles" : "gt") + (halves ? ", part, P" : ", 0u, 1u")) << ");\n}\n\n";
+      return b.str();
+    };
     o << "extern \"C\" __global__ void __launch_bounds__(256) " << symbol << "_w(\n    " << signature << ") {\n"
       << epi.str() << a256.first << "  tca::hip::gemm_f32_4w<" << nk << ">" << a256.second;
-    o << "extern \"C\" __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) " << symbol
-      << "_v(\n    " << signature << ") {\n"
-      << epi.str() << a256.first << "  tca::hip::gemm_f32_tile<" << nk << ", 256, 256>" << a256.second;
-    o << "extern \"C\" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) " << symbol
-      << "(\n    " << signature << ") {\n"
-      << epi.str() << a128.first << "  tca::hip::gemm_f32_tile<" << nk << ", 128, 128>" << a128.second;
+    o << "extern \"C\" __global__ void __launch_bounds__(256) " << symbol << "_v(\n    " << signature << ") {\n" << any(false);
+    o << "extern \"C\" __global__ void __launch_bounds__(256) " << symbol << "(\n    " << signature << ") {\n" << any(true);
     GemmKernel w;
     w.suffix = "_w";
     w.block = 256;
@@ -452,16 +460,18 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
     w.detail = "f32 mfma 32x32 tile=256x256 bk=16 4 waves of 128x128, direct-to-LDS ring (whole tiles, M, N >= 4096, K % 32 == 0, K >= 128)" + orient;
     GemmKernel v;
     v.suffix = "_v";
-    v.block = 1024;
-    v.grid = tiles(256);
+    v.grid = tiles(64);
     v.when = {M + " 4096 4294967295 1 0", N + " 4096 4294967295 1 0"};
     v.unless = w.when;
-    v.detail = "f32 mfma 32x32 tile=256x256 bk=16 16 waves, two LDS buffers (M, N >= 4096)" + orient;
+    v.detail = "f32 mfma 32x32 tile=64x64 bk=32 4 waves, register-staged, any shape (M, N >= 4096)" + orient;
     GemmKernel k;
-    k.grid = tiles(128);
+    k.grid = tiles(64);
     k.unless = v.when;
     if (!bigWhen.empty()) k.when.push_back(bigWhen);
-    k.detail = "f32 mfma 32x32 tile=128x128 bk=16 4 waves, two LDS buffers" + orient;
+    std::string halfTerms;
+    for (const auto& t : k.grid) halfTerms += " " + t;
+    k.split = K + " 1 " + std::to_string(kHalfTiles) + " 0 " + std::to_string(k.grid.size()) + halfTerms;
+    k.detail = "f32 mfma 32x32 tile=64x64 (64x32 for few tiles) bk=32 4 waves, register-staged, any shape" + orient;
     out->kernels.push_back(w);
     out->kernels.push_back(v);
     out->kernels.push_back(k);

@@ -10,21 +10,15 @@
 //                 fp32 accumulate (f16 inputs: the same kernels with the
 //                 _f16 MFMAs)
 //   fp32 inputs : v_mfma_f32_32x32x2f32 (gemm_f32_4w on whole tiles from
-//                 M, N >= 4096 on, else gemm_f32_tile), fp32 accumulate
-// Geometry of the register-staged kernels: a 256-thread workgroup (4 waves,
-// 2x2) owns a BMxBN tile of C, each wave a (BM/2)x(BN/2) sub-tile of 32x32
-// MFMA blocks. K advances in
-// BK slices staged through LDS; the next slice's global loads are issued
-// before the current slice's MFMAs so HBM latency hides under the math.
-// LDS tiles hold every MFMA operand K-contiguous for its row/column (A as
-// [m][k], B as [n][k]); a [K][N] B is transposed in registers on its way
-// into LDS. Rows are padded so a wave's operand reads spread over the banks.
+//                 M, N >= 4096 on, else gemm_f32_any), fp32 accumulate
+//   output planes of at most 2^20 elements: gemm_small
+// The any-shape kernels stage slices of K through registers into LDS with
+// unguarded, possibly unaligned 16-byte loads (gemm16_tile, gemm32_tile).
 //
-// MFMA 32x32 operand/result lane layout (CDNA3/CDNA4 ISA):
-//   A operand: lane l supplies row (l % 32), k = (l / 32) * KPL + [0, KPL)
+// v_mfma_f32_32x32x2f32 operand/result lane layout (CDNA3/CDNA4 ISA):
+//   A operand: lane l supplies row (l % 32), k = l / 32
 //   B operand: lane l supplies col (l % 32), same k
 //   result   : lane l, element i -> row 8*(i/4) + 4*(l/32) + (i%4), col l%32
-// with KPL = 8 for 32x32x16 bf16 and KPL = 1 for 32x32x2 f32.
 #ifndef TCA_HIP_GEMM_H_
 #define TCA_HIP_GEMM_H_
 
@@ -46,13 +40,6 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 // through memory, LDS and registers; F16 selects the MFMA that reads them as
 // IEEE half (v_mfma_f32_*_f16) instead of bfloat16. The fp32 accumulation,
 // the operand layout and every data movement are the same for both.
-template <bool F16, typename Acc>
-__device__ __forceinline__ Acc mfma_32x32x16_16b(const bf16x8& a, const bf16x8& b, const Acc& c) {
-  if constexpr (F16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
 template <bool F16, typename Acc>
 __device__ __forceinline__ Acc mfma_16x16x32_16b(const bf16x8& a, const bf16x8& b, const Acc& c) {
   if constexpr (F16)
@@ -215,9 +202,11 @@ __device__ __forceinline__ bf16x8 frag_b16_tr(const uint16_t* Bs, uint32_t n_col
 // apart 44, operands loaded straight into a 4-deep LDS ring 45 (8 waves) and
 // 55 (4 waves). `TINY` (K-contiguous rows or
 // [K][N] rows shorter than one chunk) loads those element by element.
+// FLUSH: the accumulators are added to a second set every 4 turns (256 k), so
+// the error grows with the root of K as it does for sums split over 16 waves.
 // `lds` holds KG * 2 * 64 * (BM + BN) values; `thread` is threadIdx.x.
 template <uint32_t BM, uint32_t BN, uint32_t WGM, uint32_t WGN, uint32_t KG, int D, bool B_NK, bool F16, bool TINY,
-          typename Epi>
+          bool FLUSH = false, typename Epi>
 __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                                             float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
                                             uint32_t m0, uint32_t n0, uint16_t* lds, uint32_t thread) {
@@ -329,6 +318,26 @@ __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, cons
   for (int i = 0; i < IM; ++i)
 #pragma unroll
     for (int j = 0; j < JN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 sum[FLUSH ? IM : 1][FLUSH ? JN : 1];
+  if constexpr (FLUSH) {
+#pragma unroll
+    for (int i = 0; i < IM; ++i)
+#pragma unroll
+      for (int j = 0; j < JN; ++j) sum[i][j] = acc[i][j];
+  }
+  auto flush = [&]() {
+    if constexpr (FLUSH) {
+#pragma unroll
+      for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            sum[i][j][e] += acc[i][j][e];
+            acc[i][j][e] = 0.0f;
+          }
+    }
+  };
   auto compute = [&](uint32_t buf) {
     const uint16_t* As = glds + buf * BUF;
     const uint16_t* Bs = As + ASL;
@@ -377,6 +386,7 @@ __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, cons
       write(Body{}, (i + 1) % D, (i + 1) & 1, k_of(t0 + i + 1u));
       load((i + 1) % D, k_of(t0 + i + 1u + D));
       compute(i & 1);
+      if (FLUSH && (t0 + i) % 4u == 3u) flush();
       __syncthreads();
     }
   }
@@ -388,9 +398,17 @@ __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, cons
         if (t + 1u < nt) write(Last{}, (i + 1) % D, (i + 1) & 1, k_of(t + 1u));
         if (t + 1u + D < nt) load((i + 1) % D, k_of(t + 1u + D));
         compute(i & 1);
+        if (FLUSH && t % 4u == 3u) flush();
         __syncthreads();
       }
     }
+  }
+  if constexpr (FLUSH) {
+    flush();
+#pragma unroll
+    for (int i = 0; i < IM; ++i)
+#pragma unroll
+      for (int j = 0; j < JN; ++j) acc[i][j] = sum[i][j];
   }
   // Block (i, j) is finished by group (i * JN + j) / (IM * JN / KG): the
   // others hand it their sums through LDS (16 bytes per lane and block).
@@ -938,200 +956,290 @@ __device__ __forceinline__ void gemm_bf16_4w(const __bf16* __restrict__ A, const
     }
 }
 
-// ---------------------------------------------------------------- fp32 path
-// Tile: BM x BN with BM, BN in {128, 256}, BK-deep slices; (BM/64)x(BN/64)
-// waves, each 64x64 = 2x2 blocks of v_mfma_f32_32x32x2f32, 4 waves per SIMD
-// (256x256: one 72 KiB block of 16 waves per CU; 128x128: four 38 KiB
-// blocks of 4 waves), at most 128 registers per lane. fp32 MFMA is not
-// power-limited on this part (an MFMA-only loop on random operands holds
-// 2.4 GHz), so the loop is built for issue:
-//   two LDS buffers, one barrier per slice: slice kt+1 is loaded into
-//   registers when slice kt starts and written into the other buffer half
-//   way through slice kt's MFMAs (every wave passed the barrier after that
-//   buffer's last reads);
-//   each 2-deep k step's fragments are read one step ahead;
-//   strides chosen so a fragment read (32 rows or columns at k, the other
-//   32 lanes at k+1) covers 64 distinct banks: LDA = BK + 2 (LDA/2 odd),
-//   [K][N] B rows of BN + 32 floats (the k+1 row lands 32 banks over).
-// Measured at 4096^3 (interleaved, one box, bitwise-equal results), TFLOP/s:
-// this loop on 128x128 tiles with 4 waves 133, 256x128 with 8 waves 135,
-// 256x256 with 16 waves 137 (the larger tiles read the L2 less per flop,
-// but leave CUs idle below 256 tiles: the emitter takes 256x256 tiles from
-// M, N >= 4096 on and 128x128 tiles below); the earlier single-buffer
-// 128x128 loop with stride BK + 1, 117; 16x16x4f32 blocks on the 128x128
-// loop, 127.
-template <bool B_NK, int BM, int BN, int BK = 16, typename Epi>
-__device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const float* __restrict__ B,
-                                              float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
-                                              uint32_t tile = ~0u) {
-  static_assert((BM == 128 || BM == 256) && BM == BN, "square 128 or 256 tiles");
-  static_assert(BK == 16 || BK == 32, "slices of 16 or 32");
-  constexpr int WN = BN / 64, THREADS = 64 * (BM / 64) * WN;
-  constexpr int LPT = BM * BK / 4 / THREADS;    // float4 per thread per operand slice
-  constexpr uint32_t VPN = BN / 4;              // float4 per [K][N] panel row
-  constexpr int LDA = BK + 2;                   // As[m][k]
-  constexpr int LDB = B_NK ? BK + 2 : BN + 32;  // Bs[n][k] (NK) or Bs[k][n] (KN)
-  constexpr int SA = BM * LDA, SB = B_NK ? BN * LDB : BK * LDB;
-  __shared__ __attribute__((aligned(16))) float lds[2 * (SA + SB)];
-  const uint32_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  uint32_t tm, tn;
-  gemm_tile_coords(tiles_m, tiles_n, &tm, &tn, tile == ~0u ? blockIdx.x : tile);
-  const uint32_t m0 = tm * BM, n0 = tn * BN;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t wm = (wave / WN) * 64u, wn = (wave % WN) * 64u;
-  const bool vec_a = (K % 4u) == 0u;
-  const bool vec_b = B_NK ? (K % 4u) == 0u : (N % 4u) == 0u;
+// ------------------------------------------------------- fp32 path, any shape
+__device__ __forceinline__ f32x4_t load16_any(const float* p) { return *reinterpret_cast<const f32x4_a4*>(p); }
 
-  f32x16 acc[2][2];
+// The four values of v moved down by n places, zeros shifted in (shift_down16
+// for 32-bit elements).
+__device__ __forceinline__ f32x4_t shift_down32(f32x4_t v, uint32_t n) {
+  const bool a = n & 1u, b = n & 2u;
+  v = f32x4_t{a ? v[1] : v[0], a ? v[2] : v[1], a ? v[3] : v[2], a ? 0.0f : v[3]};
+  v = f32x4_t{b ? v[2] : v[0], b ? v[3] : v[1], b ? 0.0f : v[2], b ? 0.0f : v[3]};
+  return n >= 4u ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : v;
+}
+
+// LDS word of element (row, 16-byte chunk c) of a [rows][32] fp32 slice: a
+// fragment read (32 rows, one chunk per half-wave) covers every bank slot
+// once per 16-lane cycle (the cycles measured at gemm_bf16_256_w8).
+__device__ __forceinline__ uint32_t swz32_rows(uint32_t row, uint32_t c) { return row * 32u + ((c ^ ((row >> 1) & 7u)) << 2); }
+// ... of element (k, n) of a [32][BN] slice: the rows k and k + 4 that the
+// halves of a wave read lie 32 banks apart.
+template <uint32_t BN>
+__device__ __forceinline__ uint32_t swz32_kn(uint32_t k, uint32_t n) {
+  if constexpr (BN >= 64u) return k * BN + (n ^ ((k & 4u) << 3));
+  else return (k ^ ((k >> 2) & 1u)) * BN + n;
+}
+
+// One BM x BN tile of C at (m0, n0), fp32, every shape: gemm16_tile's scheme on
+// v_mfma_f32_32x32x2f32. KG groups of WGM x WGN waves take every KG-th 32-deep
+// slice of K, loaded unguarded into registers while the slice before is
+// computed, in NBUF LDS buffers per group (2: one barrier per slice); their
+// sums meet in LDS. Four 2-deep MFMA steps take k = 8h + e on lanes 0-31 and
+// k = 8h + 4 + e on lanes 32-63, one 16-byte read of a K-contiguous row each.
+// fp32 MFMAs take 64 cycles per 32x32 block and 2 k, so small tiles do not
+// starve them (a 64x64 tile needs a quarter of the L1 and LDS rates), and
+// several workgroups per CU hide each other's waits.
+// FLUSH: the accumulators are added to a second set every 8 k, for an error no
+// larger than that of sums split over 16 waves.
+// `lds` holds KG * NBUF * 32 * (BM + BN) floats; `thread` is threadIdx.x.
+template <uint32_t BM, uint32_t BN, uint32_t WGM, uint32_t WGN, uint32_t KG, uint32_t NBUF, bool B_NK, bool TINY,
+          bool FLUSH = false, typename Epi>
+__device__ __forceinline__ void gemm32_tile(const float* __restrict__ A, const float* __restrict__ B,
+                                            float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
+                                            uint32_t m0, uint32_t n0, float* lds, uint32_t thread) {
+  constexpr uint32_t THREADS = 64u * WGM * WGN, TM = BM / WGM, TN = BN / WGN;
+  constexpr int IM = TM / 32, JN = TN / 32, CA = BM * 8 / THREADS, CB = BN * 8 / THREADS;
+  static_assert(CA >= 1 && CB >= 1 && (NBUF == 1 || NBUF == 2), "whole chunks per thread");
+  constexpr uint32_t ASL = BM * 32u, BUF = ASL + BN * 32u;
+  const uint32_t lane = thread & 63u, wave_id = __builtin_amdgcn_readfirstlane(thread >> 6);
+  const uint32_t grp = wave_id / (WGM * WGN), wave = wave_id % (WGM * WGN), tid = wave * 64u + lane;
+  const uint32_t wm = (wave / WGN) * TM, wn = (wave % WGN) * TN;
+  float* glds = lds + grp * (NBUF * BUF);
+  const uint32_t kch = (tid & 7u) * 4u, row0 = tid >> 3;
+  const uint32_t bk0 = tid / (BN / 4u), bn = n0 + (tid % (BN / 4u)) * 4u;
+  const float* pa[CA];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < CA; ++i) {
+    const uint32_t r = m0 + row0 + i * (THREADS / 8u);
+    pa[i] = A + static_cast<uint64_t>(r < M ? r : M - 1u) * K;
+  }
+  const float* pb[B_NK ? CB : 1];
+  uint32_t bsh = 0u;
+  if constexpr (B_NK) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < CB; ++i) {
+      const uint32_t r = n0 + row0 + i * (THREADS / 8u);
+      pb[i] = B + static_cast<uint64_t>(r < N ? r : N - 1u) * K;
+    }
+  } else {
+    const uint32_t last = N >= 4u ? N - 4u : 0u, at = bn < last ? bn : last;
+    bsh = bn - at;
+    pb[0] = B + at;
+  }
+  auto load_k = [&](const float* row, uint32_t k0) -> f32x4_t {
+    const uint32_t k = k0 + kch;
+    if constexpr (TINY) {
+      if (K < 4u) {
+        f32x4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t e = 0; e < 4u; ++e)
+          if (k + e < K) v[e] = row[k + e];
+        return v;
+      }
+    }
+    return load16_any(row + (k < K - 4u ? k : K - 4u));
+  };
+  auto load_n = [&](uint32_t k) -> f32x4_t {
+    const float* row = pb[0] + static_cast<uint64_t>(k < K ? k : K - 1u) * N;
+    if constexpr (TINY) {
+      if (N < 4u) {
+        f32x4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t e = 0; e < 4u; ++e)
+          if (bn + e < N) v[e] = row[bn + e];
+        return v;
+      }
+    }
+    return load16_any(row);
+  };
+  f32x4_t ra[CA], rb[CB];
+  auto load = [&](uint32_t k0) {
+#pragma unroll
+    for (int i = 0; i < CA; ++i) ra[i] = load_k(pa[i], k0);
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+      if constexpr (B_NK) rb[i] = load_k(pb[i], k0);
+      else rb[i] = load_n(k0 + bk0 + i * (THREADS / (BN / 4u)));
+    }
+  };
+  const bool edge_n = !B_NK && n0 + BN > N && !(TINY && N < 4u);
+  auto write = [&](uint32_t buf, uint32_t k0) {
+    float* As = glds + buf * BUF;
+    float* Bs = As + ASL;
+    if (k0 + 32u > K && !(TINY && K < 4u)) {  // the last, short slice
+      const uint32_t k = k0 + kch, n = k - (k < K - 4u ? k : K - 4u);
+#pragma unroll
+      for (int i = 0; i < CA; ++i) ra[i] = shift_down32(ra[i], n);
+      if constexpr (B_NK) {
+#pragma unroll
+        for (int i = 0; i < CB; ++i) rb[i] = shift_down32(rb[i], n);
+      }
+    }
+    if constexpr (!B_NK) {
+      if (edge_n) {
+#pragma unroll
+        for (int i = 0; i < CB; ++i) rb[i] = shift_down32(rb[i], bsh);
+      }
+      if (k0 + 32u > K) {
+#pragma unroll
+        for (int i = 0; i < CB; ++i)
+          if (k0 + bk0 + i * (THREADS / (BN / 4u)) >= K) rb[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < CA; ++i)
+      *reinterpret_cast<f32x4_t*>(&As[swz32_rows(row0 + i * (THREADS / 8u), tid & 7u)]) = ra[i];
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+      if constexpr (B_NK)
+        *reinterpret_cast<f32x4_t*>(&Bs[swz32_rows(row0 + i * (THREADS / 8u), tid & 7u)]) = rb[i];
+      else
+        *reinterpret_cast<f32x4_t*>(&Bs[swz32_kn<BN>(bk0 + i * (THREADS / (BN / 4u)), (tid % (BN / 4u)) * 4u)]) = rb[i];
+    }
+  };
+  f32x16 acc[IM][JN];
+#pragma unroll
+  for (int i = 0; i < IM; ++i)
+#pragma unroll
+    for (int j = 0; j < JN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-  float4 ra[LPT], rb[LPT];
-  // Row-major [rows][K] panel, BK columns: BM BK / 4 float4 -> LPT per thread.
-  constexpr uint32_t VPR = BK / 4;  // float4 per panel row
-  auto load_rows = [&](const float* __restrict__ P, uint32_t rows, uint32_t r0, uint32_t k0, bool vec, float4* r) {
+  f32x16 sum[FLUSH ? IM : 1][FLUSH ? JN : 1];
+  if constexpr (FLUSH) {
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const uint32_t v = i * THREADS + tid, rr = v / VPR, kv = (v % VPR) * 4u;
-      const uint32_t gr = r0 + rr, gk = k0 + kv;
-      if (vec && gr < rows && gk + 4u <= K) {
-        r[i] = *reinterpret_cast<const float4*>(P + static_cast<uint64_t>(gr) * K + gk);
-      } else {
-        float h[4];
+    for (int i = 0; i < IM; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = (gr < rows && gk + e < K) ? P[static_cast<uint64_t>(gr) * K + gk + e] : 0.0f;
-        r[i] = make_float4(h[0], h[1], h[2], h[3]);
-      }
+      for (int j = 0; j < JN; ++j) sum[i][j] = acc[i][j];
+  }
+  auto flush = [&]() {
+    if constexpr (FLUSH) {
+#pragma unroll
+      for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            sum[i][j][e] += acc[i][j][e];
+            acc[i][j][e] = 0.0f;
+          }
     }
   };
-  auto load_b_kn = [&](uint32_t k0) {
+  const uint32_t l32 = lane & 31u, hf = lane >> 5;
+  auto compute = [&](uint32_t buf) {
+    const float* As = glds + buf * BUF;
+    const float* Bs = As + ASL;
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const uint32_t v = i * THREADS + tid, kr = v / VPN, nv = (v % VPN) * 4u;
-      const uint32_t gk = k0 + kr, gn = n0 + nv;
-      if (vec_b && gk < K && gn + 4u <= N) {
-        rb[i] = *reinterpret_cast<const float4*>(B + static_cast<uint64_t>(gk) * N + gn);
-      } else {
-        float h[4];
+    for (uint32_t h = 0; h < 4u; ++h) {
+      f32x4_t fa[IM], fb[JN];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = (gk < K && gn + e < N) ? B[static_cast<uint64_t>(gk) * N + gn + e] : 0.0f;
-        rb[i] = make_float4(h[0], h[1], h[2], h[3]);
+      for (int i = 0; i < IM; ++i) fa[i] = *reinterpret_cast<const f32x4_t*>(&As[swz32_rows(wm + 32u * i + l32, 2u * h + hf)]);
+#pragma unroll
+      for (int j = 0; j < JN; ++j) {
+        const uint32_t n = wn + 32u * j + l32;
+        if constexpr (B_NK) {
+          fb[j] = *reinterpret_cast<const f32x4_t*>(&Bs[swz32_rows(n, 2u * h + hf)]);
+        } else {
+#pragma unroll
+          for (uint32_t e = 0; e < 4u; ++e) fb[j][e] = Bs[swz32_kn<BN>(8u * h + 4u * hf + e, n)];
+        }
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+          for (int j = 0; j < JN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][e], fb[j][e], acc[i][j], 0, 0, 0);
+      flush();
     }
   };
-  // Interior tiles (the whole BMxBN block in range, rows 16-byte aligned,
-  // K a multiple of BK) take unguarded float4 loads. The test is uniform
-  // over the workgroup and made once, outside the K loop (two instances of
-  // the loop): with per-lane guards alone the compiler merges the vector and
-  // scalar paths into single-float loads under divergent branches, and with
-  // the branch inside the loop the two paths join in register copies that
-  // wait for the loads just issued (125 against 137 TFLOP/s).
-  const bool interior = vec_a && vec_b && m0 + BM <= M && n0 + BN <= N && K % BK == 0u;
-  auto load_interior = [&](uint32_t k0) {
+  // Turn t of a group is slice t * KG + grp; a slice past K re-reads the rows'
+  // last chunk and is written as zeros.
+  const uint32_t ns = K / 32u + (K % 32u != 0u ? 1u : 0u), nt = ns / KG + (ns % KG != 0u ? 1u : 0u);
+  auto k_of = [&](uint32_t t) { return (t * KG + grp) * 32u; };
+  if (nt > 0u) {
+    load(k_of(0));
+    write(0u, k_of(0));
+    __syncthreads();
+  }
+  for (uint32_t t = 0; t < nt; ++t) {
+    const bool more = t + 1u < nt;
+    if (more) load(k_of(t + 1u));
+    compute(NBUF == 2u ? t & 1u : 0u);
+    if constexpr (NBUF == 1u) __syncthreads();
+    if (more) write(NBUF == 2u ? (t + 1u) & 1u : 0u, k_of(t + 1u));
+    __syncthreads();
+  }
+  if constexpr (FLUSH) {
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const uint32_t v = i * THREADS + tid, rr = v / VPR, kv = (v % VPR) * 4u;
-      ra[i] = *reinterpret_cast<const float4*>(A + static_cast<uint64_t>(m0 + rr) * K + k0 + kv);
-      if constexpr (B_NK) {
-        rb[i] = *reinterpret_cast<const float4*>(B + static_cast<uint64_t>(n0 + rr) * K + k0 + kv);
-      } else {
-        const uint32_t kr = v / VPN, nv = (v % VPN) * 4u;
-        rb[i] = *reinterpret_cast<const float4*>(B + static_cast<uint64_t>(k0 + kr) * N + n0 + nv);
-      }
-    }
-  };
-  auto load_guarded = [&](uint32_t k0) {
-    load_rows(A, M, m0, k0, vec_a, ra);
-    if constexpr (B_NK) load_rows(B, N, n0, k0, vec_b, rb);
-    else load_b_kn(k0);
-  };
-  // Rows of LDA (or LDB) floats are 8-byte aligned: a float4 of a [rows][k]
-  // panel is written as two float2.
-  auto store = [&](int buf) {
-    float* As = lds + buf * (SA + SB);
-    float* Bs = As + SA;
+    for (int i = 0; i < IM; ++i)
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const uint32_t v = i * THREADS + tid, rr = v / VPR, kv = (v % VPR) * 4u;
-      float2* p = reinterpret_cast<float2*>(&As[rr * LDA + kv]);
-      p[0] = make_float2(ra[i].x, ra[i].y);
-      p[1] = make_float2(ra[i].z, ra[i].w);
-    }
-    if constexpr (B_NK) {
+      for (int j = 0; j < JN; ++j) acc[i][j] = sum[i][j];
+  }
+  // Four rows of a block (accumulator elements 4q .. 4q+3) are finished by
+  // group (block * 4 + q) / (4 IM JN / KG): the others hand it their sums.
+  constexpr int QUADS = IM * JN * 4, OWN = QUADS / static_cast<int>(KG);
+  if constexpr (KG > 1u) {
+    static_assert(QUADS % KG == 0u && KG * QUADS * THREADS * 4u <= KG * NBUF * BUF, "the sums fit the slices' LDS");
+    f32x4_t* red = reinterpret_cast<f32x4_t*>(lds);
 #pragma unroll
-      for (int i = 0; i < LPT; ++i) {
-        const uint32_t v = i * THREADS + tid, rr = v / VPR, kv = (v % VPR) * 4u;
-        float2* p = reinterpret_cast<float2*>(&Bs[rr * LDB + kv]);
-        p[0] = make_float2(rb[i].x, rb[i].y);
-        p[1] = make_float2(rb[i].z, rb[i].w);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < LPT; ++i) {
-        const uint32_t v = i * THREADS + tid, kr = v / VPN, nv = (v % VPN) * 4u;
-        *reinterpret_cast<float4*>(&Bs[kr * LDB + nv]) = rb[i];
-      }
-    }
-  };
-
-  const uint32_t nk = (K + BK - 1) / BK;
-  auto run = [&](auto load) {  // the K loop, on one of the two load paths
-    if (nk > 0) {
-      load(0);
-      store(0);
+    for (int q = 0; q < QUADS; ++q) {
+      const f32x16& c = acc[q / 4 / JN][q / 4 % JN];
+      if (static_cast<uint32_t>(q / OWN) != grp)
+        red[(grp * QUADS + q) * THREADS + tid] = f32x4_t{c[4 * (q % 4)], c[4 * (q % 4) + 1], c[4 * (q % 4) + 2], c[4 * (q % 4) + 3]};
     }
     __syncthreads();
-    for (uint32_t kt = 0; kt < nk; ++kt) {
-      const int buf = kt & 1;
-      const float* As = lds + buf * (SA + SB);
-      const float* Bs = As + SA;
-      const bool more = kt + 1 < nk;
-      if (more) load((kt + 1) * BK);
-      float a0[2], b0[2], a1[2], b1[2];
-      auto rd = [&](int ks, float (&fa)[2], float (&fb)[2]) {  // 2-deep step ks: lane l holds k = 2ks + l/32
-        const uint32_t k = ks * 2u + (lane >> 5);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) fa[i] = As[(wm + i * 32u + (lane & 31u)) * LDA + k];
+    for (int q = 0; q < QUADS; ++q) {
+      if (static_cast<uint32_t>(q / OWN) == grp) {
+        f32x16& c = acc[q / 4 / JN][q / 4 % JN];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const uint32_t n = wn + j * 32u + (lane & 31u);
-          fb[j] = B_NK ? Bs[n * LDB + k] : Bs[k * LDB + n];
+        for (uint32_t g = 0; g < KG; ++g) {
+          if (g == grp) continue;
+          const f32x4_t v = red[(g * QUADS + q) * THREADS + tid];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) c[4 * (q % 4) + e] += v[e];
         }
-      };
-      auto mm = [&](const float (&fa)[2], const float (&fb)[2]) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
-      };
-      rd(0, a0, b0);
-#pragma unroll
-      for (int ks = 0; ks < BK / 2; ks += 2) {
-        rd(ks + 1, a1, b1);
-        mm(a0, b0);
-        if (ks + 2 < BK / 2) rd(ks + 2, a0, b0);
-        mm(a1, b1);
-        if (ks == BK / 4 && more) store(buf ^ 1);
       }
-      __syncthreads();
     }
-  };
-  if (interior) run(load_interior);
-  else run(load_guarded);
+  }
+  // acc[i][j][e] = C[r][c], r = m0 + wm + 32i + 8(e/4) + 4(lane/32) + e%4, c = n0 + wn + 32j + lane%32.
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int q = 0; q < QUADS; ++q) {
+    if (static_cast<uint32_t>(q / OWN) != grp) continue;
+    const int i = q / 4 / JN, j = q / 4 % JN;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const uint32_t r = m0 + wm + i * 32u + 8u * (e >> 2) + 4u * (lane >> 5) + (e & 3);
-        const uint32_t c = n0 + wn + j * 32u + (lane & 31u);
-        if (r < M && c < N) C[static_cast<uint64_t>(r) * N + c] = epi(acc[i][j][e], r, c);
-      }
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t r = m0 + wm + 32u * i + 8u * (q % 4) + 4u * hf + e, c = n0 + wn + 32u * j + l32;
+      if (r < M && c < N) C[static_cast<uint64_t>(r) * N + c] = epi(acc[i][j][4 * (q % 4) + e], r, c);
+    }
+  }
+}
+
+// Planes that gemm_f32_4w does not take: 64x64 of C per 256-thread workgroup,
+// or 64x32 where 64x64 tiles would be fewer than three per CU (`parts` >= 2
+// workgroups were launched per tile): the CUs' shares then differ less. The
+// kernel before (128x128 tiles, element-wise guards on edges) took 147 us for
+// 1000 x 1500 x 1001 (34 now), 317 for 1024 x 2048 x 4096 (158), 1052 for 4100
+// x 4096 x 2048 on 256x256 tiles (610). MFMA-bound: 110-120 of the 150 TFLOP/s
+// an MFMA loop reaches. 32 KiB of LDS keep five workgroups on a CU; with 48
+// (two buffers for the halves) three, and 2048 x 2048 x 4096 took 308 us
+// instead of 293.
+template <bool B_NK, typename Epi>
+__device__ __forceinline__ void gemm_f32_any(const float* __restrict__ A, const float* __restrict__ B,
+                                             float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
+                                             uint32_t tile, uint32_t part, uint32_t parts) {
+  __shared__ __attribute__((aligned(16))) float lds[2 * 32 * 128];
+  const uint32_t tiles_m = (M - 1u) / 64u + 1u, tiles_n = (N - 1u) / 64u + 1u;
+  uint32_t tm, tn;
+  gemm_tile_coords(tiles_m, tiles_n, &tm, &tn, tile);
+  const uint32_t m0 = tm * 64u, n0 = tn * 64u + part * 32u;
+  if (part >= 2u || n0 >= N) return;
+  if (K < 4u || (!B_NK && N < 4u)) {
+    if (part == 0u) gemm32_tile<64, 64, 2, 2, 1, 2, B_NK, true>(A, B, C, M, N, K, epi, m0, n0, lds, threadIdx.x);
+  } else if (parts >= 2u) {
+    gemm32_tile<64, 32, 2, 1, 2, 1, B_NK, false>(A, B, C, M, N, K, epi, m0, n0, lds, threadIdx.x);
+  } else {
+    gemm32_tile<64, 64, 2, 2, 1, 2, B_NK, false>(A, B, C, M, N, K, epi, m0, n0, lds, threadIdx.x);
+  }
 }
 
 // ------------------------------------- fp32 path, 4 waves, 128x128 per wave
@@ -1347,24 +1455,18 @@ __device__ __forceinline__ void gemm_f32_4w(const float* __restrict__ A, const f
 // on one or two CUs, walking K alone (testing/kernels/tiling/mm_splitk.tca:1-2
 // names the split-k schedule class for them). Here a workgroup of 16 waves
 // owns a 32x32 tile of C and a chunk of K:
-//   - the chunk's k steps (8 deep for f32, 16 deep for 16-bit inputs) are
-//     dealt round-robin to the 16 waves; each wave accumulates the whole
-//     32x32 tile in one MFMA block (4 x v_mfma_f32_32x32x2f32 per step, or
-//     one v_mfma_f32_32x32x16_{bf16,f16});
+//   - the chunk's k steps (16 deep for f32, 32 for 16-bit inputs) are dealt
+//     round-robin to the 16 waves; each wave accumulates the whole 32x32 tile;
 //   - the waves' tiles meet in LDS and are summed in wave order;
 //   - with P > 1 chunks (P = gemm_split_chunks(K, tiles, KCMIN, BLOCKS),
 //     the formula of the launch plan's split record) the workgroup of chunk
 //     p writes its sum to a partial scratch [P][tiles][1024] and a second
 //     kernel (gemm_small_merge) adds the P partials in chunk order.
 // Every order is fixed, so the result does not depend on the schedule.
-// Operands go from memory straight into the MFMA operand registers (no
-// staging of tiles: the waves of a workgroup read disjoint k, so nothing is
-// shared inside it; neighbouring tiles share panels through the L2):
-//   f32 step at k0, lane l (r = l % 32, h = l / 32): A[m0+r][k0+4h+e] and
-//   B[k0+4h+e][n0+r] for e = 0..3, one float4 where the operand is
-//   K-contiguous; MFMA e sums k0+e (lanes 0-31) and k0+4+e (lanes 32-63), so
-//   a step sums each of its 8 k once;
-//   16-bit step: small16_steps.
+// The waves of a workgroup read disjoint k, so nothing is shared inside it
+// (small16_steps, small32_steps); neighbouring tiles share panels through the
+// L2. Without a K split larger tiles are taken where they fill the CUs
+// (gemm_small_shape).
 // f32 result element i of lane l is C[m0 + 8(i/4) + 4(l/32) + i%4][n0 + l%32];
 // a wave's tile goes to LDS element-major (word i*64 + l: conflict-free) and
 // thread t = i*64 + l of the workgroup sums word t over the waves.
@@ -1550,14 +1652,15 @@ __device__ __forceinline__ void small16_sum(const f32x4_t (&acc)[IM][2], float* 
   }
 }
 
-// The tile a workgroup of the small kernel takes, 16-bit inputs: 32x32 while
-// K is split over workgroups (P > 1), else the largest of 128x128, 64x64 and
+// The tile a workgroup of the small kernel takes: 32x32 while K is split over
+// workgroups (P > 1), else the largest of 128x128 (16-bit inputs), 64x64 and
 // 64x32 that still gives kSmallTilesMin workgroups one tile each. A larger
 // tile reads its operands fewer times: 64 x 8192 x 8192 (B as [K][N]) takes
 // 73 us on 32x32 tiles, which read B twice, past what an L2 holds of it in
 // flight, and 54 on 64x32; 1024 x 1024 x 4096 55 on 32x32 and 22 on 64x64; 32
 // batches of 500 x 500 x 64 47 on 32x32 and 16 on 128x128. A 32x64 tile for
-// M <= 32 was within 15% either way. What bounds a few rows against a large
+// M <= 32 was within 15% either way; fp32: 1024 x 1024 x 4096 127 us before, 85
+// on 64x64, 64 x 8192 x 4096 81 before, 60 on 32x32, 52 on 64x32. What bounds a few rows against a large
 // [K][N] B (16 x 16384 x 16384, 3.5 TB/s; 5.0 with [N][K]) is its 64-byte
 // pieces of rows 32 KB apart.
 constexpr uint32_t kSmallTilesMin = 192;
@@ -1567,55 +1670,164 @@ struct SmallTile {
 template <bool H16, bool B_NK>
 __host__ __device__ __forceinline__ SmallTile gemm_small_shape(uint32_t M, uint32_t N, uint32_t K, uint32_t batch,
                                                                uint32_t P) {
-  if (!H16 || P > 1u || K < 8u || (!B_NK && N < 8u) || M <= 32u) return {32u, 32u};
+  const uint32_t chunk = H16 ? 8u : 4u;
+  if (P > 1u || K < chunk || (!B_NK && N < chunk) || M <= 32u) return {32u, 32u};
   const auto count = [&](uint32_t tm, uint32_t tn) {
     return static_cast<uint64_t>((M - 1u) / tm + 1u) * ((N - 1u) / tn + 1u) * batch;
   };
-  if (M > 64u && N > 64u && count(128u, 128u) >= kSmallTilesMin) return {128u, 128u};
+  if (H16 && M > 64u && N > 64u && count(128u, 128u) >= kSmallTilesMin) return {128u, 128u};
   if (N > 32u && count(64u, 64u) >= kSmallTilesMin) return {64u, 64u};
   if (count(64u, 32u) >= kSmallTilesMin) return {64u, 32u};
   return {32u, 32u};
 }
 
-// A wave's steps of its chunk: s = s_begin + wave + j * kSmallWaves below
-// s_end. Steps whose operands are all in range (an interior tile and a whole
-// step of K) are loaded without guards, up to four before their MFMAs (the
-// later ones under wave-uniform tests); the decision is made once, outside
-// the loops: a load that could take either path inside the loop joins the
-// two in register copies that wait for the loads just issued, which
-// serialises the steps. The rest (at most one short step of K on interior
-// tiles; every step of an edge tile) take the guarded loads one at a time.
-// `load(fast, s, &a, &b)` loads step s into registers of type Reg,
-// `mma(a, b)` accumulates it.
-template <uint32_t KS, typename Reg, typename Load, typename Mma>
-__device__ __forceinline__ void small_steps(uint32_t s_begin, uint32_t s_end, uint32_t wave, bool interior,
-                                            uint32_t K, Load&& load, Mma&& mma) {
-  using Fast = std::true_type;
-  using Slow = std::false_type;
+// small16_steps for fp32 inputs: 16-deep steps of a 32 IM x 32 tile (K >= 4, and
+// N >= 4 for a [K][N] operand), 8 IM v_mfma_f32_32x32x2f32 each; four lanes load
+// the 64 bytes of a row of A or [N][K] B, eight the 128 of a [K][N] row.
+template <int IM, int D, bool B_NK>
+__device__ __forceinline__ void small32_steps(const float* __restrict__ A, const float* __restrict__ B, uint32_t M,
+                                              uint32_t N, uint32_t K, uint32_t m0, uint32_t n0, uint32_t s_begin,
+                                              uint32_t s_end, float* stage, f32x16 (&acc)[IM]) {
+  const uint32_t thread = thread_here(), lane = thread & 63u, wave = __builtin_amdgcn_readfirstlane(thread >> 6);
+  const uint32_t r = lane >> 2, kg = (lane & 3u) * 4u;      // rows of 16: row r (+ 16), k chunk
+  const uint32_t rn = lane >> 3, ng = (lane & 7u) * 4u;     // [K][N] rows of 32: row rn (+ 8), column chunk
+  const float *pa[2 * IM], *pb[2];
+  uint32_t bsh = 0u;
+#pragma unroll
+  for (int i = 0; i < 2 * IM; ++i) {
+    const uint32_t m = m0 + r + 16u * i;
+    pa[i] = A + static_cast<uint64_t>(m < M ? m : M - 1u) * K;
+  }
+  if constexpr (B_NK) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t n = n0 + r + 16u * i;
+      pb[i] = B + static_cast<uint64_t>(n < N ? n : N - 1u) * K;
+    }
+  } else {
+    const uint32_t n = n0 + ng, at = n < N - 4u ? n : N - 4u;
+    bsh = n - at;
+    pb[0] = pb[1] = B + at;
+  }
+  f32x4_t xa[D][2 * IM], xb[D][2];
+  auto load = [&](int d, uint32_t s) {
+    const uint32_t k = s * 16u + kg, kc = k < K - 4u ? k : K - 4u;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if constexpr (B_NK) {
+        xb[d][i] = load16_any(pb[i] + kc);
+      } else {
+        const uint32_t kr = s * 16u + rn + 8u * i;
+        xb[d][i] = load16_any(pb[i] + static_cast<uint64_t>(kr < K ? kr : K - 1u) * N);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * IM; ++i) xa[d][i] = load16_any(pa[i] + kc);
+  };
+#pragma unroll
+  for (int i = 0; i < IM; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+  // One block: the two 8-deep halves of a step sum apart (a shorter chain).
+  f32x16 acc1 = acc[0];
+  const bool edge_n = !B_NK && n0 + 32u > N;
+  const auto rows16 = [](uint32_t row, uint32_t c) { return row * 16u + ((c ^ ((row >> 2) & 3u)) << 2); };
+  auto mma = [&](auto last, int d, uint32_t s) {
+    if (decltype(last)::value && s * 16u + 16u > K) {  // the short last step
+      const uint32_t k = s * 16u + kg, n = k - (k < K - 4u ? k : K - 4u);
+#pragma unroll
+      for (int i = 0; i < 2 * IM; ++i) xa[d][i] = shift_down32(xa[d][i], n);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if constexpr (B_NK) xb[d][i] = shift_down32(xb[d][i], n);
+        else if (s * 16u + rn + 8u * i >= K) xb[d][i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    }
+    if constexpr (!B_NK) {
+      if (edge_n) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) xb[d][i] = shift_down32(xb[d][i], bsh);
+      }
+    }
+    float* bst = stage + 512;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<f32x4_t*>(&bst[B_NK ? rows16(r + 16u * i, lane & 3u) : swz32_kn<32>(rn + 8u * i, ng)]) = xb[d][i];
+    const uint32_t l32 = lane & 31u, hf = lane >> 5;
+    f32x4_t fb[2];
+#pragma unroll
+    for (uint32_t h = 0; h < 2u; ++h) {
+      if constexpr (B_NK) {
+        fb[h] = *reinterpret_cast<const f32x4_t*>(&bst[rows16(l32, 2u * h + hf)]);
+      } else {
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e) fb[h][e] = bst[swz32_kn<32>(8u * h + 4u * hf + e, l32)];
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < IM; ++b) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<f32x4_t*>(&stage[rows16(r + 16u * i, lane & 3u)]) = xa[d][2 * b + i];
+#pragma unroll
+      for (uint32_t h = 0; h < 2u; ++h) {
+        const f32x4_t fa = *reinterpret_cast<const f32x4_t*>(&stage[rows16(l32, 2u * h + hf)]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f32x16& c = IM == 1 && h == 1u ? acc1 : acc[b];
+          c = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[h][e], c, 0, 0, 0);
+        }
+      }
+    }
+  };
   constexpr uint32_t W = kSmallWaves;
   uint32_t s = s_begin + wave;
-  if (interior) {
-    const uint32_t whole = K / KS;  // steps lying wholly inside K
-    const uint32_t fe = s_end < whole ? s_end : whole;
-    // After a group, s moves past the steps it took: the next of this wave's
-    // steps, so the guarded loop below starts at the first one at or past fe.
-    for (; s < fe; s += W * (1u + (s + W < fe) + (s + 2u * W < fe) + (s + 3u * W < fe))) {
-      const bool h1 = s + W < fe, h2 = s + 2u * W < fe, h3 = s + 3u * W < fe;
-      Reg a0, b0, a1, b1, a2, b2, a3, b3;
-      load(Fast{}, s, &a0, &b0);
-      if (h1) load(Fast{}, s + W, &a1, &b1);
-      if (h2) load(Fast{}, s + 2u * W, &a2, &b2);
-      if (h3) load(Fast{}, s + 3u * W, &a3, &b3);
-      mma(a0, b0);
-      if (h1) mma(a1, b1);
-      if (h2) mma(a2, b2);
-      if (h3) mma(a3, b3);
+  if (s >= s_end) return;
+  if (s + (2u * D - 1u) * W < s_end) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, s + d * W);
+    do {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        mma(std::false_type{}, d, s + d * W);
+        load(d, s + (D + d) * W);
+      }
+      s += D * W;
+    } while (s + (2u * D - 1u) * W < s_end);
+  } else {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (s + d * W < s_end) load(d, s + d * W);
+  }
+  for (; s < s_end; s += D * W) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (s + d * W < s_end) mma(std::true_type{}, d, s + d * W);
+      if (s + (D + d) * W < s_end) load(d, s + (D + d) * W);
     }
   }
-  for (; s < s_end; s += W) {
-    Reg a0, b0;
-    load(Slow{}, s, &a0, &b0);
-    mma(a0, b0);
+  if constexpr (IM == 1) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[0][e] += acc1[e];
+  }
+}
+
+// Sums the 16 waves' blocks of 32x32 MFMA results, one block at a time, in wave
+// order, and hands `out` each element: out(row, word, sum), word the
+// element's place in the block's MFMA result.
+template <int IM, typename Out>
+__device__ __forceinline__ void small32_sum(const f32x16 (&acc)[IM], float* red, Out&& out) {
+  const uint32_t tid = thread_here(), lane = tid & 63u, wave = tid >> 6;
+#pragma unroll
+  for (int b = 0; b < IM; ++b) {
+    if (b > 0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) red[wave * 1024u + static_cast<uint32_t>(i) * 64u + lane] = acc[b][i];
+    __syncthreads();
+    float sum = red[tid];
+#pragma unroll
+    for (uint32_t w = 1; w < kSmallWaves; ++w) sum += red[w * 1024u + tid];
+    out(32u * b, tid, sum);
   }
 }
 
@@ -1626,8 +1838,6 @@ __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const vo
                                            float* __restrict__ C, float* __restrict__ part, uint32_t M, uint32_t N,
                                            uint32_t K, Epi epi, SmallTile shape, uint32_t tile, uint32_t gtile,
                                            uint32_t T, uint32_t p, uint32_t P) {
-  constexpr uint32_t KS = H16 ? 16u : 8u;   // k per step
-  constexpr uint32_t KPL = H16 ? 8u : 4u;   // k per lane and step
   __shared__ __attribute__((aligned(16))) float red[kSmallWaves * 1024u];
   const uint32_t tiles_m = (M - 1u) / shape.m + 1u;
   const uint32_t m0 = (tile % tiles_m) * shape.m, n0 = (tile / tiles_m) * shape.n;
@@ -1637,11 +1847,11 @@ __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const vo
     const uint16_t* B = static_cast<const uint16_t*>(Bv);
     uint16_t* lds = reinterpret_cast<uint16_t*>(red);
     if (shape.n == 128u) {
-      gemm16_tile<128, 128, 4, 4, 1, 2, B_NK, F16, false>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
+      gemm16_tile<128, 128, 4, 4, 1, 2, B_NK, F16, false, true>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
       return;
     }
     if (shape.n == 64u) {
-      gemm16_tile<64, 64, 2, 4, 2, 2, B_NK, F16, false>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
+      gemm16_tile<64, 64, 2, 4, 2, 2, B_NK, F16, false, true>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
       return;
     }
     if (K >= 8u && (B_NK || N >= 8u)) {
@@ -1664,90 +1874,56 @@ __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const vo
       return;
     }
   }
-  const uint32_t r = lane & 31u, h = lane >> 5;
-  const uint32_t am = m0 + r, bn = n0 + r;
-  // Chunk p: whole steps [s_begin, s_end) (the last step of K may be short).
-  const uint32_t steps = K / KS + (K % KS != 0u ? 1u : 0u);
-  const uint32_t per = steps / P + (steps % P != 0u ? 1u : 0u);
+  const float* Af = static_cast<const float*>(Av);
+  const float* Bf = static_cast<const float*>(Bv);
+  const auto store = [&](uint32_t row0, uint32_t t, float sum) {
+    const uint32_t sr = small_row<false>(t), sc = small_col(t), m = m0 + row0 + sr, n = n0 + sc;
+    if (P > 1u) part[(static_cast<uint64_t>(p) * T + gtile) * 1024u + (H16 ? sr * 32u + sc : t)] = sum;
+    else if (m < M && n < N) C[static_cast<uint64_t>(m) * N + n] = epi(sum, m, n);
+  };
+  if constexpr (!H16) {
+    if (shape.n == 64u) {
+      gemm32_tile<64, 64, 2, 2, 4, 1, B_NK, false, true>(Af, Bf, C, M, N, K, epi, m0, n0, red, tid);
+      return;
+    }
+    if (K >= 4u && (B_NK || N >= 4u)) {
+      const uint32_t steps = (K - 1u) / 16u + 1u, per = (steps - 1u) / P + 1u;
+      const uint32_t s_begin = p * per < steps ? p * per : steps;
+      const uint32_t s_end = s_begin + per < steps ? s_begin + per : steps;
+      if (shape.m == 64u) {
+        f32x16 acc[2];
+        small32_steps<2, 2, B_NK>(Af, Bf, M, N, K, m0, n0, s_begin, s_end, red + wave * 1024u, acc);
+        small32_sum(acc, red, store);
+      } else {
+        f32x16 acc[1];
+        small32_steps<1, 2, B_NK>(Af, Bf, M, N, K, m0, n0, s_begin, s_end, red + wave * 1024u, acc);
+        small32_sum(acc, red, store);
+      }
+      return;
+    }
+  }
+  // Rows shorter than a chunk: element by element, 2-deep MFMA steps of k =
+  // step + lane / 32, dealt to the waves.
+  f32x16 acc[1];
+  const uint32_t am = m0 + (lane & 31u), bn = n0 + (lane & 31u);
+  const uint32_t steps = K / 2u + K % 2u, per = steps / P + (steps % P != 0u ? 1u : 0u);
   const uint32_t s_begin = p * per < steps ? p * per : steps;
   const uint32_t s_end = s_begin + per < steps ? s_begin + per : steps;
-  // Unguarded vector loads: the whole tile in range and every lane's k run
-  // 16-byte aligned (K a multiple of the run; the tensors are 16-byte
-  // aligned and so is every batch's slice then).
-  const bool interior = m0 + 32u <= M && n0 + 32u <= N && K % KPL == 0u;
-  f32x16 acc;
+  const auto value = [](const void* v, uint64_t i) -> float {
+    if constexpr (!H16) return static_cast<const float*>(v)[i];
+    else if constexpr (F16) return static_cast<float>(static_cast<const _Float16*>(v)[i]);
+    else return static_cast<float>(static_cast<const __bf16*>(v)[i]);
+  };
 #pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-  if constexpr (!H16) {
-    const float* __restrict__ A = static_cast<const float*>(Av);
-    const float* __restrict__ B = static_cast<const float*>(Bv);
-    auto load = [&](auto fast, uint32_t s, float4* a, float4* b) {
-      const uint32_t k0 = s * KS + KPL * h;
-      if constexpr (decltype(fast)::value) {
-        *a = *reinterpret_cast<const float4*>(A + static_cast<uint64_t>(am) * K + k0);
-        if constexpr (B_NK) {
-          *b = *reinterpret_cast<const float4*>(B + static_cast<uint64_t>(bn) * K + k0);
-        } else {
-          const float* q = B + static_cast<uint64_t>(k0) * N + bn;
-          *b = make_float4(q[0], q[N], q[2u * N], q[3u * N]);
-        }
-        return;
-      } else {
-      float va[4], vb[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t k = k0 + e;
-        va[e] = (am < M && k < K) ? A[static_cast<uint64_t>(am) * K + k] : 0.0f;
-        if constexpr (B_NK) vb[e] = (bn < N && k < K) ? B[static_cast<uint64_t>(bn) * K + k] : 0.0f;
-        else vb[e] = (bn < N && k < K) ? B[static_cast<uint64_t>(k) * N + bn] : 0.0f;
-      }
-      *a = make_float4(va[0], va[1], va[2], va[3]);
-      *b = make_float4(vb[0], vb[1], vb[2], vb[3]);
-      }
-    };
-    auto mma = [&](const float4& a, const float4& b) {
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
-    };
-    small_steps<KS, float4>(s_begin, s_end, wave, interior, K, load, mma);
-  } else {  // rows shorter than a chunk (K < 8, or N < 8 with a [K][N] operand): element by element
-    const uint16_t* __restrict__ A = static_cast<const uint16_t*>(Av);
-    const uint16_t* __restrict__ B = static_cast<const uint16_t*>(Bv);
-    auto load = [&](auto, uint32_t s, u32x4* a, u32x4* b) {
-      const uint32_t k0 = s * KS + KPL * h;
-      uint32_t va[8], vb[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t k = k0 + e;
-        va[e] = (am < M && k < K) ? A[static_cast<uint64_t>(am) * K + k] : 0u;
-        if constexpr (B_NK) vb[e] = (bn < N && k < K) ? B[static_cast<uint64_t>(bn) * K + k] : 0u;
-        else vb[e] = (bn < N && k < K) ? B[static_cast<uint64_t>(k) * N + bn] : 0u;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        (*a)[e] = va[2 * e] | (va[2 * e + 1] << 16);
-        (*b)[e] = vb[2 * e] | (vb[2 * e + 1] << 16);
-      }
-    };
-    auto mma = [&](const u32x4& a, const u32x4& b) {
-      acc = mfma_32x32x16_16b<F16>(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc);
-    };
-    small_steps<KS, u32x4>(s_begin, s_end, wave, false, K, load, mma);
+  for (int e = 0; e < 16; ++e) acc[0][e] = 0.0f;
+  for (uint32_t s = s_begin + wave; s < s_end; s += kSmallWaves) {
+    const uint32_t k = 2u * s + (lane >> 5);
+    float a = 0.0f, b = 0.0f;
+    if (am < M && k < K) a = value(Av, static_cast<uint64_t>(am) * K + k);
+    if (bn < N && k < K) b = value(Bv, B_NK ? static_cast<uint64_t>(bn) * K + k : static_cast<uint64_t>(k) * N + bn);
+    acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[0], 0, 0, 0);
   }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) red[wave * 1024u + static_cast<uint32_t>(i) * 64u + lane] = acc[i];
-  __syncthreads();
-  float sum = red[tid];
-#pragma unroll
-  for (uint32_t w = 1; w < kSmallWaves; ++w) sum += red[w * 1024u + tid];
-  const uint32_t sr = small_row<false>(tid), sc = small_col(tid);
-  if (P > 1u) {
-    part[(static_cast<uint64_t>(p) * T + gtile) * 1024u + (H16 ? sr * 32u + sc : tid)] = sum;
-    return;
-  }
-  if (m0 + sr < M && n0 + sc < N) C[static_cast<uint64_t>(m0 + sr) * N + n0 + sc] = epi(sum, m0 + sr, n0 + sc);
+  small32_sum(acc, red, store);
 }
 
 // The P > 1 merge: one 1024-thread workgroup per tile, thread t adds word t

@@ -1,7 +1,8 @@
-"""The 16-bit contractions' any-shape kernel (gemm16_any): which launches take
-it, and its results at the sizes where it can go wrong.
+"""The contractions' any-shape kernels (gemm16_any, gemm_f32_any) and the small
+kernel's tile shapes: which launches take them, and their results at the sizes
+where they can go wrong.
 
-Host-only: every tile of a plane has exactly one owner. The direct-to-LDS
+Host-only: every tile of a 16-bit plane has exactly one owner. The direct-to-LDS
 kernels and the any-shape kernel decide on the device with the same rule
 (gemm16_on_whole_tiles, compiled here for the host); the plan's guards may
 only skip a launch that the rule leaves idle.
@@ -95,8 +96,12 @@ def _say(*a):
     sys.stdout.flush()
 
 
-def _dev16(a, gpu, f16):
+def _dev(a, name, gpu):
     import torch
+    a = np.ascontiguousarray(a)
+    if "_f32" in name:
+        return to_dev(a, gpu)
+    f16 = "_f16" in name
     if f16:
         return to_dev(a.astype(np.float16), gpu)
     return to_dev(oracle.to_bf16_bits(a).view(np.int16), gpu).view(torch.bfloat16)
@@ -104,27 +109,27 @@ def _dev16(a, gpu, f16):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", SHAPES)
-@pytest.mark.parametrize("name", ["gemm_bf16", "gemm_bf16_nt", "gemm_f16"])
+@pytest.mark.parametrize("name", ["gemm_bf16", "gemm_bf16_nt", "gemm_f16", "gemm_f32", "gemm_f32_nt"])
 def test_any_shape_exact(gpu, M, N, K, name):
     _say("gemm any", name, M, N, K)
-    nt, f16 = name.endswith("_nt"), name == "gemm_f16"
+    nt, code = name.endswith("_nt"), 0 if "_f32" in name else 1 if "_f16" in name else 2
     rng = np.random.default_rng(M * 7 + N * 3 + K)
     a = rng.integers(-4, 5, (M, K)).astype(np.float32)
     b = rng.integers(-4, 5, (K, N)).astype(np.float32)
     p = compiled(name)
     bd = np.ascontiguousarray(b.T) if nt else b
-    sel = p.selected_symbols([TensorDesc(0x1000, (M, K), 1 if f16 else 2), TensorDesc(0x1000, bd.shape, 1 if f16 else 2),
+    sel = p.selected_symbols([TensorDesc(0x1000, (M, K), code), TensorDesc(0x1000, bd.shape, code),
                               TensorDesc(0x1000, (M, N), 0)])
-    assert "tca_%s_k0" % name in sel, sel
+    assert "tca_%s_k0%s" % (name, "_v" if code == 0 and min(M, N) >= 4096 else "") in sel, sel
     c = out_dev((M, N), gpu)
-    run(p, [_dev16(a, gpu, f16), _dev16(bd, gpu, f16), c])
+    run(p, [_dev(a, name, gpu), _dev(bd, name, gpu), c])
     got = host(c)
     assert canaries(got) == 0
     assert np.array_equal(got, a @ b)  # exact in fp32: partial sums below 2^24
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", ["bmm_bf16", "bmm_bf16_nt"])
+@pytest.mark.parametrize("name", ["bmm_bf16", "bmm_bf16_nt", "bmm_f32"])
 @pytest.mark.parametrize("B,M,N,K", [(3, 1025, 1027, 77), (2, 130, 8300, 64), (9, 1024, 1152, 96)])
 def test_any_shape_batched_exact(gpu, name, B, M, N, K):
     _say("bmm any", name, B, M, N, K)
@@ -133,12 +138,12 @@ def test_any_shape_batched_exact(gpu, name, B, M, N, K):
     a = rng.integers(-4, 5, (B, M, K)).astype(np.float32)
     b = rng.integers(-4, 5, (B, K, N)).astype(np.float32)
     c = out_dev((B, M, N), gpu)
-    run(compiled(name), [_dev16(a, gpu, False), _dev16(b.transpose(0, 2, 1) if nt else b, gpu, False), c])
+    run(compiled(name), [_dev(a, name, gpu), _dev(b.transpose(0, 2, 1) if nt else b, name, gpu), c])
     assert np.array_equal(host(c), np.matmul(a, b))
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", ["gemm_bf16", "gemm_bf16_nt"])
+@pytest.mark.parametrize("name", ["gemm_bf16", "gemm_bf16_nt", "gemm_f32", "gemm_f32_nt"])
 def test_nonfinite_operands_stay_in_their_rows(gpu, name):
     """Infinities and NaN at the ends of rows: a chunk loaded from before the
     end of its row must not bring a neighbour's values in, nor a clamped row
@@ -153,8 +158,9 @@ def test_nonfinite_operands_stay_in_their_rows(gpu, name):
     with np.errstate(invalid="ignore"):
         want = a.astype(np.float64) @ b.astype(np.float64)
     c = out_dev((M, N), gpu)
-    ta = torch.from_numpy(a).to(gpu).to(torch.bfloat16)
-    tb = torch.from_numpy(np.ascontiguousarray(b.T) if nt else b).to(gpu).to(torch.bfloat16)
+    dtype = torch.float32 if "_f32" in name else torch.bfloat16
+    ta = torch.from_numpy(a).to(gpu).to(dtype)
+    tb = torch.from_numpy(np.ascontiguousarray(b.T) if nt else b).to(gpu).to(dtype)
     run(compiled(name), [ta, tb, c])
     assert np.array_equal(host(c), want.astype(np.float32), equal_nan=True)
 
@@ -168,6 +174,10 @@ SMALL = [("gemm_bf16", 1, 16, 4096, 4100), ("gemm_bf16", 1, 33, 777, 1001), ("ge
          ("gemm_bf16_nt", 1, 1000, 1001, 333), ("gemm_f16_nt", 1, 1000, 1001, 1), ("gemm_bf16", 1, 3, 200001, 66),
          ("gemm_bf16", 1, 150001, 5, 66), ("gemm_bf16", 1, 150001, 9, 66), ("bmm_bf16_nt", 32, 500, 500, 64),
          ("bmm_bf16", 20, 500, 501, 77), ("bmm_bf16", 300, 129, 130, 8), ("bmm_bf16_nt", 70, 200, 200, 9),
+         ("gemm_f32", 1, 16, 4096, 2050), ("gemm_f32", 1, 33, 777, 1001), ("gemm_f32_nt", 1, 33, 777, 1003),
+         ("gemm_f32", 1, 61, 9001, 4), ("gemm_f32_nt", 1, 60, 8001, 67), ("gemm_f32", 1, 1000, 1001, 333),
+         ("gemm_f32_nt", 1, 1001, 1000, 130), ("gemm_f32", 1, 1000, 1001, 3), ("gemm_f32", 1, 150001, 3, 66),
+         ("gemm_f32", 1, 150001, 6, 35), ("bmm_f32", 32, 500, 501, 66), ("bmm_f32", 2000, 31, 33, 17),
          ("bmm_bf16", 3, 40, 72, 3000), ("bmm_bf16_nt", 500, 65, 33, 40), ("bmm_bf16", 2000, 31, 33, 17)]
 
 
@@ -175,13 +185,13 @@ SMALL = [("gemm_bf16", 1, 16, 4096, 4100), ("gemm_bf16", 1, 33, 777, 1001), ("ge
 @pytest.mark.parametrize("name,B,M,N,K", SMALL)
 def test_small_tile_shapes_exact(gpu, name, B, M, N, K):
     _say("small tiles", name, B, M, N, K)
-    nt, f16, batched = name.endswith("_nt"), "_f16" in name, name.startswith("bmm")
+    nt, batched = name.endswith("_nt"), name.startswith("bmm")
     rng = np.random.default_rng(B + M + N + K)
     a = rng.integers(-4, 5, (B, M, K)).astype(np.float32)
     b = rng.integers(-4, 5, (B, K, N)).astype(np.float32)
     bd = b.transpose(0, 2, 1) if nt else b
     c = out_dev((B, M, N) if batched else (M, N), gpu)
-    run(compiled(name), [_dev16(a if batched else a[0], gpu, f16), _dev16(bd if batched else bd[0], gpu, f16), c])
+    run(compiled(name), [_dev(a if batched else a[0], name, gpu), _dev(bd if batched else bd[0], name, gpu), c])
     assert np.array_equal(host(c).reshape(B, M, N), np.matmul(a, b))
 
 
