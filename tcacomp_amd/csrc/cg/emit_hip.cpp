@@ -2264,7 +2264,10 @@ class Emitter {
       << " of run-time length, lanes/row chosen at run time; NV > 0: the row is cached in registers\n";
     // EX: every lane holds exactly NV vectors (the row is NV * S vectors):
     // no loop exit, ownership test or index clamp.
-    o << "template <uint32_t V, uint32_t NV, bool EX>\n__device__ __forceinline__ void " << body_fn << "(\n    "
+    // RG: the row length is not a multiple of V. Rows then start at any element
+    // (unaligned vectors, load_vec's Any), and the TAIL < V elements past the
+    // last whole vector belong to the row's first TAIL lanes, one each.
+    o << "template <uint32_t V, uint32_t NV, bool EX, bool RG = false>\n__device__ __forceinline__ void " << body_fn << "(\n    "
       << sig << ") {\n";
     // Block and lane counts are powers of two: shifts, not divisions.
     // The launch block is max(kMinBlock, S) (the plan's pack record): derived
@@ -2272,7 +2275,8 @@ class Emitter {
     const uint32_t lgBlock = 31 - __builtin_clz(kBlock), lgMin = 31 - __builtin_clz(kMinBlock);
     o << "  const uint32_t C = " << ExtentExpr(g_, geo.col) << ";\n";
     o << "  const uint32_t VECS = C / V;\n";
-    o << "  const uint32_t LS = tca::hip::pack_lanes_log2(VECS, NV > 0u ? NV : " << kCache << "u, " << lgBlock
+    o << "  const uint32_t TAIL = RG ? C - VECS * V : 0u;\n";
+    o << "  const uint32_t LS = tca::hip::pack_lanes_log2(RG ? VECS + 1u : VECS, NV > 0u ? NV : " << kCache << "u, " << lgBlock
       << "u);  // S = 2^LS lanes per row\n";
     o << "  const uint32_t LB = LS > " << lgMin << "u ? LS : " << lgMin << "u;  // the block: 2^LB = max(" << kMinBlock
       << ", S) lanes\n";
@@ -2335,6 +2339,11 @@ class Emitter {
     // loaded up front, tiles produced in the nest as they are produced.
     for (int t : tiles)
       o << "    tca::hip::vec<" << CType(g_.tensors[t].elem) << ", V> xc" << t << "[NV > 0u ? NV : 1u];\n";
+    // The lane's element of the row's tail (RG).
+    o << "    [[maybe_unused]] const bool ok_t = lane < TAIL;\n";
+    o << "    [[maybe_unused]] const uint32_t v_t = RG ? VECS * V + (ok_t ? lane : 0u) : 0u;\n";
+    for (int t : tiles)
+      o << "    [[maybe_unused]] tca::hip::vec<" << CType(g_.tensors[t].elem) << ", 1> xc" << t << "_t{};\n";
     std::vector<int> fromMemory;
     for (int t : tiles)
       if (!produced.count(t)) fromMemory.push_back(t);
@@ -2343,9 +2352,13 @@ class Emitter {
       o << "        if (!EX && j >= NLANE) break;\n";
       o << "        const uint32_t v = EX ? lane + j * S : min(lane + j * S, VECS - 1u);\n";
       for (int t : fromMemory)
-        o << "        xc" << t << "[j] = tca::hip::load_vec_nt<" << CType(g_.tensors[t].elem) << ", V>(t" << t
+        o << "        xc" << t << "[j] = tca::hip::load_vec_nt<" << CType(g_.tensors[t].elem) << ", V, RG>(t" << t
           << " + row_base + static_cast<uint64_t>(v) * V);\n";
-      o << "      }\n    }\n";
+      o << "      }\n";
+      for (int t : fromMemory)
+        o << "      if constexpr (RG) xc" << t << "_t = tca::hip::load_vec<" << CType(g_.tensors[t].elem) << ", 1>(t" << t
+          << " + row_base + v_t);\n";
+      o << "    }\n";
     }
     // The exp-sum of a softmax pair (a max, then a sum of expf(E - max)) in
     // the general register-cached body: its terms take the hardware
@@ -2384,6 +2397,9 @@ class Emitter {
       }
       return eg.Gen(c.root.fn.body);
     };
+    // `any` is the alignment argument of the vector accesses: RG inside the
+    // row body's template, nothing in the split kernels.
+    std::string any = ", RG";
     // Operand vectors of pass p at the (clamped) vector index variable `vc`,
     // named x<t><sfx>: cached tiles alias the cache, others are loaded.
     auto operands = [&](std::ostringstream& b, size_t p, const std::string& ind, bool cached, const std::string& vc,
@@ -2396,11 +2412,11 @@ class Emitter {
           // Re-read by a later pass: let the caches keep it.
           const bool again = lastPass[t] != static_cast<int>(p) || produced.count(t);
           b << ind << "const auto x" << t << sfx << " = tca::hip::" << (again ? "load_vec" : "load_vec_nt") << "<"
-            << T << ", V>(t" << t << " + row_base + static_cast<uint64_t>(" << vc << ") * V);\n";
+            << T << ", V" << any << ">(t" << t << " + row_base + static_cast<uint64_t>(" << vc << ") * V);\n";
         }
       }
       for (int t : passCols[p])
-        b << ind << "const auto x" << t << sfx << " = tca::hip::load_vec<" << CType(g_.tensors[t].elem) << ", V>(t"
+        b << ind << "const auto x" << t << sfx << " = tca::hip::load_vec<" << CType(g_.tensors[t].elem) << ", V" << any << ">(t"
           << t << " + static_cast<uint64_t>(" << vc << ") * V);\n";
     };
     // Work of pass p on one vector (operands x<t><sfx>, index `vc`). `ok`: the
@@ -2442,10 +2458,48 @@ class Emitter {
       if (!isReg(st) || an_.hbm_local[st]) {
         const bool again = tiles.count(st) > 0 && !cached;
         b << ind << "if (active" << (ok == "true" ? std::string() : " && " + ok) << ") tca::hip::"
-          << (again ? "store_vec" : "store_vec_nt") << "<" << T << ", V>(t" << st
+          << (again ? "store_vec" : "store_vec_nt") << "<" << T << ", V" << any << ">(t" << st
           << " + row_base + static_cast<uint64_t>(" << vc << ") * V, outv" << sfx << ");\n";
       }
       if (cached && tiles.count(st)) b << ind << "xc" << st << "[j] = outv" << sfx << ";\n";
+    };
+    // Pass p on the lane's element of the row's tail (RG; folded or stored
+    // only by the TAIL lanes that own one).
+    auto tailOperands = [&](std::ostringstream& b, size_t p, const std::string& ind) {
+      b << ind << "constexpr uint32_t q = 0u;\n";
+      for (int t : passTiles[p]) {
+        const std::string T = CType(g_.tensors[t].elem);
+        b << ind << "tca::hip::vec<" << T << ", 1> x" << t << "_t = xc" << t << "_t;\n";
+        b << ind << "if constexpr (NV == 0u) x" << t << "_t = tca::hip::load_vec<" << T << ", 1>(t" << t
+          << " + row_base + v_t);\n";
+      }
+      for (int t : passCols[p])
+        b << ind << "const auto x" << t << "_t = tca::hip::load_vec<" << CType(g_.tensors[t].elem) << ", 1>(t" << t
+          << " + v_t);\n";
+    };
+    auto tailWork = [&](std::ostringstream& b, size_t p, const std::string& ind) {
+      b << ind << "if constexpr (RG) {\n";
+      const std::string I = ind + "  ";
+      tailOperands(b, p, I);
+      const ir::Chain& c0 = g_.chains[passes[p][0]];
+      if (!c0.reduces.empty()) {
+        for (int ci : passes[p]) {
+          const std::string P = "part" + std::to_string(ci);
+          std::ostringstream es;
+          const std::string ev = elemValue(es, I, g_.chains[ci], "_t");
+          b << es.str() << I << P << " = ok_t ? comb" << ci << "(" << P << ", " << ev << ") : " << P << ";\n";
+        }
+      } else {
+        const int st = c0.store_tensor;
+        const std::string T = CType(g_.tensors[st].elem);
+        std::ostringstream es;
+        const std::string ev = elemValue(es, I, c0, "_t");
+        b << es.str() << I << "tca::hip::vec<" << T << ", 1> outv_t{};\n" << I << "outv_t.set(0, " << ev << ");\n";
+        if (!isReg(st) || an_.hbm_local[st])
+          b << I << "if (active && ok_t) tca::hip::store_vec<" << T << ", 1>(t" << st << " + row_base + v_t, outv_t);\n";
+        if (tiles.count(st)) b << I << "xc" << st << "_t = outv_t;\n";
+      }
+      b << ind << "}\n";
     };
     // Vector k of the lane: index, ownership, clamped index.
     auto index = [&](std::ostringstream& b, const std::string& ind, const std::string& k, const std::string& sfx) {
@@ -2518,6 +2572,7 @@ class Emitter {
       operands(b, p, "        ", false, "vc", "");
       work(b, p, "        ", false, "vc", "ok", "", false);
       b << "      }\n    }\n";
+      tailWork(b, p, "    ");
       o << b.str();
       if (!red) return;
       for (int ci : passes[p])
@@ -2653,7 +2708,15 @@ class Emitter {
         b << K << upd;
       else
         b << K << "if (ok) " << upd;
-      b << J << "}\n" << I << "}\n";
+      b << J << "}\n" << I << "}\n" << I << "if constexpr (RG) {\n";
+      tailOperands(b, p, J);
+      {
+        std::ostringstream es;
+        const std::string ev = elemValue(es, J, A, "_t");
+        b << es.str() << J << "const float et[1] = {" << (online ? "ok_t ? " + ev + " : -__builtin_inff()" : ev) << "};\n";
+        b << J << (online ? "tca::hip::online_expsum_add(om, os, et);\n" : "if (ok_t) tca::hip::chan_add(cs, cm, cn, et);\n");
+      }
+      b << I << "}\n";
       o << b.str();
       // The row's lanes (SEG per segment), then its waves in order.
       if (online) {
@@ -2752,6 +2815,7 @@ class Emitter {
     // wave has read them.
     o << "    if (grp + gridDim.x < ngroups) __syncthreads();\n";
     o << "  }\n}\n";
+    any.clear();
     // Few long rows: each row split over many blocks. Applies when the nest
     // is one pass of reductions (no row maps, no per-row chains) and the
     // rows are indexed by at most one axis. A partial kernel folds a chunk
@@ -3557,7 +3621,19 @@ class Emitter {
           vk.symbol = symbol + (cached ? "_c" : "_s") + std::to_string(w.v) +
                       (kc > kCache ? "x" + std::to_string(kc) : "") + (exact ? "e" : "");
           vk.block = kBlock;
-          vk.pack = cdim + " " + std::to_string((cached ? kc : kCache) * w.v) + " " + std::to_string(kMinBlock);
+          // Row lengths that are no multiple of the widest vector W use it all
+          // the same, unaligned, 4 vectors per lane (RG), once a row has a
+          // lane for each tail element. With vectors of w.v elements, softmax
+          // took 462 us for [4096, 50257] (370-381 so: two reads and a write at
+          // 6.5 TB/s), 42 for [8192, 2047] (26), 47 from bf16 (22); u8 row sums
+          // of [8192, 16001] 92 (30); below 2 W^2 elements both are launch-bound.
+          const uint32_t W = widths[0].v;
+          // Cached rows of a single pass over 4-element vectors keep the lanes
+          // of the narrow width, with vectors twice as wide.
+          const bool ragged = w.v != W;
+          const bool lanesKept = ragged && cached && passes.size() == 1 && W == 4;
+          const uint32_t rv = lanesKept ? 2 * w.v : W, rn = lanesKept ? kCache * w.v / rv : kCache;
+          vk.pack = cdim + " " + std::to_string(ragged ? rn * rv : (cached ? kc : kCache) * w.v) + " " + std::to_string(kMinBlock);
           vk.grid.push_back(DimProduct(geo.outer) + "/pack");
           vk.when.push_back(cdim + " " + std::to_string(lo) + " " + std::to_string(hi) + " " + std::to_string(w.mod) +
                             " " + std::to_string(w.rem));
@@ -3573,7 +3649,24 @@ class Emitter {
           }
           o << "extern \"C\" __global__ void __launch_bounds__(" << kBlock << ") " << vk.symbol << "(\n    " << sig
             << ") {\n";
-          if (cached && canExact) {
+          if (ragged) {
+            const std::string ext = ExtentExpr(g_, geo.col);
+            if (cached && ci == 0) {
+              o << "  if (" << ext << " <= " << 2 * W * W << "u) " << body_fn << "<" << w.v << "u, " << kc << "u, false>(" << args
+                << ");\n  else ";
+            } else {
+              o << "  ";
+            }
+            // A nest of several passes keeps rows of up to 4 vectors a lane in
+            // registers where the narrow widths streamed them: layernorm over
+            // 4000 rows of 10001 87 us against 117, softmax from bf16 over the
+            // same 67 against 89 ([4096, 50257], which still streams in this
+            // kernel, 381 against 370).
+            if (!cached && passes.size() > 1 && lo <= uint64_t{kBlock} * kCache * W)
+              o << "if (" << ext << " <= " << uint64_t{kBlock} * kCache * W << "u) " << body_fn << "<" << W << "u, " << kCache
+                << "u, false, true>(" << args << ");\n  else ";
+            o << body_fn << "<" << rv << "u, " << (cached ? rn : 0u) << "u, false, true>(" << args << ");\n}\n";
+          } else if (cached && canExact) {
             o << "  " << body_fn << "<" << w.v << "u, " << kc << "u, " << (exact ? "true" : "false") << ">(" << args
               << ");\n}\n";
           } else if (cached) {

@@ -16,6 +16,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace tca {
 namespace hip {
 
@@ -66,15 +68,77 @@ struct alignas(sizeof(T) * N) vec<T, N, true> {
   }
 };
 
-template <typename T, int N>
+// N elements from any element address, as 16-byte (or one narrower) accesses:
+// gfx950 serves them unaligned (the amdhsa unaligned access mode), so a row
+// that starts at an odd element still moves 16 bytes per lane. NT: as
+// load_vec_nt. store_vec_any is the store.
+template <typename T, int BYTES>
+struct any_word {  // BYTES per access, aligned as T is
+  typedef unsigned int w1 __attribute__((ext_vector_type(BYTES / 4), aligned(1)));
+  typedef unsigned int w2 __attribute__((ext_vector_type(BYTES / 4), aligned(2)));
+  typedef unsigned int w4 __attribute__((ext_vector_type(BYTES / 4), aligned(4)));
+  typedef typename std::conditional<sizeof(T) == 1, w1, typename std::conditional<sizeof(T) == 2, w2, w4>::type>::type type;
+};
+
+template <typename T, int N, bool NT>
+__device__ __forceinline__ vec<T, N> load_vec_any(const T* __restrict__ p) {
+  constexpr int kBytes = static_cast<int>(sizeof(T)) * N;
+  if constexpr (kBytes % 4 != 0) {
+    vec<T, N> r;
+    for (int i = 0; i < N; ++i) r.set(i, p[i]);
+    return r;
+  } else {
+    constexpr int kStep = kBytes < 16 ? kBytes : 16;
+    typedef typename any_word<T, kStep>::type W;
+    typedef unsigned int R __attribute__((ext_vector_type(kStep / 4)));
+    struct {
+      R w[kBytes / kStep];
+    } r;
+#pragma unroll
+    for (int i = 0; i < kBytes / kStep; ++i) {
+      const W* q = reinterpret_cast<const W*>(reinterpret_cast<const char*>(p) + i * kStep);
+      if constexpr (NT) r.w[i] = __builtin_nontemporal_load(q);
+      else r.w[i] = *q;
+    }
+    return __builtin_bit_cast(vec<T, N>, r);
+  }
+}
+
+template <typename T, int N, bool NT>
+__device__ __forceinline__ void store_vec_any(T* __restrict__ p, const vec<T, N>& x) {
+  constexpr int kBytes = static_cast<int>(sizeof(T)) * N;
+  if constexpr (kBytes % 4 != 0) {
+    for (int i = 0; i < N; ++i) p[i] = x[i];
+  } else {
+    constexpr int kStep = kBytes < 16 ? kBytes : 16;
+    typedef typename any_word<T, kStep>::type W;
+    typedef unsigned int R __attribute__((ext_vector_type(kStep / 4)));
+    struct S {
+      R w[kBytes / kStep];
+    };
+    const S r = __builtin_bit_cast(S, x);
+#pragma unroll
+    for (int i = 0; i < kBytes / kStep; ++i) {
+      W* q = reinterpret_cast<W*>(reinterpret_cast<char*>(p) + i * kStep);
+      if constexpr (NT) __builtin_nontemporal_store(static_cast<W>(r.w[i]), q);
+      else *q = r.w[i];
+    }
+  }
+}
+
+// Any: the address is aligned as an element only.
+template <typename T, int N, bool Any = false>
 __device__ __forceinline__ vec<T, N> load_vec(const T* __restrict__ p) {
-  return *reinterpret_cast<const vec<T, N>*>(p);
+  if constexpr (Any) return load_vec_any<T, N, false>(p);
+  else return *reinterpret_cast<const vec<T, N>*>(p);
 }
 
 // Streaming load: data read exactly once by this kernel.
-template <typename T, int N>
+template <typename T, int N, bool Any = false>
 __device__ __forceinline__ vec<T, N> load_vec_nt(const T* __restrict__ p) {
-  if constexpr (sizeof(T) * N == 16) {
+  if constexpr (Any) {
+    return load_vec_any<T, N, true>(p);
+  } else if constexpr (sizeof(T) * N == 16) {
     typedef unsigned int u4 __attribute__((ext_vector_type(4)));
     u4 r = __builtin_nontemporal_load(reinterpret_cast<const u4*>(p));
     return __builtin_bit_cast(vec<T, N>, r);
@@ -87,16 +151,19 @@ __device__ __forceinline__ vec<T, N> load_vec_nt(const T* __restrict__ p) {
   }
 }
 
-template <typename T, int N>
+template <typename T, int N, bool Any = false>
 __device__ __forceinline__ void store_vec(T* __restrict__ p, const vec<T, N>& x) {
-  *reinterpret_cast<vec<T, N>*>(p) = x;
+  if constexpr (Any) store_vec_any<T, N, false>(p, x);
+  else *reinterpret_cast<vec<T, N>*>(p) = x;
 }
 
 // Streaming store: the output is not re-read by this kernel, so keep it out
 // of the caches' way.
-template <typename T, int N>
+template <typename T, int N, bool Any = false>
 __device__ __forceinline__ void store_vec_nt(T* __restrict__ p, const vec<T, N>& x) {
-  if constexpr (sizeof(T) * N == 16) {
+  if constexpr (Any) {
+    store_vec_any<T, N, true>(p, x);
+  } else if constexpr (sizeof(T) * N == 16) {
     typedef unsigned int u4 __attribute__((ext_vector_type(4)));
     __builtin_nontemporal_store(*reinterpret_cast<const u4*>(&x), reinterpret_cast<u4*>(p));
   } else if constexpr (sizeof(T) * N == 8) {
