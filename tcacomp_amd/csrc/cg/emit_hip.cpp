@@ -1431,6 +1431,17 @@ class Emitter {
         return "c" + std::to_string(a);
       };
     };
+    // A vector access whose rows are 16-byte aligned only when `vec` holds
+    // (the extent is a multiple of 4). Bound by memory; the unaligned form is
+    // the same instruction and costs its cache lines again only where rows
+    // end in the middle of one. y = x g + b + z^T, f32: with element-wise
+    // accesses instead [3001, 2049] took 36.4 us (2.0 TB/s), now 18.4 us (4.0
+    // TB/s); [8192, 8191] 249 us, now 186; aligned [8192, 8192] is as before
+    // (128 us, 6.3 TB/s). Streamed (nt) stores stay: with cached ones
+    // [8192, 8191] took 211 us.
+    auto either = [](const std::string& vec, const std::string& fn, const std::string& T, const std::string& at) {
+      return vec + " ? tca::hip::" + fn + "<" + T + ", 4>(" + at + ") : tca::hip::" + fn + "<" + T + ", 4, true>(" + at + ")";
+    };
     // 1. Output rows p0 + tr + Q i, 4 L values each. The operands read
     // straight from memory are loaded first, so their latency overlaps the
     // tile's (whose LDS writes wait for its own loads).
@@ -1447,7 +1458,7 @@ class Emitter {
     }
     o << "#pragma unroll\n  for (uint32_t i = 0; i < 4u; ++i) {\n";
     o << "    const uint32_t p = p0 + tr + " << Qs << " * i;\n";
-    o << "    full[i] = p < " << EP << " && l_vec && lb + 3u < " << EL << ";\n";
+    o << "    full[i] = p < " << EP << " && lb + 3u < " << EL << ";\n";
     o << "    if (full[i]) {\n";
     for (const auto& r : ops) {
       const std::string T = CType(g_.tensors[r.op->tensor].elem), t = "t" + std::to_string(r.op->tensor);
@@ -1455,8 +1466,9 @@ class Emitter {
       // Aligned operands are read once (streamed); row-contiguous ones are
       // re-read by every row of the grid.
       if (r.cls == TileCls::Aligned || r.cls == TileCls::RowVec)
-        o << "      " << nm << "[i] = tca::hip::load_vec" << (r.cls == TileCls::Aligned ? "_nt" : "") << "<" << T
-          << ", 4>(" << t << " + " << Offset(r.op->tensor, r.op->axes, coordFn("lb", "p")) << ");\n";
+        o << "      " << nm << "[i] = " << either("l_vec", r.cls == TileCls::Aligned ? "load_vec_nt" : "load_vec", T,
+                                                   t + " + " + Offset(r.op->tensor, r.op->axes, coordFn("lb", "p")))
+          << ";\n";
       else if (r.cls == TileCls::Bcast)
         o << "      " << nm << "[i] = " << t << "[" << Offset(r.op->tensor, r.op->axes, coordFn("lb", "p")) << "];\n";
     }
@@ -1471,9 +1483,9 @@ class Emitter {
       o << "  tca::hip::vec<" << T << ", 4> " << zv << "[4];\n  bool " << zf << "[4];\n";
       o << "#pragma unroll\n  for (uint32_t i = 0; i < 4u; ++i) {\n";
       o << "    const uint32_t l = l0 + tr + " << Qs << " * i, p = p0 + 4u * tc;\n";
-      o << "    " << zf << "[i] = l < " << EL << " && p_vec && p + 3u < " << EP << ";\n";
-      o << "    if (" << zf << "[i]) " << zv << "[i] = tca::hip::load_vec_nt<" << T << ", 4>(" << t << " + "
-        << Offset(r.op->tensor, r.op->axes, coordFn("l", "p")) << ");\n";
+      o << "    " << zf << "[i] = l < " << EL << " && p + 3u < " << EP << ";\n";
+      o << "    if (" << zf << "[i]) " << zv << "[i] = "
+        << either("p_vec", "load_vec_nt", T, t + " + " + Offset(r.op->tensor, r.op->axes, coordFn("l", "p"))) << ";\n";
       o << "  }\n";
       o << "#pragma unroll\n  for (uint32_t i = 0; i < 4u; ++i) {\n";
       o << "    const uint32_t lr = tr + " << Qs << " * i, l = l0 + lr, p = p0 + 4u * tc;\n";
@@ -1517,10 +1529,11 @@ class Emitter {
       o << bodyS.str();
       o << "        out.set(q, " << val << ");\n";
       o << "      }\n";
-      o << "      tca::hip::store_vec_nt<" << sT << ", 4>(t" << c.store_tensor << " + "
-        << Offset(c.store_tensor, c.store_axes, coordFn("lb", "p")) << ", out);\n";
+      const std::string at = "t" + std::to_string(c.store_tensor) + " + " + Offset(c.store_tensor, c.store_axes, coordFn("lb", "p"));
+      o << "      if (l_vec) tca::hip::store_vec_nt<" << sT << ", 4>(" << at << ", out);\n";
+      o << "      else tca::hip::store_vec_nt<" << sT << ", 4, true>(" << at << ", out);\n";
     }
-    // Ragged edge or L not a multiple of 4: element by element.
+    // The last, partial vector of a row: element by element.
     o << "    } else {\n";
     o << "      for (uint32_t q = 0; q < 4u; ++q) {\n";
     o << "        if (lb + q >= " << EL << ") break;\n";
