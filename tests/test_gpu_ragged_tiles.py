@@ -7,7 +7,7 @@ import pytest
 
 from helpers import canaries, compiled, host, out_dev, run, to_dev
 from tcacomp_amd.compiler import compile_program
-from tcacomp_amd.pkg import TF32, At, NewBuilder
+from tileprog import three_transposed
 
 pytestmark = pytest.mark.gpu
 
@@ -15,19 +15,9 @@ SIZES = [(1, 1), (3, 2), (5, 7), (127, 129), (129, 127), (130, 126), (128, 131),
          (257, 514), (1001, 1002), (1003, 999)]
 
 
-def _three_transposed():
-    """y = z0^T + z1^T + z2^T: three transposed operands take 64x64 tiles."""
-    b = NewBuilder("ew_tr3_ragged")
-    R, C = b.Dim("R", 0), b.Dim("C", 0)
-    zs = [b.Tensor("z%d" % i, TF32, C, R) for i in range(3)]
-    y = b.Tensor("y", TF32, R, C)
-    b.Stmt().Iter(R, C).Map([At(z, C, R) for z in zs], lambda p, q, r: b.Add(b.Add(p, q), r)).As(R, C).Store(y, R, C)
-    return b.Build()
-
-
 @pytest.fixture(scope="module")
 def three():
-    return compile_program(_three_transposed())
+    return compile_program(three_transposed())
 
 
 def _check(prog, arrays, want, gpu):
