@@ -2642,7 +2642,7 @@ class Emitter {
     // (tca::hip::online_expsum_add) or the pairwise triple (sum, centred sum
     // of squares, count: tca::hip::chan_add); the row's lanes meet by
     // shuffles (both merges are symmetric, so every lane ends with the same
-    // value) and its waves through LDS in wave order. The register-cached
+    // value), and its waves' values through LDS the same way. The register-cached
     // bodies keep the two passes (the row is read from registers either way).
     std::vector<int> streamPair(passes.size(), 0);  // 1 softmax (online), 2 mean and centred squares
     if (opts_.allow_pass_fusion)
@@ -2731,16 +2731,22 @@ class Emitter {
       }
       b << I << "}\n";
       o << b.str();
-      // The row's lanes (SEG per segment), then its waves in order.
+      // The row's lanes (SEG per segment), then its waves: lane l takes wave l
+      // % WPR of the row, and the lanes meet as before. Against the waves in
+      // order (15 dependent merges, each a rounding of the whole sum):
+      // softmax [4096, 50257] 382 -> 371 us, its distance from 64 bits
+      // 9.5e-8 -> 8.2e-8; layernorm [5000, 40000] 360 -> 348, 7.8e-8 -> 6.9e-8.
+      const std::string waves = J + "__syncthreads();\n" + J +
+                                "const uint32_t wl = ((threadIdx.x >> 6) & ~(WPR - 1u)) + (threadIdx.x & (WPR - 1u));\n";
       if (online) {
         o << I << "for (uint32_t off = SEG >> 1; off > 0u; off >>= 1)\n"
           << I << "  tca::hip::online_expsum_merge(om, os, __shfl_xor(om, off, 64), __shfl_xor(os, off, 64));\n";
         o << I << "if (WPR > 1u) {\n" << J << "if ((threadIdx.x & 63u) == 0u) {\n" << K << "red" << sa
           << "[threadIdx.x >> 6] = om;\n" << K << "red" << sb << "[threadIdx.x >> 6] = os;\n" << J << "}\n";
-        o << J << "__syncthreads();\n" << J << "const uint32_t w0 = (threadIdx.x >> 6) & ~(WPR - 1u);\n";
-        o << J << "om = red" << sa << "[w0];\n" << J << "os = red" << sb << "[w0];\n";
-        o << J << "for (uint32_t w = 1; w < WPR; ++w) tca::hip::online_expsum_merge(om, os, red" << sa << "[w0 + w], red"
-          << sb << "[w0 + w]);\n" << I << "}\n";
+        o << waves;
+        o << J << "om = red" << sa << "[wl];\n" << J << "os = red" << sb << "[wl];\n";
+        o << J << "for (uint32_t off = WPR >> 1; off > 0u; off >>= 1)\n"
+          << K << "tca::hip::online_expsum_merge(om, os, __shfl_xor(om, off, 64), __shfl_xor(os, off, 64));\n" << I << "}\n";
       } else {
         o << I << "__shared__ float rn" << sa << "[" << kBlock / 64 << "];\n";
         o << I << "for (uint32_t off = SEG >> 1; off > 0u; off >>= 1)\n"
@@ -2749,10 +2755,11 @@ class Emitter {
         o << I << "if (WPR > 1u) {\n" << J << "if ((threadIdx.x & 63u) == 0u) {\n" << K << "red" << sa
           << "[threadIdx.x >> 6] = cs;\n" << K << "red" << sb << "[threadIdx.x >> 6] = cm;\n" << K << "rn" << sa
           << "[threadIdx.x >> 6] = cn;\n" << J << "}\n";
-        o << J << "__syncthreads();\n" << J << "const uint32_t w0 = (threadIdx.x >> 6) & ~(WPR - 1u);\n";
-        o << J << "cs = red" << sa << "[w0];\n" << J << "cm = red" << sb << "[w0];\n" << J << "cn = rn" << sa << "[w0];\n";
-        o << J << "for (uint32_t w = 1; w < WPR; ++w)\n" << J << "  tca::hip::chan_merge_present(cs, cm, cn, red" << sa
-          << "[w0 + w], red" << sb << "[w0 + w], rn" << sa << "[w0 + w]);\n" << I << "}\n";
+        o << waves;
+        o << J << "cs = red" << sa << "[wl];\n" << J << "cm = red" << sb << "[wl];\n" << J << "cn = rn" << sa << "[wl];\n";
+        o << J << "for (uint32_t off = WPR >> 1; off > 0u; off >>= 1)\n"
+          << K << "tca::hip::chan_merge_present(cs, cm, cn, __shfl_xor(cs, off, 64), __shfl_xor(cm, off, 64), "
+             "__shfl_xor(cn, off, 64));\n" << I << "}\n";
       }
       // A's result: init once (an empty row yields init), the fold, then
       // its piped map.
@@ -3637,7 +3644,7 @@ class Emitter {
           // Row lengths that are no multiple of the widest vector W use it all
           // the same, unaligned, 4 vectors per lane (RG), once a row has a
           // lane for each tail element. With vectors of w.v elements, softmax
-          // took 462 us for [4096, 50257] (370-381 so: two reads and a write at
+          // took 462 us for [4096, 50257] (371 so: two reads and a write at
           // 6.5 TB/s), 42 for [8192, 2047] (26), 47 from bf16 (22); u8 row sums
           // of [8192, 16001] 92 (30); below 2 W^2 elements both are launch-bound.
           const uint32_t W = widths[0].v;
@@ -3674,7 +3681,7 @@ class Emitter {
             // registers where the narrow widths streamed them: layernorm over
             // 4000 rows of 10001 87 us against 117, softmax from bf16 over the
             // same 67 against 89 ([4096, 50257], which still streams in this
-            // kernel, 381 against 370).
+            // kernel, took 381 against 370 then).
             if (!cached && passes.size() > 1 && lo <= uint64_t{kBlock} * kCache * W)
               o << "if (" << ext << " <= " << uint64_t{kBlock} * kCache * W << "u) " << body_fn << "<" << W << "u, " << kCache
                 << "u, false, true>(" << args << ");\n  else ";

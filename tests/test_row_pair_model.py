@@ -11,7 +11,7 @@ scaling) and centred sum of squares, then merged into the lane's (S, M2, n)
 with Chan, Golub & LeVeque's pairwise update in its commutative form
 (tca::hip::chan_merge_present: the two M2 add first, the means and the
 weight by reciprocals). The lanes of a wave meet in a butterfly (offsets
-32 .. 1), the 16 waves in wave order. The finish takes the mean a = S inv_n
+32 .. 1), the 16 waves in another (8 .. 1). The finish takes the mean a = S inv_n
 and sum (x - a)^2 = M2 + n (S / n - a)^2."""
 import numpy as np
 import pytest
@@ -95,9 +95,12 @@ def model_row(x, inv_n, mistake=None):
         s, m2, n = _merge(s, m2, n, s[partner], m2[partner], n[partner], mistake)
         off >>= 1
     ws, wm2, wn = s[::64], m2[::64], n[::64]
-    cs, cm, cn = ws[:1], wm2[:1], wn[:1]
-    for w in range(1, S // 64):
-        cs, cm, cn = _merge(cs, cm, cn, ws[w:w + 1], wm2[w:w + 1], wn[w:w + 1], mistake)
+    cs, cm, cn = ws, wm2, wn
+    off = S // 128
+    while off:
+        partner = np.arange(S // 64) ^ off
+        cs, cm, cn = _merge(cs, cm, cn, cs[partner], cm[partner], cn[partner], mistake)
+        off >>= 1
     mean = F(cs[0] * F(inv_n))
     pd = F(cs[0] / cn[0] - mean)
     total = F(cm[0] + cn[0] * pd * pd)
@@ -213,9 +216,12 @@ def model_softmax_row(x, mistake=None):
         m, s = _online_merge(m, s, m[partner], s[partner])
         off >>= 1
     wm, wsum = m[::64], s[::64]
-    cm, cs = wm[:1], wsum[:1]
-    for w in range(1, S // 64):
-        cm, cs = _online_merge(cm, cs, wm[w:w + 1], wsum[w:w + 1])
+    cm, cs = wm, wsum
+    off = S // 128
+    while off:
+        partner = np.arange(S // 64) ^ off
+        cm, cs = _online_merge(cm, cs, cm[partner], cs[partner])
+        off >>= 1
     a = F(max(F(-np.inf), cm[0]))
     return a, F(cs[0] * _exp(np.array([cm[0] - a], F))[0])
 
