@@ -81,6 +81,15 @@ __device__ __forceinline__ uint32_t thread_here() {
   return t;
 }
 
+// Between the writes and the reads of LDS that lanes of one wave exchange, and
+// between those reads and the next writes. The hardware completes the LDS
+// operations of one wave in order, so this costs no instruction; it tells the
+// compiler, which sees one thread only, that other lanes' values are read.
+__device__ __forceinline__ void wave_exchange() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Unaligned 16-byte accesses: gfx950 serves a 16-byte vector load or store
 // at any element address (the amdhsa unaligned access mode), so rows whose
 // length is not a multiple of the vector still move 16 bytes per lane.
@@ -1574,12 +1583,19 @@ __device__ __forceinline__ void small16_steps(const uint16_t* __restrict__ A, co
         for (int j = 0; j < 2; ++j) xb[d][j] = shift_down16(xb[d][j], bsh);
       }
     }
-    // LDS operations of one wave complete in order: a region is rewritten
-    // behind the reads of what it held.
+    // A region is rewritten behind the reads of what it held.
     uint16_t* bst = stage + 1024;
+    wave_exchange();
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       *reinterpret_cast<u32x4*>(&bst[B_NK ? swz_rows32(r + 16u * j, lane & 3u) : swz_kn<32>(r + 16u * j, kg)]) = xb[d][j];
+    auto stage_a = [&](int h) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<u32x4*>(&stage[swz_rows32(r + 16u * i, lane & 3u)]) = xa[d][2 * h + i];
+    };
+    stage_a(0);
+    wave_exchange();
     bf16x8 fb[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -1588,9 +1604,11 @@ __device__ __forceinline__ void small16_steps(const uint16_t* __restrict__ A, co
     }
 #pragma unroll
     for (int h = 0; h < IM / 2; ++h) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        *reinterpret_cast<u32x4*>(&stage[swz_rows32(r + 16u * i, lane & 3u)]) = xa[d][2 * h + i];
+      if (h > 0) {
+        wave_exchange();
+        stage_a(h);
+        wave_exchange();
+      }
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const bf16x8 fa = *reinterpret_cast<const bf16x8*>(&stage[swz_rows32(16u * i + (lane & 15u), lane >> 4)]);
@@ -1637,6 +1655,7 @@ __device__ __forceinline__ void small16_sum(const f32x4_t (&acc)[IM][2], float* 
 #pragma unroll
   for (int h = 0; h < IM / 2; ++h) {
     if (h > 0) __syncthreads();
+    else wave_exchange();  // the wave's rows held its operands
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1750,9 +1769,17 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
       }
     }
     float* bst = stage + 512;
+    wave_exchange();
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       *reinterpret_cast<f32x4_t*>(&bst[B_NK ? rows16(r + 16u * i, lane & 3u) : swz32_kn<32>(rn + 8u * i, ng)]) = xb[d][i];
+    auto stage_a = [&](int b) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<f32x4_t*>(&stage[rows16(r + 16u * i, lane & 3u)]) = xa[d][2 * b + i];
+    };
+    stage_a(0);
+    wave_exchange();
     const uint32_t l32 = lane & 31u, hf = lane >> 5;
     f32x4_t fb[2];
 #pragma unroll
@@ -1766,9 +1793,11 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
     }
 #pragma unroll
     for (int b = 0; b < IM; ++b) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        *reinterpret_cast<f32x4_t*>(&stage[rows16(r + 16u * i, lane & 3u)]) = xa[d][2 * b + i];
+      if (b > 0) {
+        wave_exchange();
+        stage_a(b);
+        wave_exchange();
+      }
 #pragma unroll
       for (uint32_t h = 0; h < 2u; ++h) {
         const f32x4_t fa = *reinterpret_cast<const f32x4_t*>(&stage[rows16(l32, 2u * h + hf)]);
@@ -1821,6 +1850,7 @@ __device__ __forceinline__ void small32_sum(const f32x16 (&acc)[IM], float* red,
 #pragma unroll
   for (int b = 0; b < IM; ++b) {
     if (b > 0) __syncthreads();
+    else wave_exchange();
 #pragma unroll
     for (int i = 0; i < 16; ++i) red[wave * 1024u + static_cast<uint32_t>(i) * 64u + lane] = acc[b][i];
     __syncthreads();
