@@ -351,34 +351,28 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
   // Output planes of at most kGemmSmallMax elements: 32x32 tiles with K
   // split over the 16 waves of a workgroup and, when the tiles are fewer
   // than the split target, over P chunks (the split record; P > 1 adds the
-  // merge kernel). The tile kernels below carry the complementary guard.
+  // merge kernel); where there are many, its forms of larger tiles, each a
+  // function of its own and on as many workgroups as tiles: in one function
+  // the largest tile's registers, spills and branches were every launch's
+  // (f32 32x32x32 3.2 us on the device, now 2.4; 128x64x256 4.8, now 4.05; 1000 x
+  // 1000 x 512 17, now 13.8; bf16 32 x 500 x 500 x 64 15.2, now 11.4; 1024 x 1024 x
+  // 4096 23.5, now 21.1). The tile kernels below carry the complementary guard.
   std::string bigWhen;
   if (small) {
     const std::string Ms = g.dims[m.m].name, Ns = g.dims[m.n].name, Ks = g.dims[m.k].name;
     const uint32_t kKcMin = bf16 ? 1024u : 512u;  // 4 steps per wave and chunk
-    const uint32_t kBlocks = 512u;                // two 16-wave workgroups per CU
-    // Workgroups past the tiles return at once, but dispatching one costs
-    // 5.5 ns (16 waves each): 64 batches of 1000 x 1000 planes, 65536 tiles of
-    // 32x32 on 4096 of 128x128, spent 250 us on it.
+    const uint32_t kBlocks = 512u;                // two 16-wave workgroups for each CU, one after the other
+    // Dispatching a workgroup of 16 waves costs 5.5 ns, so many batches walk
+    // their tiles; a single contraction has about 500 tiles of a form at most,
+    // and none of its kernels walks (a loop over tiles costs registers).
     const uint32_t kStride = 1024u;
     const std::string part = "__gemmpart" + std::to_string(nest), pdim = "__gemmdim" + std::to_string(nest);
     out->extra_dims.push_back(pdim + " " + std::to_string(uint64_t{kBlocks} * 1024u));
     out->extra_tensors.push_back(part + " f32 local 1 " + pdim);
     const std::string psig = ",\n    float* __restrict__ pw /* " + part + " */";
-    auto body = [&](bool merge) {
-      std::ostringstream b;
-      const std::string h16 = bf16 ? "true" : "false";
-      // P from the 32x32 tiles, as the split record computes it.
-      b << epi.str() << "  const uint32_t P = tca::hip::gemm_split_chunks(K, " << nb
-        << " * (((M + 31u) / 32u) * ((N + 31u) / 32u)), " << kKcMin << "u, " << kBlocks << "u);\n";
-      if (merge)
-        b << "  const uint32_t tiles = ((M + 31u) / 32u) * ((N + 31u) / 32u), T = " << nb << " * tiles, gt = blockIdx.x;\n";
-      else
-        b << "  const auto shape = tca::hip::gemm_small_shape<" << h16 << ", " << nk << ">(M, N, K, " << nb << ", P);\n"
-          << "  const uint32_t tiles = ((M - 1u) / shape.m + 1u) * ((N - 1u) / shape.n + 1u), T = " << nb << " * tiles;\n"
-          << "  for (uint32_t w = blockIdx.x; w < T * P; w += gridDim.x) {\n"
-          << "  if (w != blockIdx.x) __syncthreads();\n"
-          << "  const uint32_t p = w / T, gt = tca::hip::gemm_small_tile(w - p * T, T);\n";
+    const std::string h16 = bf16 ? "true" : "false", sf16 = f16 ? "true" : "false";
+    // The operands of the tile that `gt` counts: (batch, tile) of it.
+    auto call = [&](std::ostringstream& b, const std::string& fn, bool merge, const std::string& rest) {
       std::string a = "t" + std::to_string(ta), bo = "t" + std::to_string(tb), cc = "t" + std::to_string(tc);
       if (batched) {
         b << "  const uint32_t bb = gt / tiles, tile = gt - bb * tiles;\n";
@@ -388,17 +382,66 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
       } else {
         b << "  const uint32_t tile = gt;\n";
       }
-      if (merge)
-        b << "  tca::hip::gemm_small_merge<" << h16 << ">(" << cc << ", pw, M, N, epi, tile, gt, T, P);\n}\n\n";
-      else
-        b << "  tca::hip::gemm_small<" << h16 << ", " << nk << ", decltype(epi)" << (f16 ? ", true" : "") << ">(" << a
-          << ", " << bo << ", " << cc << ", pw, M, N, K, epi, shape, tile, gt, T, p, P);\n  }\n}\n\n";
+      b << "  tca::hip::" << fn << "(" << (merge ? "" : a + ", " + bo + ", ") << cc << rest << ");\n";
+    };
+    // One tile, w, per workgroup, or a walk over them with the grid as its
+    // stride (w stays below 2^32: C has fewer elements by more than any
+    // grid, Bind's kMaxElems).
+    auto walk = [](bool strided, const std::string& bound) {
+      return strided ? "  for (uint32_t w = blockIdx.x; w < " + bound + "; w += gridDim.x) {\n  if (w != blockIdx.x) __syncthreads();\n"
+                     : std::string("  const uint32_t w = blockIdx.x;\n  {\n");
+    };
+    auto body = [&](bool merge) {
+      std::ostringstream b;
+      // P from the 32x32 tiles, as the split record computes it.
+      b << epi.str() << "  const uint32_t tiles = ((M + 31u) / 32u) * ((N + 31u) / 32u), T = " << nb << " * tiles;\n"
+        << "  const uint32_t P = tca::hip::gemm_split_chunks(K, T, " << kKcMin << "u, " << kBlocks << "u);\n";
+      if (merge) {
+        b << "  const uint32_t gt = blockIdx.x;\n";
+        call(b, "gemm_small_merge<" + h16 + ">", true, ", pw, M, N, epi, tile, gt, T, P");
+        b << "}\n\n";
+      } else {
+        b << walk(batched, "T * P") << "  const uint32_t p = P > 1u ? w / T : 0u, gt = tca::hip::gemm_small_tile(w - p * T, T);\n";
+        call(b, "gemm_small<" + h16 + ", " + nk + ", decltype(epi)" + (f16 ? ", true" : "") + ">", false,
+             ", pw, M, N, K, epi, tile, gt, T, p, P");
+        b << "  }\n}\n\n";
+      }
+      return b.str();
+    };
+    // Forms that walk: those whose registers hold the loop without scratch.
+    auto strided = [&](uint32_t TN) { return batched && TN > 32u && (bf16 || !m.b_nk); };
+    auto formBody = [&](uint32_t TM, uint32_t TN) {
+      std::ostringstream b;
+      const std::string tm = std::to_string(TM) + "u", tn = std::to_string(TN) + "u";
+      b << epi.str() << "  const uint32_t tiles = ((M - 1u) / " << tm << " + 1u) * ((N - 1u) / " << tn << " + 1u), T = " << nb
+        << " * tiles;\n"
+        << walk(strided(TN), "T") << "  const uint32_t gt = tca::hip::gemm_small_tile(w, T);\n";
+      call(b, "gemm_small_form<" + h16 + ", " + nk + ", " + tm + ", " + tn + ", " + sf16 + ">", false, ", M, N, K, epi, tile");
+      b << "  }\n}\n\n";
       return b.str();
     };
     o << "extern \"C\" __global__ void __launch_bounds__(1024) " << symbol << "_s(\n    " << signature << psig
       << ") {\n" << body(false);
     o << "extern \"C\" __global__ void __launch_bounds__(1024) " << symbol << "_sm(\n    " << signature << psig
       << ") {\n" << body(true);
+    // Larger tiles while kSmallTilesMin workgroups get one (then K is not
+    // split: P is 1 from 257 tiles of 32x32 on) and rows are a chunk and more.
+    const uint32_t kSmallTilesMin = 192u, chunk = bf16 ? 8u : 4u;
+    std::vector<std::string> forms;
+    for (const auto& f : {std::make_pair(128u, 128u), std::make_pair(64u, 64u), std::make_pair(64u, 32u)}) {
+      if (f.first == 128u && !bf16) continue;
+      const std::string fs = symbol + "_s" + std::to_string(f.first) + "x" + std::to_string(f.second);
+      o << "extern \"C\" __global__ void __launch_bounds__(1024) " << fs << "(\n    " << signature << psig << ") {\n"
+        << formBody(f.first, f.second);
+      // More rows (and columns) than the next smaller tile has.
+      const uint32_t mMin = f.first / 2u + 1u, nMin = f.second > 32u ? f.second / 2u + 1u : m.b_nk ? 1u : chunk;
+      const std::string stride = std::to_string(strided(f.second) ? kStride : 0u);
+      forms.push_back(fs + " " + stride + " 4 " + std::to_string(kSmallTilesMin) +
+                      (batched ? " 3 " + g.dims[m.batch].name + "/1 " : std::string(" 2 ")) + Ms + "/" +
+                      std::to_string(f.first) + " " + Ns + "/" + std::to_string(f.second) + " " + std::to_string(mMin) +
+                      " 1 " + Ms + "/1 " + std::to_string(nMin) + " 1 " + Ns + "/1 " + std::to_string(chunk) + " 1 " + Ks +
+                      "/1");
+    }
     std::vector<std::string> t32;
     if (batched) t32.push_back(g.dims[m.batch].name + "/1");
     t32.push_back(Ms + "/32");
@@ -408,7 +451,7 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
     const std::string splitRec = Ks + " " + std::to_string(kKcMin) + " " + std::to_string(kBlocks);
     const std::string smallWhen = Ms + "*" + Ns + " 0 " + std::to_string(kGemmSmallMax) + " 1 0";
     bigWhen = Ms + "*" + Ns + " " + std::to_string(kGemmSmallMax + 1) + " 18446744073709551615 1 0";
-    const std::string ty = f16 ? "f16 mfma 32x32x16" : bf16 ? "bf16 mfma 32x32x16" : "f32 mfma 32x32x2";
+    const std::string ty = f16 ? "f16 mfma 16x16x32" : bf16 ? "bf16 mfma 16x16x32" : "f32 mfma 32x32x2";
     GemmKernel s;
     s.suffix = "_s";
     s.block = 1024;
@@ -416,11 +459,13 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
     s.when = {smallWhen};
     s.extra_args = {"ptr " + part};
     s.split = splitRec + " 0 " + splitTerms;
-    s.detail = ty + " tile=32x32, K split over 16 waves (and P chunks of >= " + std::to_string(kKcMin) +
+    s.detail = ty + (bf16 ? " tile=32x32 (128x128, 64x64, 64x32 where 192 fit)" : " tile=32x32 (64x64, 64x32 where 192 fit)") +
+               ", K split over 16 waves (and P chunks of >= " + std::to_string(kKcMin) +
                " when the tiles are fewer than " + std::to_string(kBlocks) + "; M*N <= " +
                std::to_string(kGemmSmallMax) + ")" + orient;
     GemmKernel sm = s;
-    s.stride = kStride;
+    s.stride = batched ? kStride : 0u;
+    s.forms = forms;
     sm.suffix = "_sm";
     sm.split = splitRec + " 1 " + splitTerms;
     sm.detail = ty + " small-tile merge: the P chunk partials of each 32x32 tile added in chunk order (P > 1 only)";
@@ -1018,6 +1063,7 @@ class Emitter {
     std::string pack;               // packed row kernel: "<dim> <epl> <min block>"
     std::string split;              // row-split reduction: "<dim> <rows-min> <blocks> <merge> <n> <terms>"
     uint32_t stride = 0;
+    std::vector<std::string> forms;  // "<symbol> <stride> <n> ...": the plan's form records
   };
 
   // -------------------------------------------------------------- analysis
@@ -4931,6 +4977,7 @@ class Emitter {
       for (const auto& a : gk.extra_args) k.args.push_back(a);
       k.split = gk.split;
       k.stride = gk.stride;
+      k.forms = gk.forms;
       AddKernel(k, Family::Gemm, n.chains, gk.detail);
     }
     return true;
@@ -4971,6 +5018,7 @@ class Emitter {
       if (!k.pack.empty()) p << "pack " << k.pack << "\n";
       if (!k.split.empty()) p << "split " << k.split << "\n";
       if (k.stride != 0) p << "stride " << k.stride << "\n";
+      for (const auto& f : k.forms) p << "form " << f << "\n";
       for (const auto& w : k.when) p << "when " << w << "\n";
       for (const auto& w : k.unless) p << "unless " << w << "\n";
     }

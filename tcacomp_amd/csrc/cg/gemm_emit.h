@@ -43,6 +43,7 @@ struct GemmKernel {
   std::vector<std::string> extra_args;  // plan args after the signature's ("ptr <local>")
   std::string split;                    // the plan's split record, if any
   uint32_t stride = 0;                  // the plan's stride record, if > 0
+  std::vector<std::string> forms;       // the plan's form records
   std::string detail;
 };
 

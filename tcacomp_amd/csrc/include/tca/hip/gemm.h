@@ -1475,7 +1475,7 @@ __device__ __forceinline__ void gemm_f32_4w(const float* __restrict__ A, const f
 // The waves of a workgroup read disjoint k, so nothing is shared inside it
 // (small16_steps, small32_steps); neighbouring tiles share panels through the
 // L2. Without a K split larger tiles are taken where they fill the CUs
-// (gemm_small_shape).
+// (gemm_small_form).
 // f32 result element i of lane l is C[m0 + 8(i/4) + 4(l/32) + i%4][n0 + l%32];
 // a wave's tile goes to LDS element-major (word i*64 + l: conflict-free) and
 // thread t = i*64 + l of the workgroup sums word t over the waves.
@@ -1671,35 +1671,6 @@ __device__ __forceinline__ void small16_sum(const f32x4_t (&acc)[IM][2], float* 
   }
 }
 
-// The tile a workgroup of the small kernel takes: 32x32 while K is split over
-// workgroups (P > 1), else the largest of 128x128 (16-bit inputs), 64x64 and
-// 64x32 that still gives kSmallTilesMin workgroups one tile each. A larger
-// tile reads its operands fewer times: 64 x 8192 x 8192 (B as [K][N]) takes
-// 73 us on 32x32 tiles, which read B twice, past what an L2 holds of it in
-// flight, and 54 on 64x32; 1024 x 1024 x 4096 55 on 32x32 and 22 on 64x64; 32
-// batches of 500 x 500 x 64 47 on 32x32 and 16 on 128x128. A 32x64 tile for
-// M <= 32 was within 15% either way; fp32: 1024 x 1024 x 4096 127 us before, 85
-// on 64x64, 64 x 8192 x 4096 81 before, 60 on 32x32, 52 on 64x32. What bounds a few rows against a large
-// [K][N] B (16 x 16384 x 16384, 3.5 TB/s; 5.0 with [N][K]) is its 64-byte
-// pieces of rows 32 KB apart.
-constexpr uint32_t kSmallTilesMin = 192;
-struct SmallTile {
-  uint32_t m, n;
-};
-template <bool H16, bool B_NK>
-__host__ __device__ __forceinline__ SmallTile gemm_small_shape(uint32_t M, uint32_t N, uint32_t K, uint32_t batch,
-                                                               uint32_t P) {
-  const uint32_t chunk = H16 ? 8u : 4u;
-  if (P > 1u || K < chunk || (!B_NK && N < chunk) || M <= 32u) return {32u, 32u};
-  const auto count = [&](uint32_t tm, uint32_t tn) {
-    return static_cast<uint64_t>((M - 1u) / tm + 1u) * ((N - 1u) / tn + 1u) * batch;
-  };
-  if (H16 && M > 64u && N > 64u && count(128u, 128u) >= kSmallTilesMin) return {128u, 128u};
-  if (N > 32u && count(64u, 64u) >= kSmallTilesMin) return {64u, 64u};
-  if (count(64u, 32u) >= kSmallTilesMin) return {64u, 32u};
-  return {32u, 32u};
-}
-
 // small16_steps for fp32 inputs: 16-deep steps of a 32 IM x 32 tile (K >= 4, and
 // N >= 4 for a [K][N] operand), 8 IM v_mfma_f32_32x32x2f32 each; four lanes load
 // the 64 bytes of a row of A or [N][K] B, eight the 128 of a [K][N] row.
@@ -1709,7 +1680,10 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
                                               uint32_t s_end, float* stage, f32x16 (&acc)[IM]) {
   const uint32_t thread = thread_here(), lane = thread & 63u, wave = __builtin_amdgcn_readfirstlane(thread >> 6);
   const uint32_t r = lane >> 2, kg = (lane & 3u) * 4u;      // rows of 16: row r (+ 16), k chunk
-  const uint32_t rn = lane >> 3, ng = (lane & 7u) * 4u;     // [K][N] rows of 32: row rn (+ 8), column chunk
+  // [K][N] rows of 32: row rn (+ 8), column chunk. Lane group q takes row q/2
+  // + 4 (q%2), so that in LDS the rows k and k + 4 that the halves of a wave
+  // read are neighbours: writes and reads go through the 64 banks in lane order.
+  const uint32_t rn = (lane >> 4) + 4u * ((lane >> 3) & 1u), ng = (lane & 7u) * 4u;
   const float *pa[2 * IM], *pb[2];
   uint32_t bsh = 0u;
 #pragma unroll
@@ -1772,7 +1746,7 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
     wave_exchange();
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      *reinterpret_cast<f32x4_t*>(&bst[B_NK ? rows16(r + 16u * i, lane & 3u) : swz32_kn<32>(rn + 8u * i, ng)]) = xb[d][i];
+      *reinterpret_cast<f32x4_t*>(&bst[B_NK ? rows16(r + 16u * i, lane & 3u) : 256u * i + 4u * lane]) = xb[d][i];
     auto stage_a = [&](int b) {
 #pragma unroll
       for (int i = 0; i < 2; ++i)
@@ -1788,7 +1762,7 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
         fb[h] = *reinterpret_cast<const f32x4_t*>(&bst[rows16(l32, 2u * h + hf)]);
       } else {
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) fb[h][e] = bst[swz32_kn<32>(8u * h + 4u * hf + e, l32)];
+        for (uint32_t e = 0; e < 4u; ++e) fb[h][e] = bst[256u * h + 64u * e + lane];  // k = 8h + 4hf + e, column l32
       }
     }
 #pragma unroll
@@ -1861,80 +1835,52 @@ __device__ __forceinline__ void small32_sum(const f32x16 (&acc)[IM], float* red,
   }
 }
 
-// `tile` is the tile within its contraction (of `shape`, column-major), `gtile` the tile's index over all T tiles of the
-// launch (batches included): the partial scratch is indexed by it.
+// One 32x32 tile of C, over chunk p of P of K. `tile` is the tile within its
+// contraction (column-major), `gtile` its index over all T tiles of the launch
+// (batches included): the partial scratch is indexed by it.
 template <bool H16, bool B_NK, typename Epi, bool F16 = false>
 __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const void* __restrict__ Bv,
                                            float* __restrict__ C, float* __restrict__ part, uint32_t M, uint32_t N,
-                                           uint32_t K, Epi epi, SmallTile shape, uint32_t tile, uint32_t gtile,
-                                           uint32_t T, uint32_t p, uint32_t P) {
+                                           uint32_t K, Epi epi, uint32_t tile, uint32_t gtile, uint32_t T, uint32_t p,
+                                           uint32_t P) {
   __shared__ __attribute__((aligned(16))) float red[kSmallWaves * 1024u];
-  const uint32_t tiles_m = (M - 1u) / shape.m + 1u;
-  const uint32_t m0 = (tile % tiles_m) * shape.m, n0 = (tile / tiles_m) * shape.n;
+  const uint32_t tiles_m = (M - 1u) / 32u + 1u;
+  const uint32_t m0 = (tile % tiles_m) * 32u, n0 = (tile / tiles_m) * 32u;
   const uint32_t tid = thread_here(), lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if constexpr (H16) {
-    const uint16_t* A = static_cast<const uint16_t*>(Av);
-    const uint16_t* B = static_cast<const uint16_t*>(Bv);
-    uint16_t* lds = reinterpret_cast<uint16_t*>(red);
-    if (shape.n == 128u) {
-      gemm16_tile<128, 128, 4, 4, 1, 2, B_NK, F16, false, true>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
-      return;
-    }
-    if (shape.n == 64u) {
-      gemm16_tile<64, 64, 2, 4, 2, 2, B_NK, F16, false, true>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
-      return;
-    }
-    if (K >= 8u && (B_NK || N >= 8u)) {
-      const uint32_t steps = (K - 1u) / 32u + 1u, per = (steps - 1u) / P + 1u;
+    if (__builtin_expect(K >= 8u && (B_NK || N >= 8u), 1)) {
+      const uint32_t steps = (K - 1u) / 32u + 1u, per = P > 1u ? (steps - 1u) / P + 1u : steps;
       const uint32_t s_begin = p * per < steps ? p * per : steps;
       const uint32_t s_end = s_begin + per < steps ? s_begin + per : steps;
-      const auto store = [&](uint32_t row, uint32_t col, float sum) {
+      f32x4_t acc[2][2];
+      small16_steps<2, 4, B_NK, F16>(static_cast<const uint16_t*>(Av), static_cast<const uint16_t*>(Bv), M, N, K, m0, n0,
+                                     s_begin, s_end, reinterpret_cast<uint16_t*>(red) + wave * 2048u, acc);
+      small16_sum(acc, red, [&](uint32_t row, uint32_t col, float sum) {
         if (P > 1u) part[(static_cast<uint64_t>(p) * T + gtile) * 1024u + row * 32u + col] = sum;
         else if (m0 + row < M && n0 + col < N) C[static_cast<uint64_t>(m0 + row) * N + n0 + col] = epi(sum, m0 + row, n0 + col);
-      };
-      if (shape.m == 64u) {
-        f32x4_t acc[4][2];
-        small16_steps<4, 2, B_NK, F16>(A, B, M, N, K, m0, n0, s_begin, s_end, lds + wave * 2048u, acc);
-        small16_sum(acc, red, store);
-      } else {
-        f32x4_t acc[2][2];
-        small16_steps<2, 4, B_NK, F16>(A, B, M, N, K, m0, n0, s_begin, s_end, lds + wave * 2048u, acc);
-        small16_sum(acc, red, store);
-      }
+      });
       return;
     }
   }
-  const float* Af = static_cast<const float*>(Av);
-  const float* Bf = static_cast<const float*>(Bv);
-  const auto store = [&](uint32_t row0, uint32_t t, float sum) {
-    const uint32_t sr = small_row<false>(t), sc = small_col(t), m = m0 + row0 + sr, n = n0 + sc;
+  const auto store = [&](uint32_t, uint32_t t, float sum) {
+    const uint32_t sr = small_row<false>(t), sc = small_col(t), m = m0 + sr, n = n0 + sc;
     if (P > 1u) part[(static_cast<uint64_t>(p) * T + gtile) * 1024u + (H16 ? sr * 32u + sc : t)] = sum;
     else if (m < M && n < N) C[static_cast<uint64_t>(m) * N + n] = epi(sum, m, n);
   };
+  f32x16 acc[1];
   if constexpr (!H16) {
-    if (shape.n == 64u) {
-      gemm32_tile<64, 64, 2, 2, 4, 1, B_NK, false, true>(Af, Bf, C, M, N, K, epi, m0, n0, red, tid);
-      return;
-    }
-    if (K >= 4u && (B_NK || N >= 4u)) {
-      const uint32_t steps = (K - 1u) / 16u + 1u, per = (steps - 1u) / P + 1u;
+    if (__builtin_expect(K >= 4u && (B_NK || N >= 4u), 1)) {
+      const uint32_t steps = (K - 1u) / 16u + 1u, per = P > 1u ? (steps - 1u) / P + 1u : steps;
       const uint32_t s_begin = p * per < steps ? p * per : steps;
       const uint32_t s_end = s_begin + per < steps ? s_begin + per : steps;
-      if (shape.m == 64u) {
-        f32x16 acc[2];
-        small32_steps<2, 2, B_NK>(Af, Bf, M, N, K, m0, n0, s_begin, s_end, red + wave * 1024u, acc);
-        small32_sum(acc, red, store);
-      } else {
-        f32x16 acc[1];
-        small32_steps<1, 2, B_NK>(Af, Bf, M, N, K, m0, n0, s_begin, s_end, red + wave * 1024u, acc);
-        small32_sum(acc, red, store);
-      }
+      small32_steps<1, 2, B_NK>(static_cast<const float*>(Av), static_cast<const float*>(Bv), M, N, K, m0, n0, s_begin,
+                                s_end, red + wave * 1024u, acc);
+      small32_sum(acc, red, store);
       return;
     }
   }
   // Rows shorter than a chunk: element by element, 2-deep MFMA steps of k =
   // step + lane / 32, dealt to the waves.
-  f32x16 acc[1];
   const uint32_t am = m0 + (lane & 31u), bn = n0 + (lane & 31u);
   const uint32_t steps = K / 2u + K % 2u, per = steps / P + (steps % P != 0u ? 1u : 0u);
   const uint32_t s_begin = p * per < steps ? p * per : steps;
@@ -1954,6 +1900,58 @@ __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const vo
     acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[0], 0, 0, 0);
   }
   small32_sum(acc, red, store);
+}
+
+// The forms of the small kernel: TM x TN tiles of C, 128x128 (16-bit inputs),
+// 64x64 or 64x32, all of K in one chunk. The plan picks the largest of which
+// there are kSmallTilesMin (emit_hip.cpp), rows of a chunk and more; fewer
+// tiles, or a K split over workgroups, stay 32x32 (gemm_small). A larger tile
+// reads its operands fewer times: 64 x 8192 x 8192 (B as [K][N]) takes 73 us on
+// 32x32 tiles, which read B twice, past what an L2 holds of it in flight, and
+// 54 on 64x32; 1024 x 1024 x 4096 55 on 32x32 and 21 on 64x64; 32 batches of 500
+// x 500 x 64 47 on 32x32 and 11 on 128x128. A 32x64 tile for M <= 32 was within
+// 15% either way; fp32: 1024 x 1024 x 4096 127 us before, 85 on 64x64, 64 x 8192
+// x 4096 81 before, 60 on 32x32, 52 on 64x32. What bounds a few rows against a
+// large [K][N] B (16 x 16384 x 16384, 3.5 TB/s; 5.0 with [N][K]) is its 64-byte
+// pieces of rows 32 KB apart.
+template <bool H16, bool B_NK, uint32_t TM, uint32_t TN, bool F16, typename Epi>
+__device__ __forceinline__ void gemm_small_form(const void* __restrict__ Av, const void* __restrict__ Bv,
+                                                float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
+                                                uint32_t tile) {
+  static_assert((TM == 64u && (TN == 32u || TN == 64u)) || (H16 && TM == 128u && TN == 128u), "the small kernel's forms");
+  __shared__ __attribute__((aligned(16))) float red[kSmallWaves * 1024u];
+  const uint32_t tiles_m = (M - 1u) / TM + 1u;
+  const uint32_t m0 = (tile % tiles_m) * TM, n0 = (tile / tiles_m) * TN;
+  const uint32_t tid = thread_here(), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if constexpr (H16) {
+    const uint16_t* A = static_cast<const uint16_t*>(Av);
+    const uint16_t* B = static_cast<const uint16_t*>(Bv);
+    uint16_t* lds = reinterpret_cast<uint16_t*>(red);
+    if constexpr (TN == 128u) {
+      gemm16_tile<128, 128, 4, 4, 1, 2, B_NK, F16, false, true>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
+    } else if constexpr (TN == 64u) {
+      gemm16_tile<64, 64, 2, 4, 2, 2, B_NK, F16, false, true>(A, B, C, M, N, K, epi, m0, n0, lds, tid);
+    } else {
+      f32x4_t acc[4][2];
+      small16_steps<4, 2, B_NK, F16>(A, B, M, N, K, m0, n0, 0u, (K - 1u) / 32u + 1u, lds + wave * 2048u, acc);
+      small16_sum(acc, red, [&](uint32_t row, uint32_t col, float sum) {
+        if (m0 + row < M && n0 + col < N) C[static_cast<uint64_t>(m0 + row) * N + n0 + col] = epi(sum, m0 + row, n0 + col);
+      });
+    }
+  } else {
+    const float* A = static_cast<const float*>(Av);
+    const float* B = static_cast<const float*>(Bv);
+    if constexpr (TN == 64u) {
+      gemm32_tile<64, 64, 2, 2, 4, 1, B_NK, false, true>(A, B, C, M, N, K, epi, m0, n0, red, tid);
+    } else {
+      f32x16 acc[2];
+      small32_steps<2, 2, B_NK>(A, B, M, N, K, m0, n0, 0u, (K - 1u) / 16u + 1u, red + wave * 1024u, acc);
+      small32_sum(acc, red, [&](uint32_t row0, uint32_t t, float sum) {
+        const uint32_t m = m0 + row0 + small_row<false>(t), n = n0 + small_col(t);
+        if (m < M && n < N) C[static_cast<uint64_t>(m) * N + n] = epi(sum, m, n);
+      });
+    }
+  }
 }
 
 // The P > 1 merge: one 1024-thread workgroup per tile, thread t adds word t

@@ -250,6 +250,32 @@ bool Parse(const std::string& text, Plan* out, std::string* err) {
       if (p.kernels.empty()) return bad("stride before any kernel");
       if (tok.size() != 2 || !ParseU64(tok[1], &p.kernels.back().stride) || p.kernels.back().stride == 0)
         return bad("stride <workgroups>");
+    } else if (kw == "form") {
+      if (p.kernels.empty()) return bad("form before any kernel");
+      const std::string usage = "form <symbol> <stride> <n> <min> <n-terms> <term>... ...";
+      Form f;
+      uint64_t n = 0;
+      if (tok.size() < 4 || !ParseU64(tok[2], &f.stride) || !ParseU64(tok[3], &n) || n == 0 || n > tok.size()) return bad(usage);
+      f.symbol = tok[1];
+      size_t at = 4;
+      for (uint64_t i = 0; i < n; ++i) {
+        Form::Bound b;
+        uint64_t nt = 0;
+        if (at + 2 > tok.size() || !ParseU64(tok[at], &b.min) || !ParseU64(tok[at + 1], &nt) || nt > tok.size() ||
+            at + 2 + nt > tok.size())
+          return bad(usage);
+        at += 2;
+        for (uint64_t j = 0; j < nt; ++j) {
+          Term t;
+          std::string e;
+          if (!ParseTerm(p, tok[at++], &t, &e)) return bad(e);
+          if (t.packed) return bad("a form's term cannot divide by 'pack'");
+          b.terms.push_back(t);
+        }
+        f.bounds.push_back(b);
+      }
+      if (at != tok.size()) return bad(usage);
+      p.kernels.back().forms.push_back(f);
     } else if (kw == "when" || kw == "unless") {
       if (p.kernels.empty()) return bad(kw + " before any kernel");
       Guard g;
@@ -368,6 +394,14 @@ std::string Serialize(const Plan& p) {
       o << "\n";
     }
     if (k.stride != 0) o << "stride " << k.stride << "\n";
+    for (const auto& f : k.forms) {
+      o << "form " << f.symbol << " " << f.stride << " " << f.bounds.size();
+      for (const auto& b : f.bounds) {
+        o << " " << b.min << " " << b.terms.size();
+        for (const auto& t : b.terms) o << " " << TermText(p, t);
+      }
+      o << "\n";
+    }
     for (const auto& g : k.when) o << "when " << GuardText(p, g) << "\n";
     for (const auto& g : k.unless) o << "unless " << GuardText(p, g) << "\n";
   }
@@ -560,6 +594,28 @@ uint32_t PackRows(const Kernel& k, const std::vector<uint32_t>& dims, uint32_t* 
   while (lanes < k.block && lanes * k.pack_epl < dims[k.pack_dim]) lanes <<= 1;
   *block = static_cast<uint32_t>(std::max<uint64_t>(k.pack_min_block, lanes));
   return static_cast<uint32_t>(*block / lanes);
+}
+
+int SelectedForm(const Kernel& k, const std::vector<uint32_t>& dims, uint64_t* grid) {
+  for (size_t i = 0; i < k.forms.size(); ++i) {
+    const Form& f = k.forms[i];
+    uint64_t g = 0;
+    bool all = true;
+    for (size_t j = 0; all && j < f.bounds.size(); ++j) {
+      uint64_t v = 1;  // saturates rather than wraps
+      for (const auto& t : f.bounds[j].terms) {
+        bool overflow = false;
+        const uint64_t x = TermValue(k, t, dims, &overflow);
+        v = overflow || (x != 0 && v > ~uint64_t{0} / x) ? ~uint64_t{0} : v * x;
+      }
+      if (j == 0) g = v;
+      all = v >= f.bounds[j].min;
+    }
+    if (!all) continue;
+    *grid = f.stride != 0 && g > f.stride ? f.stride : g;
+    return static_cast<int>(i);
+  }
+  return -1;
 }
 
 bool Selected(const Kernel& k, const std::vector<uint32_t>& dims) {

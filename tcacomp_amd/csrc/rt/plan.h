@@ -27,6 +27,12 @@
 //       P > 1 (the partials of a nest whose P == 1 case is a mode-2 kernel).
 //   stride <n>    (for the last kernel) the kernel walks its work with the
 //       grid as its stride: at most n workgroups are launched
+//   form <symbol> <stride> <n> <min> <n-terms> <term>... ...    (for the last
+//       kernel) a launch runs the function <symbol>, of the same block and
+//       arguments, in the kernel's place when each of the n products of terms is
+//       at least its <min>, on as many workgroups as the first product (at most
+//       <stride> if that is not 0); the first such form wins. Without one the
+//       kernel itself runs, which is right at every size that its forms are.
 //   when <dim> <lo> <hi> <mod> <rem>    (for the last kernel) the kernel runs only
 //       when lo <= dim <= hi and dim % mod == rem; every guard of a kernel must
 //       hold. <dim> may be a product of dims, d1*d2*... (its value taken in
@@ -98,6 +104,17 @@ struct Guard {
   bool pow2 = false;  // additionally dim / mod is a power of two (rem == 0)
 };
 
+// A function that stands in for its kernel where every bound holds.
+struct Form {
+  struct Bound {
+    uint64_t min = 0;
+    std::vector<Term> terms;  // their product is at least `min`
+  };
+  std::string symbol;
+  uint64_t stride = 0;  // > 0: the most workgroups launched
+  std::vector<Bound> bounds;  // the first is the grid
+};
+
 struct Kernel {
   std::string symbol;
   uint32_t block = 256;
@@ -116,6 +133,7 @@ struct Kernel {
   int split_mode = 0;
   std::vector<Term> split_terms;
   uint64_t stride = 0;  // > 0: the most workgroups launched (a grid-stride kernel)
+  std::vector<Form> forms;
 };
 
 enum SplitMode { kSplitPartial = 0, kSplitMerge = 1, kSplitSingle = 2, kSplitPartialMany = 3 };
@@ -161,6 +179,9 @@ bool GridSize(const Kernel& k, const Plan& p, const std::vector<uint32_t>& dims,
 uint32_t PackRows(const Kernel& k, const std::vector<uint32_t>& dims, uint32_t* block);
 // Row chunks P of a split kernel (1 for a kernel without a split record).
 uint64_t SplitChunks(const Kernel& k, const std::vector<uint32_t>& dims);
+// The form of k that the bound dims run, an index into k.forms, and its grid;
+// -1 (the grid as it was): k itself.
+int SelectedForm(const Kernel& k, const std::vector<uint32_t>& dims, uint64_t* grid);
 // Whether every guard of k holds for the bound dims.
 bool Selected(const Kernel& k, const std::vector<uint32_t>& dims);
 // Packs the kernel arguments per the HIP kernarg ABI (natural alignment):

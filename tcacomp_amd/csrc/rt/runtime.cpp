@@ -134,6 +134,7 @@ struct tca_program_s {
   tca::plan::Plan plan;
   hipModule_t mod = nullptr;
   std::vector<hipFunction_t> funcs;
+  std::vector<std::vector<hipFunction_t>> forms;  // per kernel: its forms' functions
   // HBM locals and partial scratch, one workspace per stream the program is
   // launched on: launches on one stream are ordered and may share it,
   // launches on different streams may overlap and must not.
@@ -350,14 +351,21 @@ int tca_program_load(const char* hsaco_path, const char* plan_text, tca_program*
     return hip_fail(err, "hipModuleLoad");
   }
   for (const auto& k : p->plan.kernels) {
-    hipFunction_t fn = nullptr;
-    err = hipModuleGetFunction(&fn, p->mod, k.symbol.c_str());
-    if (err != hipSuccess) {
-      (void)hipModuleUnload(p->mod);
-      delete p;
-      return fail(TCA_ERR_NOT_FOUND, "program_load: kernel %s missing from %s", k.symbol.c_str(), hsaco_path);
+    std::vector<std::string> symbols = {k.symbol};
+    for (const auto& f : k.forms) symbols.push_back(f.symbol);
+    std::vector<hipFunction_t> fns;
+    for (const auto& s : symbols) {
+      hipFunction_t fn = nullptr;
+      err = hipModuleGetFunction(&fn, p->mod, s.c_str());
+      if (err != hipSuccess) {
+        (void)hipModuleUnload(p->mod);
+        delete p;
+        return fail(TCA_ERR_NOT_FOUND, "program_load: kernel %s missing from %s", s.c_str(), hsaco_path);
+      }
+      fns.push_back(fn);
     }
-    p->funcs.push_back(fn);
+    p->funcs.push_back(fns[0]);
+    p->forms.emplace_back(fns.begin() + 1, fns.end());
   }
   *out = p;
   return TCA_OK;
@@ -512,6 +520,7 @@ int prepare_launch(tca_program p, const tca_tensor* tensors, uint32_t n_tensors,
     uint64_t grid = 0;
     if (!tca::plan::GridSize(k, pl, dims, &grid, &err)) return fail(TCA_ERR_LAUNCH, "%s", err.c_str());
     if (grid == 0) continue;  // nothing to compute (an empty output)
+    const int form = tca::plan::SelectedForm(k, dims, &grid);
     if (grid > 0x7fffffffull)
       return fail(TCA_ERR_LAUNCH, "kernel %s: grid %llu exceeds 2^31-1", k.symbol.c_str(),
                   static_cast<unsigned long long>(grid));
@@ -520,7 +529,7 @@ int prepare_launch(tca_program p, const tca_tensor* tensors, uint32_t n_tensors,
     rc = check_geometry(static_cast<uint32_t>(grid), block, k.lds, l.max_threads, l.max_lds);
     if (rc != TCA_OK) return rc;
     tca_program_s::Prepared::Launch L;
-    L.fn = p->funcs.empty() ? nullptr : p->funcs[ki];
+    L.fn = p->funcs.empty() ? nullptr : form < 0 ? p->funcs[ki] : p->forms[ki][form];
     L.grid = static_cast<uint32_t>(grid);
     L.block = block;
     L.lds = k.lds;
