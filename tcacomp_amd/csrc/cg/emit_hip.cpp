@@ -1063,7 +1063,7 @@ class Emitter {
     std::string pack;               // packed row kernel: "<dim> <epl> <min block>"
     std::string split;              // row-split reduction: "<dim> <rows-min> <blocks> <merge> <n> <terms>"
     uint32_t stride = 0;
-    std::vector<std::string> forms;  // "<symbol> <stride> <n> ...": the plan's form records
+    std::vector<std::string> forms;  // the plan's form records after their keyword (and formpack lines)
   };
 
   // -------------------------------------------------------------- analysis
@@ -2325,8 +2325,9 @@ class Emitter {
     // no loop exit, ownership test or index clamp.
     // RG: the row length is not a multiple of V. Rows then start at any element
     // (unaligned vectors, load_vec's Any), and the TAIL < V elements past the
-    // last whole vector belong to the row's first TAIL lanes, one each.
-    o << "template <uint32_t V, uint32_t NV, bool EX, bool RG = false>\n__device__ __forceinline__ void " << body_fn << "(\n    "
+    // last whole vector belong to the row's first TAIL lanes, one each. NT
+    // false: with RG, vectors go through the caches, not past them.
+    o << "template <uint32_t V, uint32_t NV, bool EX, bool RG = false, bool NT = true>\n__device__ __forceinline__ void " << body_fn << "(\n    "
       << sig << ") {\n";
     // Block and lane counts are powers of two: shifts, not divisions.
     // The launch block is max(kMinBlock, S) (the plan's pack record): derived
@@ -2411,7 +2412,7 @@ class Emitter {
       o << "        if (!EX && j >= NLANE) break;\n";
       o << "        const uint32_t v = EX ? lane + j * S : min(lane + j * S, VECS - 1u);\n";
       for (int t : fromMemory)
-        o << "        xc" << t << "[j] = tca::hip::load_vec_nt<" << CType(g_.tensors[t].elem) << ", V, RG>(t" << t
+        o << "        xc" << t << "[j] = tca::hip::load_vec_nt<" << CType(g_.tensors[t].elem) << ", V, RG, NT>(t" << t
           << " + row_base + static_cast<uint64_t>(v) * V);\n";
       o << "      }\n";
       for (int t : fromMemory)
@@ -2456,9 +2457,9 @@ class Emitter {
       }
       return eg.Gen(c.root.fn.body);
     };
-    // `any` is the alignment argument of the vector accesses: RG inside the
+    // `any` are the alignment arguments of the vector accesses: RG inside the
     // row body's template, nothing in the split kernels.
-    std::string any = ", RG";
+    std::string any = ", RG", anyNt = ", RG, NT";
     // Operand vectors of pass p at the (clamped) vector index variable `vc`,
     // named x<t><sfx>: cached tiles alias the cache, others are loaded.
     auto operands = [&](std::ostringstream& b, size_t p, const std::string& ind, bool cached, const std::string& vc,
@@ -2471,7 +2472,7 @@ class Emitter {
           // Re-read by a later pass: let the caches keep it.
           const bool again = lastPass[t] != static_cast<int>(p) || produced.count(t);
           b << ind << "const auto x" << t << sfx << " = tca::hip::" << (again ? "load_vec" : "load_vec_nt") << "<"
-            << T << ", V" << any << ">(t" << t << " + row_base + static_cast<uint64_t>(" << vc << ") * V);\n";
+            << T << ", V" << (again ? any : anyNt) << ">(t" << t << " + row_base + static_cast<uint64_t>(" << vc << ") * V);\n";
         }
       }
       for (int t : passCols[p])
@@ -2517,7 +2518,7 @@ class Emitter {
       if (!isReg(st) || an_.hbm_local[st]) {
         const bool again = tiles.count(st) > 0 && !cached;
         b << ind << "if (active" << (ok == "true" ? std::string() : " && " + ok) << ") tca::hip::"
-          << (again ? "store_vec" : "store_vec_nt") << "<" << T << ", V" << any << ">(t" << st
+          << (again ? "store_vec" : "store_vec_nt") << "<" << T << ", V" << (again ? any : anyNt) << ">(t" << st
           << " + row_base + static_cast<uint64_t>(" << vc << ") * V, outv" << sfx << ");\n";
       }
       if (cached && tiles.count(st)) b << ind << "xc" << st << "[j] = outv" << sfx << ";\n";
@@ -2882,6 +2883,7 @@ class Emitter {
     o << "    if (grp + gridDim.x < ngroups) __syncthreads();\n";
     o << "  }\n}\n";
     any.clear();
+    anyNt.clear();
     // Few long rows: each row split over many blocks. Applies when the nest
     // is one pass of reductions (no row maps, no per-row chains) and the
     // rows are indexed by at most one axis. A partial kernel folds a chunk
@@ -3689,17 +3691,17 @@ class Emitter {
           vk.block = kBlock;
           // Row lengths that are no multiple of the widest vector W use it all
           // the same, unaligned, 4 vectors per lane (RG), once a row has a
-          // lane for each tail element. With vectors of w.v elements, softmax
-          // took 462 us for [4096, 50257] (371 so: two reads and a write at
-          // 6.5 TB/s), 42 for [8192, 2047] (26), 47 from bf16 (22); u8 row sums
-          // of [8192, 16001] 92 (30); below 2 W^2 elements both are launch-bound.
+          // lane for each tail element (wideFrom). With vectors of w.v elements,
+          // softmax took 462 us for [4096, 50257] (371 so: two reads and a write
+          // at 6.5 TB/s), 42 for [8192, 2047] (26), 47 from bf16 (22); u8 row sums
+          // of [8192, 16001] 92 (30). A kernel whose row lengths start below
+          // wideFrom keeps vectors of w.v elements; its wide bodies are forms of
+          // it, with lanes, blocks and registers of their own.
           const uint32_t W = widths[0].v;
-          // Cached rows of a single pass over 4-element vectors keep the lanes
-          // of the narrow width, with vectors twice as wide.
           const bool ragged = w.v != W;
-          const bool lanesKept = ragged && cached && passes.size() == 1 && W == 4;
-          const uint32_t rv = lanesKept ? 2 * w.v : W, rn = lanesKept ? kCache * w.v / rv : kCache;
-          vk.pack = cdim + " " + std::to_string(ragged ? rn * rv : (cached ? kc : kCache) * w.v) + " " + std::to_string(kMinBlock);
+          const uint64_t wideFrom = 2 * W * W + 1;
+          const bool wide = ragged && lo >= wideFrom;  // no shorter rows
+          vk.pack = cdim + " " + std::to_string(wide ? kCache * W : (cached ? kc : kCache) * w.v) + " " + std::to_string(kMinBlock);
           vk.grid.push_back(DimProduct(geo.outer) + "/pack");
           vk.when.push_back(cdim + " " + std::to_string(lo) + " " + std::to_string(hi) + " " + std::to_string(w.mod) +
                             " " + std::to_string(w.rem));
@@ -3715,14 +3717,54 @@ class Emitter {
           }
           o << "extern \"C\" __global__ void __launch_bounds__(" << kBlock << ") " << vk.symbol << "(\n    " << sig
             << ") {\n";
-          if (ragged) {
-            const std::string ext = ExtentExpr(g_, geo.col);
-            if (cached && ci == 0) {
-              o << "  if (" << ext << " <= " << 2 * W * W << "u) " << body_fn << "<" << w.v << "u, " << kc << "u, false>(" << args
-                << ");\n  else ";
+          if (ragged && !wide) {
+            o << "  " << body_fn << "<" << w.v << "u, " << kc << "u, false>(" << args << ");\n}\n";
+            // Many short rows: 8 blocks of 256 lanes per CU walk them (bf16 sums
+            // of [65536, 127] 7.5 us, 9.0 with a block per 8 rows).
+            const uint32_t kWalk = 2048;
+            vk.stride = kWalk;
+            const bool several = passes.size() > 1;
+            // Wide forms. A single pass over 4-element vectors keeps the lanes and
+            // the walk of the narrow body, with vectors twice as wide (f32 sums of
+            // [65536, 62] 4.2 us narrow, 3.5 so; of [65536, 511] 37 on 4-element
+            // vectors with a block per row group, 28 either way here).
+            const bool twice = !several && W == 4;
+            const uint32_t rv = twice ? 2 * w.v : W, rn = twice ? kCache / 2 : kCache;
+            // For rows of `from` elements and more, `elems` in all if not 0.
+            auto rule = [&](const std::string& suffix, uint64_t from, uint64_t elems) {
+              std::string f = vk.symbol + suffix + " " + std::to_string(twice ? kWalk : 0u) + (elems ? " 3" : " 2") + " 0 1 " +
+                              vk.grid.back() + " " + std::to_string(from) + " 1 " + cdim + "/1";
+              if (elems) f += " " + std::to_string(elems) + " 2 " + DimProduct(geo.outer) + "/1 " + cdim + "/1";
+              vk.forms.push_back(f + "\nformpack " + std::to_string(rn * rv));
+            };
+            auto form = [&](const std::string& suffix, bool nt) {
+              o << "extern \"C\" __global__ void __launch_bounds__(" << kBlock << ") " << vk.symbol << suffix << "(\n    " << sig
+                << ") {\n  " << body_fn << "<" << rv << "u, " << rn << "u, false, true, " << (nt ? "true" : "false") << ">("
+                << args << ");\n}\n";
+            };
+            // "r" streams; up to 64 vectors, where 16 lanes move 256 bytes of a row
+            // that shares its first and last cache line with its neighbours, "rc"
+            // keeps them in the caches (softmax [65536, 127] 13.9 us, 24
+            // streamed; [4096, 1023] 9.0, 8.0 streamed).
+            const uint64_t kStream = 64 * W + 1;
+            if (!twice) {
+              form("r", true);
+              // Few rows of several passes are faster on the narrow body's many
+              // lanes: softmax [4096, 101] 3.1 us narrow, 4.1 wide, layernorm [4096,
+              // 127] 3.3 and 3.4; [4096, 161] 3.9 and 3.5, [500, 2047] 5.2 and 4.5;
+              // past 2048 elements it would take most of a block for a row (softmax
+              // [16, 4095] 4.8, 4.0).
+              const uint64_t kMany = several ? 600000 : 0;
+              if (several) rule("r", std::max<uint64_t>(wideFrom, 2049), 0);
+              rule("r", std::max(wideFrom, kStream), kMany);
+              rule("rc", wideFrom, kMany);
             } else {
-              o << "  ";
+              rule("rc", wideFrom, 0);
             }
+            form("rc", false);
+          } else if (ragged) {
+            const std::string ext = ExtentExpr(g_, geo.col);
+            o << "  ";
             // A nest of several passes keeps rows of up to 4 vectors a lane in
             // registers where the narrow widths streamed them: layernorm over
             // 4000 rows of 10001 87 us against 117, softmax from bf16 over the
@@ -3731,7 +3773,7 @@ class Emitter {
             if (!cached && passes.size() > 1 && lo <= uint64_t{kBlock} * kCache * W)
               o << "if (" << ext << " <= " << uint64_t{kBlock} * kCache * W << "u) " << body_fn << "<" << W << "u, " << kCache
                 << "u, false, true>(" << args << ");\n  else ";
-            o << body_fn << "<" << rv << "u, " << (cached ? rn : 0u) << "u, false, true>(" << args << ");\n}\n";
+            o << body_fn << "<" << W << "u, " << (cached ? kCache : 0u) << "u, false, true>(" << args << ");\n}\n";
           } else if (cached && canExact) {
             o << "  " << body_fn << "<" << w.v << "u, " << kc << "u, " << (exact ? "true" : "false") << ">(" << args
               << ");\n}\n";

@@ -133,11 +133,13 @@ __device__ __forceinline__ vec<T, N> load_vec(const T* __restrict__ p) {
   else return *reinterpret_cast<const vec<T, N>*>(p);
 }
 
-// Streaming load: data read exactly once by this kernel.
-template <typename T, int N, bool Any = false>
+// Streaming load: data read exactly once by this kernel. NT false: kept in the
+// caches all the same (short unaligned rows, whose vectors share cache lines).
+template <typename T, int N, bool Any = false, bool NT = true>
 __device__ __forceinline__ vec<T, N> load_vec_nt(const T* __restrict__ p) {
+  static_assert(NT || Any, "aligned vectors stream");
   if constexpr (Any) {
-    return load_vec_any<T, N, true>(p);
+    return load_vec_any<T, N, NT>(p);
   } else if constexpr (sizeof(T) * N == 16) {
     typedef unsigned int u4 __attribute__((ext_vector_type(4)));
     u4 r = __builtin_nontemporal_load(reinterpret_cast<const u4*>(p));
@@ -159,10 +161,11 @@ __device__ __forceinline__ void store_vec(T* __restrict__ p, const vec<T, N>& x)
 
 // Streaming store: the output is not re-read by this kernel, so keep it out
 // of the caches' way.
-template <typename T, int N, bool Any = false>
+template <typename T, int N, bool Any = false, bool NT = true>
 __device__ __forceinline__ void store_vec_nt(T* __restrict__ p, const vec<T, N>& x) {
+  static_assert(NT || Any, "aligned vectors stream");
   if constexpr (Any) {
-    store_vec_any<T, N, true>(p, x);
+    store_vec_any<T, N, NT>(p, x);
   } else if constexpr (sizeof(T) * N == 16) {
     typedef unsigned int u4 __attribute__((ext_vector_type(4)));
     __builtin_nontemporal_store(*reinterpret_cast<const u4*>(&x), reinterpret_cast<u4*>(p));

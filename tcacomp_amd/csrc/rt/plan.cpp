@@ -269,13 +269,19 @@ bool Parse(const std::string& text, Plan* out, std::string* err) {
           Term t;
           std::string e;
           if (!ParseTerm(p, tok[at++], &t, &e)) return bad(e);
-          if (t.packed) return bad("a form's term cannot divide by 'pack'");
+          if (t.packed && (i != 0 || p.kernels.back().pack_dim < 0))
+            return bad("a form's term divides by 'pack' only in the grid of a packed kernel");
           b.terms.push_back(t);
         }
         f.bounds.push_back(b);
       }
       if (at != tok.size()) return bad(usage);
       p.kernels.back().forms.push_back(f);
+    } else if (kw == "formpack") {
+      if (p.kernels.empty() || p.kernels.back().forms.empty() || p.kernels.back().pack_dim < 0)
+        return bad("formpack before any form of a packed kernel");
+      uint64_t* epl = &p.kernels.back().forms.back().pack_epl;
+      if (tok.size() != 2 || !ParseU64(tok[1], epl) || *epl == 0) return bad("formpack <elements per lane>");
     } else if (kw == "when" || kw == "unless") {
       if (p.kernels.empty()) return bad(kw + " before any kernel");
       Guard g;
@@ -401,6 +407,7 @@ std::string Serialize(const Plan& p) {
         for (const auto& t : b.terms) o << " " << TermText(p, t);
       }
       o << "\n";
+      if (f.pack_epl != 0) o << "formpack " << f.pack_epl << "\n";
     }
     for (const auto& g : k.when) o << "when " << GuardText(p, g) << "\n";
     for (const auto& g : k.unless) o << "unless " << GuardText(p, g) << "\n";
@@ -596,24 +603,31 @@ uint32_t PackRows(const Kernel& k, const std::vector<uint32_t>& dims, uint32_t* 
   return static_cast<uint32_t>(*block / lanes);
 }
 
-int SelectedForm(const Kernel& k, const std::vector<uint32_t>& dims, uint64_t* grid) {
+Kernel FormKernel(const Kernel& k, int i) {
+  const Form& f = k.forms[i];
+  Kernel fk = k;
+  fk.symbol = f.symbol;
+  fk.grid = f.bounds[0].terms;
+  fk.split_dim = -1;
+  fk.stride = f.stride;
+  if (f.pack_epl != 0) fk.pack_epl = f.pack_epl;
+  return fk;
+}
+
+int SelectedForm(const Kernel& k, const std::vector<uint32_t>& dims) {
   for (size_t i = 0; i < k.forms.size(); ++i) {
-    const Form& f = k.forms[i];
-    uint64_t g = 0;
+    const Kernel fk = FormKernel(k, static_cast<int>(i));
     bool all = true;
-    for (size_t j = 0; all && j < f.bounds.size(); ++j) {
+    for (const auto& b : k.forms[i].bounds) {
       uint64_t v = 1;  // saturates rather than wraps
-      for (const auto& t : f.bounds[j].terms) {
+      for (const auto& t : b.terms) {
         bool overflow = false;
-        const uint64_t x = TermValue(k, t, dims, &overflow);
+        const uint64_t x = TermValue(fk, t, dims, &overflow);
         v = overflow || (x != 0 && v > ~uint64_t{0} / x) ? ~uint64_t{0} : v * x;
       }
-      if (j == 0) g = v;
-      all = v >= f.bounds[j].min;
+      all = all && v >= b.min;
     }
-    if (!all) continue;
-    *grid = f.stride != 0 && g > f.stride ? f.stride : g;
-    return static_cast<int>(i);
+    if (all) return static_cast<int>(i);
   }
   return -1;
 }

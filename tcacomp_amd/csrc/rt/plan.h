@@ -33,6 +33,9 @@
 //       at least its <min>, on as many workgroups as the first product (at most
 //       <stride> if that is not 0); the first such form wins. Without one the
 //       kernel itself runs, which is right at every size that its forms are.
+//   formpack <epl>    (for the last form of a packed kernel) the form's own
+//       elements per lane in place of the pack record's; its grid may divide by
+//       'pack', its own rows per block
 //   when <dim> <lo> <hi> <mod> <rem>    (for the last kernel) the kernel runs only
 //       when lo <= dim <= hi and dim % mod == rem; every guard of a kernel must
 //       hold. <dim> may be a product of dims, d1*d2*... (its value taken in
@@ -112,6 +115,7 @@ struct Form {
   };
   std::string symbol;
   uint64_t stride = 0;  // > 0: the most workgroups launched
+  uint64_t pack_epl = 0;  // > 0: a packed kernel's elements per lane
   std::vector<Bound> bounds;  // the first is the grid
 };
 
@@ -179,9 +183,10 @@ bool GridSize(const Kernel& k, const Plan& p, const std::vector<uint32_t>& dims,
 uint32_t PackRows(const Kernel& k, const std::vector<uint32_t>& dims, uint32_t* block);
 // Row chunks P of a split kernel (1 for a kernel without a split record).
 uint64_t SplitChunks(const Kernel& k, const std::vector<uint32_t>& dims);
-// The form of k that the bound dims run, an index into k.forms, and its grid;
-// -1 (the grid as it was): k itself.
-int SelectedForm(const Kernel& k, const std::vector<uint32_t>& dims, uint64_t* grid);
+// The form of k that the bound dims run, an index into k.forms; -1: k itself.
+int SelectedForm(const Kernel& k, const std::vector<uint32_t>& dims);
+// k with the geometry of its form i (symbol, grid, stride, packing).
+Kernel FormKernel(const Kernel& k, int i);
 // Whether every guard of k holds for the bound dims.
 bool Selected(const Kernel& k, const std::vector<uint32_t>& dims);
 // Packs the kernel arguments per the HIP kernarg ABI (natural alignment):

@@ -520,12 +520,14 @@ int prepare_launch(tca_program p, const tca_tensor* tensors, uint32_t n_tensors,
     uint64_t grid = 0;
     if (!tca::plan::GridSize(k, pl, dims, &grid, &err)) return fail(TCA_ERR_LAUNCH, "%s", err.c_str());
     if (grid == 0) continue;  // nothing to compute (an empty output)
-    const int form = tca::plan::SelectedForm(k, dims, &grid);
+    const int form = tca::plan::SelectedForm(k, dims);
+    const tca::plan::Kernel run = form < 0 ? k : tca::plan::FormKernel(k, form);
+    if (form >= 0 && !tca::plan::GridSize(run, pl, dims, &grid, &err)) return fail(TCA_ERR_LAUNCH, "%s", err.c_str());
     if (grid > 0x7fffffffull)
-      return fail(TCA_ERR_LAUNCH, "kernel %s: grid %llu exceeds 2^31-1", k.symbol.c_str(),
+      return fail(TCA_ERR_LAUNCH, "kernel %s: grid %llu exceeds 2^31-1", run.symbol.c_str(),
                   static_cast<unsigned long long>(grid));
     uint32_t block = k.block;
-    (void)tca::plan::PackRows(k, dims, &block);  // packed row kernels size the block at launch
+    (void)tca::plan::PackRows(run, dims, &block);  // packed row kernels size the block at launch
     rc = check_geometry(static_cast<uint32_t>(grid), block, k.lds, l.max_threads, l.max_lds);
     if (rc != TCA_OK) return rc;
     tca_program_s::Prepared::Launch L;
