@@ -36,10 +36,12 @@ def on_whole_tiles(tmp_path_factory):
                         os.path.join(REPO, "tests", "c", "gemm_edge.hip"), "-o", str(out)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
 
-    def ask(shapes):
-        p = subprocess.run([str(out)], input="".join("%d %d %d %d\n" % s for s in shapes), capture_output=True,
+    def ask(shapes, *args):
+        p = subprocess.run([str(out)] + list(args), input="".join("%d %d %d %d\n" % s for s in shapes), capture_output=True,
                            text=True, timeout=60)
         assert p.returncode == 0, p.stderr
+        if args == ("steps",):
+            return [[int(v) for v in l.split()] for l in p.stdout.splitlines()]
         return [bool(int(v)) for v in p.stdout.split()]
     return ask
 
@@ -78,6 +80,15 @@ def test_every_tile_has_one_kernel(on_whole_tiles, name):
         if edges:
             assert "" in sel, (m, n, k, b, sel)
         assert not {"_s", "_sm"} & sel
+
+
+def test_short_slices_take_no_empty_steps(on_whole_tiles):
+    """The fp32 kernel steps through K 8 deep: over all groups of waves as many
+    steps as hold any of K (whole 32-deep slices doubled the work at K = 16)."""
+    shapes = [(1, 1, k, g) for k in (0, 1, 7, 8, 9, 16, 24, 31, 32, 33, 64, 65, 100, 127, 1000, 1001) for g in (1, 2, 4)]
+    for (_, _, k, g), steps in zip(shapes, on_whole_tiles(shapes, "steps")):
+        assert sum(steps) == -(-k // 8), (k, g, steps)
+        assert steps[0] <= 4 * -(-(-(-k // 32)) // g) and steps[0] - steps[-1] <= 4, (k, g, steps)
 
 
 # M, N, K: remainders of the 64- and 128-row tiles and of the 64-deep slice, K

@@ -68,7 +68,7 @@ def _form(plan, dims):
     # batches: as many tiles together; forms that walk stop at 1024 workgroups
     ("bmm_bf16_nt", (32, 500, 500, 64), "128x128", 512), ("bmm_bf16", (64, 1000, 1000, 64), "128x128", 1024),
     ("bmm_bf16", (64, 64, 1000, 64), "64x64", 1024), ("bmm_bf16", (200, 64, 64, 64), "64x64", 200),
-    ("bmm_bf16", (11, 128, 128, 64), "", None), ("bmm_f32", (32, 500, 500, 64), "64x64", 1024),
+    ("bmm_bf16", (11, 128, 128, 64), "", None), ("bmm_f32", (32, 500, 500, 64), "64x64", 2048),
     ("bmm_f32", (500, 40, 32, 64), "64x32", 500)])
 def test_form_rule(name, dims, form, grid):
     plan = programs.CONFIG_PROGRAMS[name]().emit().plan
