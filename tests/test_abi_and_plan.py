@@ -262,13 +262,15 @@ def test_chain_segment_static_drops_the_local():
     (4100, 4096, 4128, ["_v", ""]),
     (4096, 4096, 4100, [""]),        # K % 32 != 0: no tile takes the direct-to-LDS path
     (4096, 4100, 4096, [""]),        # N % 8 != 0: [K][N] rows not 16-byte aligned, no direct-to-LDS tile
-    (257, 4096, 4096, ["_w", ""]), (1025, 1025, 16, [""]),
+    # planes of fewer than 128 whole tiles: the any-shape kernel takes every tile,
+    # so the direct-to-LDS kernel, which would find none, is not launched
+    (257, 4096, 4096, [""]), (2048, 2048, 4096, [""]), (1025, 1025, 16, [""]),
     # output planes of at most 2^20 elements: the small-tile K-split kernel
     (255, 4096, 4096, ["_s"]), (512, 512, 0, ["_s"]), (512, 512, 16, ["_s"]), (64, 64, 4096, ["_s", "_sm"])])
 def test_bf16_gemm_kernel_selection(M, N, K, want):
     """The bf16 contraction's three tile kernels: an 8-wave direct-to-LDS kernel
-    runs when a whole tile can take it (A in 64-deep slices when K % 64 == 0
-    and K >= 256, else in 32-deep slices), the register-staged one unless
+    runs when it takes whole tiles (planes of at least 128 of them; A in 64-deep
+    slices when K % 64 == 0 and K >= 256, else in 32-deep slices), the register-staged one unless
     every tile does (plan `when` / `unless` guards); output planes of
     M*N <= 2^20 take the small-tile kernel instead (and its merge when K is
     split over workgroups)."""

@@ -79,6 +79,8 @@ def test_every_tile_has_one_kernel(on_whole_tiles, name):
             assert ("_w" if k % 64 == 0 and k >= 256 else "_v") in sel, (m, n, k, b, sel)
         if edges:
             assert "" in sel, (m, n, k, b, sel)
+        if m * n * b < WHOLE_MIN:  # no tile is the direct-to-LDS kernels': neither is launched
+            assert sel == {""}, (m, n, k, b, sel)
         assert not {"_s", "_sm"} & sel
 
 
