@@ -415,9 +415,9 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
       std::ostringstream b;
       const std::string tm = std::to_string(TM) + "u", tn = std::to_string(TN) + "u";
       b << epi.str() << "  const uint32_t tiles = ((M - 1u) / " << tm << " + 1u) * ((N - 1u) / " << tn << " + 1u), T = " << nb
-        << " * tiles;\n"
+        << " * tiles;\n  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);\n"
         << walk(strided(TN), "T") << "  const uint32_t gt = tca::hip::gemm_small_tile(w, T);\n";
-      call(b, "gemm_small_form<" + h16 + ", " + nk + ", " + tm + ", " + tn + ", " + sf16 + ">", false, ", M, N, K, epi, tile");
+      call(b, "gemm_small_form<" + h16 + ", " + nk + ", " + tm + ", " + tn + ", " + sf16 + ">", false, ", M, N, K, epi, tile, wave");
       b << "  }\n}\n\n";
       return b.str();
     };
@@ -429,20 +429,23 @@ bool EmitGemm(const Graph& g, const ir::Chain& c, const GemmMatch& m, const std:
     // split: P is 1 from 257 tiles of 32x32 on) and rows are a chunk and more.
     const uint32_t kSmallTilesMin = 192u, chunk = bf16 ? 8u : 4u;
     std::vector<std::string> forms;
-    for (const auto& f : {std::make_pair(128u, 128u), std::make_pair(64u, 64u), std::make_pair(64u, 32u)}) {
-      if (f.first == 128u && !bf16) continue;
-      const std::string fs = symbol + "_s" + std::to_string(f.first) + "x" + std::to_string(f.second);
-      o << "extern \"C\" __global__ void __launch_bounds__(1024) " << fs << "(\n    " << signature << psig << ") {\n"
-        << formBody(f.first, f.second);
-      // More rows (and columns) than the next smaller tile has.
-      const uint32_t mMin = f.first / 2u + 1u, nMin = f.second > 32u ? f.second / 2u + 1u : m.b_nk ? 1u : chunk;
-      const std::string stride = std::to_string(strided(f.second) ? kStride : 0u);
-      forms.push_back(fs + " " + stride + " 4 " + std::to_string(kSmallTilesMin) +
+    // Of tiles of TM x TN: planes of so many rows, columns and k at least.
+    auto form = [&](uint32_t TM, uint32_t TN, uint32_t mMin, uint32_t nMin, uint32_t kMin) {
+      forms.push_back(symbol + "_s" + std::to_string(TM) + "x" + std::to_string(TN) + " " +
+                      std::to_string(strided(TN) ? kStride : 0u) + " 4 " + std::to_string(kSmallTilesMin) +
                       (batched ? " 3 " + g.dims[m.batch].name + "/1 " : std::string(" 2 ")) + Ms + "/" +
-                      std::to_string(f.first) + " " + Ns + "/" + std::to_string(f.second) + " " + std::to_string(mMin) +
-                      " 1 " + Ms + "/1 " + std::to_string(nMin) + " 1 " + Ns + "/1 " + std::to_string(chunk) + " 1 " + Ks +
-                      "/1");
-    }
+                      std::to_string(TM) + " " + Ns + "/" + std::to_string(TN) + " " + std::to_string(mMin) + " 1 " + Ms +
+                      "/1 " + std::to_string(nMin) + " 1 " + Ns + "/1 " + std::to_string(kMin) + " 1 " + Ks + "/1");
+    };
+    const uint32_t nChunk = m.b_nk ? 1u : chunk;
+    // More rows, and columns, than the next smaller tile has.
+    if (bf16) form(128, 128, 65, 65, chunk);
+    form(64, 64, 33, 33, chunk);
+    form(64, 32, 33, nChunk, chunk);
+    for (const auto& f : {std::make_pair(128u, 128u), std::make_pair(64u, 64u), std::make_pair(64u, 32u)})
+      if (bf16 || f.first < 128u)
+        o << "extern \"C\" __global__ void __launch_bounds__(1024) " << symbol << "_s" << f.first << "x" << f.second
+          << "(\n    " << signature << psig << ") {\n" << formBody(f.first, f.second);
     std::vector<std::string> t32;
     if (batched) t32.push_back(g.dims[m.batch].name + "/1");
     t32.push_back(Ms + "/32");

@@ -80,6 +80,12 @@ __device__ __forceinline__ uint32_t thread_here() {
   asm volatile("" : "+v"(t));
   return t;
 }
+// ... and the lane, counted, so that not even the thread index is kept.
+__device__ __forceinline__ uint32_t lane_here() {
+  uint32_t lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  return lane;
+}
 
 // Between the writes and the reads of LDS that lanes of one wave exchange, and
 // between those reads and the next writes. The hardware completes the LDS
@@ -211,11 +217,18 @@ __device__ __forceinline__ bf16x8 frag_b16_tr(const uint16_t* Bs, uint32_t n_col
 // apart 44, operands loaded straight into a 4-deep LDS ring 45 (8 waves) and
 // 55 (4 waves). `TINY` (K-contiguous rows or
 // [K][N] rows shorter than one chunk) loads those element by element.
-// FLUSH: the accumulators are added to a second set every 4 turns (256 k), so
-// the error grows with the root of K as it does for sums split over 16 waves.
+// PAIRS: the two 32-deep products of a slice start from zero, their sum is added
+// to the accumulators, and every 8 turns these to a second set (in the long loop
+// the second product adds to the first). A matrix instruction that adds to a
+// running sum rounds it worse than an addition does, so chains of them show where
+// K is short. Distance from 64 bits, 1e-8, by 16 waves' sums / chains of 8
+// instructions / pairs: 32 batches of 500 x 500, K = 64 4.02 / 4.23 / 3.91, K = 256
+// 7.39 / 8.55 / 5.63; 1000 x 1000, K = 1000 8.87 / 9.29 / 7.49, K = 4096 11.5 / 10.6 /
+// 8.57. Many batches pay up to 5% of their time for it (64 x 1024 x 1024 x 32 76.6 us
+// by chains, 80.3).
 // `lds` holds KG * 2 * 64 * (BM + BN) values; `thread` is threadIdx.x.
 template <uint32_t BM, uint32_t BN, uint32_t WGM, uint32_t WGN, uint32_t KG, int D, bool B_NK, bool F16, bool TINY,
-          bool FLUSH = false, typename Epi>
+          bool PAIRS = false, typename Epi>
 __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                                             float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
                                             uint32_t m0, uint32_t n0, uint16_t* lds, uint32_t thread) {
@@ -327,29 +340,28 @@ __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, cons
   for (int i = 0; i < IM; ++i)
 #pragma unroll
     for (int j = 0; j < JN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  f32x4 sum[FLUSH ? IM : 1][FLUSH ? JN : 1];
-  if constexpr (FLUSH) {
+  f32x4 sum[PAIRS ? IM : 1][PAIRS ? JN : 1];
+  if constexpr (PAIRS) {
 #pragma unroll
     for (int i = 0; i < IM; ++i)
 #pragma unroll
       for (int j = 0; j < JN; ++j) sum[i][j] = acc[i][j];
   }
   auto flush = [&]() {
-    if constexpr (FLUSH) {
+    if constexpr (PAIRS) {
 #pragma unroll
       for (int i = 0; i < IM; ++i)
 #pragma unroll
-        for (int j = 0; j < JN; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            sum[i][j][e] += acc[i][j][e];
-            acc[i][j][e] = 0.0f;
-          }
+        for (int j = 0; j < JN; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
     }
   };
-  auto compute = [&](uint32_t buf) {
+  auto compute = [&](auto last, uint32_t buf) {
     const uint16_t* As = glds + buf * BUF;
     const uint16_t* Bs = As + ASL;
+    f32x4 pair[PAIRS ? IM : 1][PAIRS ? JN : 1];
 #pragma unroll
     for (uint32_t h = 0; h < 2u; ++h) {
       bf16x8 fa[IM], fb[JN];
@@ -368,7 +380,19 @@ __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, cons
 #pragma unroll
       for (int j = 0; j < JN; ++j)
 #pragma unroll
-        for (int i = 0; i < IM; ++i) acc[i][j] = mfma_16x16x32_16b<F16>(fb[j], fa[i], acc[i][j]);
+        for (int i = 0; i < IM; ++i) {
+          if constexpr (PAIRS) {
+            // The long loop: the second product adds to the first.
+            constexpr bool kChain = !decltype(last)::value;
+            const f32x4 from = kChain && h == 1u ? pair[i][j] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            const f32x4 v = mfma_16x16x32_16b<F16>(fb[j], fa[i], from);
+            if (h == 0u) pair[i][j] = v;
+            else acc[i][j] += kChain ? v : pair[i][j] + v;
+          } else {
+            acc[i][j] = mfma_16x16x32_16b<F16>(fb[j], fa[i], acc[i][j]);
+          }
+        }
+      if (PAIRS && h == 0u) __builtin_amdgcn_sched_barrier(0);
     }
   };
   // Turn t of a group (slice t * KG + grp) is written into LDS while turn t-1
@@ -394,8 +418,8 @@ __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, cons
     for (int i = 0; i < U; ++i) {
       write(Body{}, (i + 1) % D, (i + 1) & 1, k_of(t0 + i + 1u));
       load((i + 1) % D, k_of(t0 + i + 1u + D));
-      compute(i & 1);
-      if (FLUSH && (t0 + i) % 4u == 3u) flush();
+      compute(Body{}, i & 1);
+      if (PAIRS && (t0 + i) % 8u == 7u) flush();
       __syncthreads();
     }
   }
@@ -406,13 +430,13 @@ __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, cons
       if (t < nt) {
         if (t + 1u < nt) write(Last{}, (i + 1) % D, (i + 1) & 1, k_of(t + 1u));
         if (t + 1u + D < nt) load((i + 1) % D, k_of(t + 1u + D));
-        compute(i & 1);
-        if (FLUSH && t % 4u == 3u) flush();
+        compute(Last{}, i & 1);
+        if (PAIRS && t % 8u == 7u) flush();
         __syncthreads();
       }
     }
   }
-  if constexpr (FLUSH) {
+  if constexpr (PAIRS) {
     flush();
 #pragma unroll
     for (int i = 0; i < IM; ++i)
@@ -441,7 +465,8 @@ __device__ __forceinline__ void gemm16_tile(const uint16_t* __restrict__ A, cons
     }
   }
   // acc[i][j][e] = C[m][n], m = m0 + wm + 16i + lane%16, n = n0 + wn + 16j + 4(lane/16) + e.
-  const uint32_t mr = m0 + wm + (lane & 15u), nc = n0 + wn + 4u * (lane >> 4);
+  const uint32_t last = lane_here();  // not kept through the loop
+  const uint32_t mr = m0 + wm + (last & 15u), nc = n0 + wn + 4u * (last >> 4);
 #pragma unroll
   for (int b = 0; b < IM * JN; ++b) {
     const int i = b / JN, j = b % JN;
@@ -1194,7 +1219,7 @@ __device__ __forceinline__ void gemm32_tile(const float* __restrict__ A, const f
     const float* As = glds + (NBUF == 2u ? (whole & 1u) * BUF : 0u);
     const uint32_t steps = slice_steps32(K, k_of(whole));
 #pragma unroll 1
-    for (uint32_t h = 0; h < steps; ++h) step(As, As + ASL, h, thread_here() & 63u);
+    for (uint32_t h = 0; h < steps; ++h) step(As, As + ASL, h, lane_here());
     __syncthreads();
   }
   if constexpr (FLUSH) {
@@ -1695,7 +1720,8 @@ __device__ __forceinline__ void small16_sum(const f32x4_t (&acc)[IM][2], float* 
 // small16_steps for fp32 inputs: 16-deep steps of a 32 IM x 32 tile (K >= 4, and
 // N >= 4 for a [K][N] operand), 8 IM v_mfma_f32_32x32x2f32 each; four lanes load
 // the 64 bytes of a row of A or [N][K] B, eight the 128 of a [K][N] row.
-template <int IM, int D, bool B_NK>
+// HALVES: the 8-deep halves of the steps are dealt to the waves instead.
+template <int IM, int D, bool B_NK, bool HALVES = false>
 __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const float* __restrict__ B, uint32_t M,
                                               uint32_t N, uint32_t K, uint32_t m0, uint32_t n0, uint32_t s_begin,
                                               uint32_t s_end, float* stage, f32x16 (&acc)[IM]) {
@@ -1746,7 +1772,9 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
   f32x16 acc1 = acc[0];
   const bool edge_n = !B_NK && n0 + 32u > N;
   const auto rows16 = [](uint32_t row, uint32_t c) { return row * 16u + ((c ^ ((row >> 2) & 3u)) << 2); };
-  auto mma = [&](auto last, int d, uint32_t s) {
+  const uint32_t hsel = wave & 1u;
+  auto mma = [&](auto last, auto one, int d, uint32_t s) {
+    constexpr bool kOne = decltype(one)::value;  // the 8-deep half hsel of the step only
     if (decltype(last)::value && s * 16u + 16u > K) {  // the short last step
       const uint32_t k = s * 16u + kg, n = k - (k < K - 4u ? k : K - 4u);
 #pragma unroll
@@ -1795,6 +1823,7 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
       }
 #pragma unroll
       for (uint32_t h = 0; h < 2u; ++h) {
+        if (kOne && h != hsel) continue;
         const f32x4_t fa = *reinterpret_cast<const f32x4_t*>(&stage[rows16(l32, 2u * h + hf)]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -1804,6 +1833,16 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
       }
     }
   };
+  using Body = std::false_type;
+  using Last = std::true_type;
+  if constexpr (HALVES) {
+    for (uint32_t s = s_begin + (wave >> 1); s < s_end; s += kSmallWaves / 2u) {
+      load(0, s);
+      mma(Last{}, std::true_type{}, 0, s);
+    }
+    return;
+  }
+  constexpr std::false_type both{};
   constexpr uint32_t W = kSmallWaves;
   uint32_t s = s_begin + wave;
   if (s >= s_end) return;
@@ -1813,7 +1852,7 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
     do {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
-        mma(std::false_type{}, d, s + d * W);
+        mma(Body{}, both, d, s + d * W);
         load(d, s + (D + d) * W);
       }
       s += D * W;
@@ -1826,7 +1865,7 @@ __device__ __forceinline__ void small32_steps(const float* __restrict__ A, const
   for (; s < s_end; s += D * W) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      if (s + d * W < s_end) mma(std::true_type{}, d, s + d * W);
+      if (s + d * W < s_end) mma(Last{}, both, d, s + d * W);
       if (s + (D + d) * W < s_end) load(d, s + (D + d) * W);
     }
   }
@@ -1930,20 +1969,21 @@ __device__ __forceinline__ void gemm_small(const void* __restrict__ Av, const vo
 // reads its operands fewer times: 64 x 8192 x 8192 (B as [K][N]) takes 73 us on
 // 32x32 tiles, which read B twice, past what an L2 holds of it in flight, and
 // 54 on 64x32; 1024 x 1024 x 4096 55 on 32x32 and 21 on 64x64; 32 batches of 500
-// x 500 x 64 47 on 32x32 and 11 on 128x128. A 32x64 tile for M <= 32 was within
+// x 500 x 64 47 on 32x32 and 12 on 128x128. A 32x64 tile for M <= 32 was within
 // 15% either way; fp32: 1024 x 1024 x 4096 127 us before, 85 on 64x64, 64 x 8192
 // x 4096 81 before, 60 on 32x32, 52 on 64x32. What bounds a few rows against a
 // large [K][N] B (16 x 16384 x 16384, 3.5 TB/s; 5.0 with [N][K]) is its 64-byte
 // pieces of rows 32 KB apart.
+// `wave` is the thread's, in a scalar register.
 template <bool H16, bool B_NK, uint32_t TM, uint32_t TN, bool F16, typename Epi>
 __device__ __forceinline__ void gemm_small_form(const void* __restrict__ Av, const void* __restrict__ Bv,
                                                 float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
-                                                uint32_t tile) {
+                                                uint32_t tile, uint32_t wave) {
   static_assert((TM == 64u && (TN == 32u || TN == 64u)) || (H16 && TM == 128u && TN == 128u), "the small kernel's forms");
   __shared__ __attribute__((aligned(16))) float red[kSmallWaves * 1024u];
   const uint32_t tiles_m = (M - 1u) / TM + 1u;
   const uint32_t m0 = (tile % tiles_m) * TM, n0 = (tile / tiles_m) * TN;
-  const uint32_t tid = thread_here(), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t tid = wave * 64u + lane_here();
   if constexpr (H16) {
     const uint16_t* A = static_cast<const uint16_t*>(Av);
     const uint16_t* B = static_cast<const uint16_t*>(Bv);
@@ -1966,7 +2006,12 @@ __device__ __forceinline__ void gemm_small_form(const void* __restrict__ Av, con
       gemm32_tile<64, 64, 2, 2, 4, 1, B_NK, false, true>(A, B, C, M, N, K, epi, m0, n0, red, tid);
     } else {
       f32x16 acc[2];
-      small32_steps<2, 2, B_NK>(A, B, M, N, K, m0, n0, 0u, (K - 1u) / 16u + 1u, red + wave * 1024u, acc);
+      const uint32_t steps = (K - 1u) / 16u + 1u;
+      // Up to K = 144, where most waves get one half: more of them work, and no
+      // chain of matrix instructions is longer than with sums of 8 k (60 x 8001 x
+      // 64 4.2 us and 7.7e-8 from 64 bits; 6.2 us, 8.4e-8 by whole steps).
+      if (steps <= 9u) small32_steps<2, 1, B_NK, true>(A, B, M, N, K, m0, n0, 0u, steps, red + wave * 1024u, acc);
+      else small32_steps<2, 2, B_NK>(A, B, M, N, K, m0, n0, 0u, steps, red + wave * 1024u, acc);
       small32_sum(acc, red, [&](uint32_t row0, uint32_t t, float sum) {
         const uint32_t m = m0 + row0 + small_row<false>(t), n = n0 + small_col(t);
         if (m < M && n < N) C[static_cast<uint64_t>(m) * N + n] = epi(sum, m, n);
