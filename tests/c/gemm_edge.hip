@@ -1,6 +1,7 @@
 // Host driver for the __host__ __device__ rules of tca/hip/gemm.h (test
 // program): reads "m n k batch" lines on stdin and prints 1 for each whose
-// whole 256x256 tiles the direct-to-LDS kernels take, else 0. With the argument
+// whole 256x256 tiles the direct-to-LDS kernels take, else 0 (with any argument:
+// in a plan without the small kernel, where no plane is too small). With the argument
 // "steps": the 8-deep MFMA steps that the fp32 kernel takes over K = k in 32-deep
 // slices dealt to `batch` groups of waves, largest group first.
 #include <algorithm>

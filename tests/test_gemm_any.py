@@ -84,6 +84,23 @@ def test_every_tile_has_one_kernel(on_whole_tiles, name):
         assert not {"_s", "_sm"} & sel
 
 
+def test_every_tile_has_one_kernel_without_the_small_kernel(on_whole_tiles):
+    """A plan of the tile kernels alone: whole tiles are the direct-to-LDS
+    kernels' however few they are."""
+    from tcacomp_amd import compiler, programs
+    from tcacomp_amd.pkg import EMIT_NO_GEMM_SPLIT
+    prog = compiler.CompiledProgram("gemm_bf16", programs.CONFIG_PROGRAMS["gemm_bf16"]().emit(flags=EMIT_NO_GEMM_SPLIT), "")
+    shapes = [(256, 256, 256, 1), (256, 256, 32, 1), (300, 256, 64, 1), (255, 4096, 4096, 1), (512, 520, 96, 1),
+              (512, 516, 96, 1), (2048, 2048, 4096, 1), (16, 16, 16, 1), (256, 256, 100, 1)]
+    for (m, n, k, _), whole in zip(shapes, on_whole_tiles(shapes, "all")):
+        sel = {s[len("tca_gemm_bf16_k0"):] for s in prog.selected_symbols(
+            [TensorDesc(0x1000, (m, k), 2), TensorDesc(0x1000, (k, n), 2), TensorDesc(0x1000, (m, n), 0)])}
+        assert whole == (k % 32 == 0 and n % 8 == 0)
+        has_whole = whole and m >= 256 and n >= 256
+        assert (("_w" if k % 64 == 0 and k >= 256 else "_v") in sel) == has_whole, (m, n, k, sel)
+        assert ("" in sel) == (not has_whole or m % 256 != 0 or n % 256 != 0), (m, n, k, sel)
+
+
 def test_short_slices_take_no_empty_steps(on_whole_tiles):
     """The fp32 kernel steps through K 8 deep: over all groups of waves as many
     steps as hold any of K (whole 32-deep slices doubled the work at K = 16)."""
