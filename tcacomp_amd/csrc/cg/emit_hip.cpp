@@ -2494,8 +2494,13 @@ class Emitter {
         // Unaligned wide vectors (RG) fold pairwise, then into the lane's value:
         // wide lanes hold 4 times the narrow body's elements, and one by one
         // their sums are further from 64 bits (softmax [8192, 255] 6.9e-8, narrow
-        // 6.3e-8, so 6.4e-8; the time is the same).
-        if (cached) {
+        // 6.3e-8, so 6.4e-8; the time is the same). Maxima and minima do not round.
+        bool rounds = false;
+        for (int ci : passes[p]) {
+          const ir::Expr& f = g_.exprs[g_.chains[ci].reduces[0].fn.body];
+          rounds = rounds || (f.op == Op::Bin && g_.exprs[g_.chains[ci].root.fn.body].type == Elem::F32);
+        }
+        if (cached && rounds) {
           b << ind << "if constexpr (RG) {\n";
           for (int ci : passes[p])
             b << ind << "  " << CType(g_.exprs[g_.chains[ci].root.fn.body].type) << " fold" << ci << "[V];\n";
@@ -2532,7 +2537,7 @@ class Emitter {
             b << ind << "  " << P << " = " << ok << " ? " << folded << " : " << P << ";\n";
         }
         b << ind << "}\n";
-        if (cached) b << ind << "}\n";
+        if (cached && rounds) b << ind << "}\n";
         for (int ci : passes[p])
           if (FoldFenced(g_.exprs[g_.chains[ci].root.fn.body].type))
             b << ind << "tca::hip::fold_fence(part" << ci << ");\n";
