@@ -55,7 +55,8 @@ struct GemmEmitted {
 
 // Output planes of at most kGemmSmallMax elements (M*N) take the small-tile
 // kernel (32x32 tiles, K split over the waves of a workgroup and, when the
-// tiles are few, over workgroups); larger ones the 128/256 tile kernels.
+// tiles are few, over workgroups; larger tiles where there are many); larger
+// ones the tile kernels.
 constexpr uint64_t kGemmSmallMax = 1ull << 20;
 // 16-bit planes (all batches together) of at least kGemmWholeMin elements,
 // 128 tiles of 256x256, run on the direct-to-LDS kernels where they are whole

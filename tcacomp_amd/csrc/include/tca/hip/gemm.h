@@ -134,8 +134,9 @@ constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | (7 << 4) | ((lg
 // sides): a round of 256x256 tiles takes 95 us, 128x128 tiles 0.16 us each,
 // and the ragged edges, which gemm16_any takes afterwards, 40 us. Planes that
 // are whole tiles throughout compare the first two: from WHOLE_MIN elements
-// on (150 tiles; the plan's guards carry the same bound, and skip gemm16_any
-// there); planes with edges also pay the third. WHOLE_MIN 0: always.
+// on (128 tiles; the times cross at 150, but with that bound 2304 x 4096 x 4096
+// took 109 us against 84; the plan's guards carry the same bound, and skip
+// gemm16_any there); planes with edges also pay the third. WHOLE_MIN 0: always.
 template <uint64_t WHOLE_MIN>
 __host__ __device__ __forceinline__ bool gemm16_on_whole_tiles(uint32_t M, uint32_t N, uint32_t batch) {
   if constexpr (WHOLE_MIN == 0u) return true;
@@ -517,7 +518,7 @@ __device__ __forceinline__ void gemm16_any(const __bf16* __restrict__ A, const _
 }
 
 // -------------------------------------------- bf16 path, 8 waves per tile
-// The direct-to-LDS tiles (gemm_bf16_dma_tile): 512 threads, 2 waves per
+// Whole tiles (gemm16_whole_coords), loaded straight into LDS: 512 threads, 2 waves per
 // SIMD, each wave 128x64 of C as 8x4 blocks of v_mfma_f32_16x16x32_bf16
 // (32 accumulators of 4, 225 VGPRs, no scratch).
 //
@@ -1277,7 +1278,9 @@ __device__ __forceinline__ void gemm32_tile(const float* __restrict__ A, const f
 // x 4096 x 2048 on 256x256 tiles (610). MFMA-bound: 110-120 of the 150 TFLOP/s
 // an MFMA loop reaches. 32 KiB of LDS keep five workgroups on a CU; with 48
 // (two buffers for the halves) three, and 2048 x 2048 x 4096 took 308 us
-// instead of 293.
+// instead of 293. Sums are one chain over K (two, where 64x32 tiles deal the
+// slices to two groups): 1000 x 1500 x 1001, in two, 4.0e-7 from 64 bits, 2000 x
+// 3000 x 1001, in one, 5.7e-7, as the kernel before had at both.
 template <bool B_NK, typename Epi>
 __device__ __forceinline__ void gemm_f32_any(const float* __restrict__ A, const float* __restrict__ B,
                                              float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, Epi epi,
@@ -1316,9 +1319,9 @@ __device__ __forceinline__ void gemm_f32_any(const float* __restrict__ A, const 
 // lanes 0-31 and k = 8h + 4 + e on lanes 32-63, so a lane reads the four k
 // of its row it needs for four steps with one 16-byte read (an [n][k] B
 // too; a [k][n] B as four 4-byte reads). Every k of the slice is summed once;
-// the order of the sums differs from gemm_f32_tile's.
-// Measured interleaved with gemm_f32_tile<.., 256, 256> at 4096^3 (rotated
-// inputs, one box): 945-947 against 1030-1033 us, 145.3 against 133.3
+// the order of the sums is the any-shape kernel's.
+// Measured interleaved with a register-staged kernel of 16 waves of 64x64 in
+// 256x256 tiles, k in order, at 4096^3 (rotated inputs, one box): 945-947 against 1030-1033 us, 145.3 against 133.3
 // TFLOP/s; the error against a float64 sum of the same products 6.95e-5
 // against 8.37e-5 on 64 sampled elements.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
