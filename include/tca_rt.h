@@ -139,7 +139,9 @@ int tca_program_check(tca_program p, const tca_tensor* tensors, uint32_t n_tenso
  * carry variants of one kernel specialised on a run-time dim; their guards
  * pick one), and, when `grids` / `blocks` are not NULL, the grid and block
  * each selected kernel would launch with (0 for the others; packed row
- * kernels size their block at launch). Host-only. No counterpart in the
+ * kernels size their block at launch). Where the plan gives a kernel forms,
+ * a launch may run one in its place: the same arguments and result, its own
+ * function and grid. Host-only. No counterpart in the
  * reference (its launcher has a single kernel per DSL kernel); for tests and
  * profilers. */
 int tca_program_selected(tca_program p, const tca_tensor* tensors, uint32_t n_tensors,
